@@ -17,8 +17,12 @@ CLI = os.path.join(HERE, "mbr_nogui")
 CALIB = os.path.join(HERE, "mbr_calib")
 OBJDIR = os.path.join(HERE, "_build")
 
-SOURCES = ["mbr_api.cpp", "mbr_kernels.hip", "mbr_adjoint.hip", "mbr_post.hip", "mbr_post_order.cpp",
-           "mbr_settings.cpp", "mbr_image.cpp"]
+# (source, unit): the render kernels are compiled once per unit of launches
+# (MBR_PART), in parallel
+KERNEL_UNITS = (2, 3, 4, 1, 0, 5)
+SOURCES = [("mbr_kernels.hip", u) for u in KERNEL_UNITS] + [
+    (src, None) for src in ("mbr_api.cpp", "mbr_adjoint.hip", "mbr_post.hip", "mbr_post_order.cpp",
+                            "mbr_settings.cpp", "mbr_image.cpp")]
 
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 FLAGS = [
@@ -39,9 +43,13 @@ FLAGS = [
 EXTRA = {}
 
 
-def _compile(src):
-    obj = os.path.join(OBJDIR, os.path.splitext(src)[0] + ".o")
-    cmd = [HIPCC, "-x", "hip", *FLAGS, *EXTRA.get(src, []), "-c", os.path.join(CSRC, src), "-o", obj]
+def _compile(job):
+    src, unit = job
+    name, part = os.path.splitext(src)[0], []
+    if unit is not None:
+        name, part = f"{name}.{unit}", [f"-DMBR_PART={unit}"]
+    obj = os.path.join(OBJDIR, name + ".o")
+    cmd = [HIPCC, "-x", "hip", *FLAGS, *EXTRA.get(src, []), *part, "-c", os.path.join(CSRC, src), "-o", obj]
     r = subprocess.run(cmd, capture_output=True, text=True)
     if r.returncode != 0:
         raise RuntimeError(f"hipcc failed for {src}:\n{' '.join(cmd)}\n{r.stdout}\n{r.stderr}")

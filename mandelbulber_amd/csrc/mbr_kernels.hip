@@ -16,6 +16,14 @@
 #include "mbr_kernels.hpp"
 #include "mbr_shade.hpp"
 
+// This source is compiled once per unit of launches, in parallel (build.py);
+// without MBR_PART it holds them all.
+#ifdef MBR_PART
+#define MBR_UNIT(k) (MBR_PART == (k))
+#else
+#define MBR_UNIT(k) 1
+#endif
+
 namespace mbr {
 
 constexpr int kBlock = 256;
@@ -1346,10 +1354,12 @@ __global__ void __launch_bounds__(kBlock) k_finish_fx(const DevScene *__restrict
 }
 
 // ----------------------------------------------------------- reflections
+#if MBR_UNIT(5)
 __global__ void k_refl_clear(uint8_t *active, int n) {
   const int r = blockIdx.x * kBlock + threadIdx.x;
   if (r < n) active[r] = 0;
 }
+#endif
 
 // The mirrored rays of the reflecting hits of `prev` (src/Render3D.cpp:
 // 478-498): normal at the hit (CalculateNormals with the hit's threshold as
@@ -1550,6 +1560,7 @@ __global__ void __launch_bounds__(kBlock) k_refl_finish(const DevScene *__restri
 // ---------------------------------------------------------------- launch
 static inline dim3 grid_for(int n) { return dim3((unsigned)((n + kBlock - 1) / kBlock)); }
 
+#if MBR_UNIT(5)
 hipError_t launch_refl_clear(const BandBufs &next, int band_rays, hipStream_t s) {
   if (band_rays <= 0) return hipSuccess;
   hipLaunchKernelGGL(k_refl_clear, grid_for(band_rays), dim3(kBlock), 0, s, next.active, band_rays);
@@ -1608,6 +1619,9 @@ hipError_t launch_refl_finish(const DevScene *sc, const BandBufs *levels, int n_
   return hipGetLastError();
 }
 
+#endif  // reflections
+
+#if MBR_UNIT(0)
 hipError_t launch_march(int precision, const DevScene *sc, const BandBufs &b, int band_first, int band_rays,
                         int formula, int plain, int persist_blocks, unsigned long long *stats, hipStream_t s,
                         bool ip8) {
@@ -1650,6 +1664,9 @@ hipError_t launch_march(int precision, const DevScene *sc, const BandBufs &b, in
   return hipGetLastError();
 }
 
+#endif  // march
+
+#if MBR_UNIT(1)
 hipError_t launch_march_fix(int precision, const DevScene *sc, const BandBufs &b, int band_first, int formula,
                             int persist_blocks, unsigned long long *stats, hipStream_t s, bool ip8) {
   const dim3 grid((unsigned)std::max(1, persist_blocks));
@@ -1689,6 +1706,9 @@ hipError_t launch_march_fix(int precision, const DevScene *sc, const BandBufs &b
   return hipGetLastError();
 }
 
+#endif  // continuation
+
+#if MBR_UNIT(4)
 __global__ void k_band_reset(unsigned long long *counters) {
   if (threadIdx.x < CNT_COUNT) counters[threadIdx.x] = 0;
 }
@@ -1707,118 +1727,141 @@ hipError_t launch_zero(unsigned long long *p, int n, hipStream_t s) {
   return hipGetLastError();
 }
 
-hipError_t launch_shade(int precision, const DevScene *sc, const BandBufs &b, int band_first, AODev ao,
-                        ShadeBufs sbuf, int persist_blocks, unsigned long long *stats, hipStream_t s,
-                        hipEvent_t ev_ao0, hipEvent_t ev_ao1) {
+#endif  // resets
+
+// The shading launches of one element type (T: the path's precision).
+template <class T>
+hipError_t shade_run(const DevScene *sc, const BandBufs &b, int band_first, AODev ao, ShadeBufs sbuf,
+                     int persist_blocks, unsigned long long *stats, hipStream_t s, hipEvent_t ev_ao0,
+                     hipEvent_t ev_ao1);
+
+#if MBR_UNIT(2) || MBR_UNIT(3)
+template <class T>
+hipError_t shade_run(const DevScene *sc, const BandBufs &b, int band_first, AODev ao, ShadeBufs sbuf,
+                     int persist_blocks, unsigned long long *stats, hipStream_t s, hipEvent_t ev_ao0,
+                     hipEvent_t ev_ao1) {
   const int formula = sbuf.formula;
   // persistent grids: enough workgroups to fill every CU several times; the
   // kernels loop over the band's hits
   const dim3 grid((unsigned)std::max(1, persist_blocks));
-  auto run = [&](auto tag) -> hipError_t {
-    using T = decltype(tag);
-    SurfBufs<T> sb;
-    sb.base = (T *)sbuf.base;
-    sb.spec = (T *)sbuf.spec;
-    sb.col = (T *)sbuf.col;
-    sb.fast_ao = (T *)sbuf.fast_ao;
-    sb.ao = (T *)sbuf.ao;
-    sb.aux = (T *)sbuf.aux;
-    sb.n = sbuf.n;
-    const bool generic = formula_generic(formula);
-    auto surf = [&](auto deep_tag) {
-      constexpr bool D = decltype(deep_tag)::value;
-      if constexpr (!D) {
-        if (generic) {
-          hipLaunchKernelGGL((k_surface<T, 0, false>), grid, dim3(kBlock), 0, s, sc, b, band_first, sb, stats);
-          return;
-        }
-      }
-      if (formula == 7)
-        hipLaunchKernelGGL((k_surface<T, 7, D>), grid, dim3(kBlock), 0, s, sc, b, band_first, sb, stats);
-      else if (formula == 8)
-        hipLaunchKernelGGL((k_surface<T, 8, D>), grid, dim3(kBlock), 0, s, sc, b, band_first, sb, stats);
-      else
-        hipLaunchKernelGGL((k_surface<T, 2, D>), grid, dim3(kBlock), 0, s, sc, b, band_first, sb, stats);
-    };
-    auto aok = [&](auto deep_tag, auto plain_tag) {
-      constexpr bool D = decltype(deep_tag)::value;
-      constexpr bool Pl = decltype(plain_tag)::value;
-      if constexpr (!D && Pl && std::is_same<T, float>::value) {
-        if (formula == 7)
-          hipLaunchKernelGGL((k_ao_f32_plain<T, 7>), grid, dim3(kBlock), 0, s, sc, b, ao, sb, stats);
-        else if (formula == 8)
-          hipLaunchKernelGGL((k_ao_f32_plain<T, 8>), grid, dim3(kBlock), 0, s, sc, b, ao, sb, stats);
-        else if (sbuf.ip8)
-          hipLaunchKernelGGL((k_ao_f32_plain<T, 2, 8>), grid, dim3(kBlock), 0, s, sc, b, ao, sb, stats);
-        else
-          hipLaunchKernelGGL((k_ao_f32_plain<T, 2>), grid, dim3(kBlock), 0, s, sc, b, ao, sb, stats);
+  SurfBufs<T> sb;
+  sb.base = (T *)sbuf.base;
+  sb.spec = (T *)sbuf.spec;
+  sb.col = (T *)sbuf.col;
+  sb.fast_ao = (T *)sbuf.fast_ao;
+  sb.ao = (T *)sbuf.ao;
+  sb.aux = (T *)sbuf.aux;
+  sb.n = sbuf.n;
+  const bool generic = formula_generic(formula);
+  auto surf = [&](auto deep_tag) {
+    constexpr bool D = decltype(deep_tag)::value;
+    if constexpr (!D) {
+      if (generic) {
+        hipLaunchKernelGGL((k_surface<T, 0, false>), grid, dim3(kBlock), 0, s, sc, b, band_first, sb, stats);
         return;
       }
-      if constexpr (!D && !Pl) {
-        if (generic) {
-          hipLaunchKernelGGL((k_ao<T, 0, false, false>), grid, dim3(kBlock), 0, s, sc, b, ao, sb, stats);
-          return;
-        }
-      }
-      if constexpr (!D && Pl && std::is_same<T, double>::value) {
-        if (formula == 2 && sbuf.ip8) {  // FP64_DEMOIVRE
-          hipLaunchKernelGGL((k_ao<T, 2, false, true, 8>), grid, dim3(kBlock), 0, s, sc, b, ao, sb, stats);
-          return;
-        }
-      }
-      if (formula == 7)
-        hipLaunchKernelGGL((k_ao<T, 7, D, Pl>), grid, dim3(kBlock), 0, s, sc, b, ao, sb, stats);
-      else if (formula == 8)
-        hipLaunchKernelGGL((k_ao<T, 8, D, Pl>), grid, dim3(kBlock), 0, s, sc, b, ao, sb, stats);
-      else
-        hipLaunchKernelGGL((k_ao<T, 2, D, Pl>), grid, dim3(kBlock), 0, s, sc, b, ao, sb, stats);
-    };
-    // deep-zoom variants only for FP32 shading of scenes that need them
-    const bool deep = sbuf.deep && sizeof(T) < 8 && !generic;
-    if (deep) surf(std::true_type{});
-    else surf(std::false_type{});
-    if (sbuf.lights) {
-      if (generic) {
-        if constexpr (std::is_same<T, double>::value)
-          hipLaunchKernelGGL((k_aux<T, 0, false>), grid, dim3(kBlock), 0, s, sc, b, band_first, sb, stats);
-      } else {
-        auto aux = [&](auto deep_tag) {
-          constexpr bool D = decltype(deep_tag)::value;
-          if (formula == 7)
-            hipLaunchKernelGGL((k_aux<T, 7, D>), grid, dim3(kBlock), 0, s, sc, b, band_first, sb, stats);
-          else if (formula == 8)
-            hipLaunchKernelGGL((k_aux<T, 8, D>), grid, dim3(kBlock), 0, s, sc, b, band_first, sb, stats);
-          else
-            hipLaunchKernelGGL((k_aux<T, 2, D>), grid, dim3(kBlock), 0, s, sc, b, band_first, sb, stats);
-        };
-        if (deep) aux(std::true_type{});
-        else aux(std::false_type{});
-      }
     }
-    if (ev_ao0) {
-      hipError_t e = hipEventRecord(ev_ao0, s);
-      if (e != hipSuccess) return e;
-    }
-    if (sbuf.slow_ao) {
-      // plain scenes (no primitives, limits, interior mode, iteration
-      // threshold, pre-folds or Julia constant) take a variant without those
-      // branches and the scene constants they keep live
-      if (deep) aok(std::true_type{}, std::false_type{});
-      else if (sbuf.plain && !generic) aok(std::false_type{}, std::true_type{});
-      else aok(std::false_type{}, std::false_type{});
-    }
-    if (ev_ao1) {
-      hipError_t e = hipEventRecord(ev_ao1, s);
-      if (e != hipSuccess) return e;
-    }
-    hipLaunchKernelGGL((k_compose<T, T>), grid, dim3(kBlock), 0, s, sc, b, ao, sb);
-    return hipGetLastError();
+    if (formula == 7)
+      hipLaunchKernelGGL((k_surface<T, 7, D>), grid, dim3(kBlock), 0, s, sc, b, band_first, sb, stats);
+    else if (formula == 8)
+      hipLaunchKernelGGL((k_surface<T, 8, D>), grid, dim3(kBlock), 0, s, sc, b, band_first, sb, stats);
+    else
+      hipLaunchKernelGGL((k_surface<T, 2, D>), grid, dim3(kBlock), 0, s, sc, b, band_first, sb, stats);
   };
+  auto aok = [&](auto deep_tag, auto plain_tag) {
+    constexpr bool D = decltype(deep_tag)::value;
+    constexpr bool Pl = decltype(plain_tag)::value;
+    if constexpr (!D && Pl && std::is_same<T, float>::value) {
+      if (formula == 7)
+        hipLaunchKernelGGL((k_ao_f32_plain<T, 7>), grid, dim3(kBlock), 0, s, sc, b, ao, sb, stats);
+      else if (formula == 8)
+        hipLaunchKernelGGL((k_ao_f32_plain<T, 8>), grid, dim3(kBlock), 0, s, sc, b, ao, sb, stats);
+      else if (sbuf.ip8)
+        hipLaunchKernelGGL((k_ao_f32_plain<T, 2, 8>), grid, dim3(kBlock), 0, s, sc, b, ao, sb, stats);
+      else
+        hipLaunchKernelGGL((k_ao_f32_plain<T, 2>), grid, dim3(kBlock), 0, s, sc, b, ao, sb, stats);
+      return;
+    }
+    if constexpr (!D && !Pl) {
+      if (generic) {
+        hipLaunchKernelGGL((k_ao<T, 0, false, false>), grid, dim3(kBlock), 0, s, sc, b, ao, sb, stats);
+        return;
+      }
+    }
+    if constexpr (!D && Pl && std::is_same<T, double>::value) {
+      if (formula == 2 && sbuf.ip8) {  // FP64_DEMOIVRE
+        hipLaunchKernelGGL((k_ao<T, 2, false, true, 8>), grid, dim3(kBlock), 0, s, sc, b, ao, sb, stats);
+        return;
+      }
+    }
+    if (formula == 7)
+      hipLaunchKernelGGL((k_ao<T, 7, D, Pl>), grid, dim3(kBlock), 0, s, sc, b, ao, sb, stats);
+    else if (formula == 8)
+      hipLaunchKernelGGL((k_ao<T, 8, D, Pl>), grid, dim3(kBlock), 0, s, sc, b, ao, sb, stats);
+    else
+      hipLaunchKernelGGL((k_ao<T, 2, D, Pl>), grid, dim3(kBlock), 0, s, sc, b, ao, sb, stats);
+  };
+  // deep-zoom variants only for FP32 shading of scenes that need them
+  const bool deep = sbuf.deep && sizeof(T) < 8 && !generic;
+  if (deep) surf(std::true_type{});
+  else surf(std::false_type{});
+  if (sbuf.lights) {
+    if (generic) {
+      if constexpr (std::is_same<T, double>::value)
+        hipLaunchKernelGGL((k_aux<T, 0, false>), grid, dim3(kBlock), 0, s, sc, b, band_first, sb, stats);
+    } else {
+      auto aux = [&](auto deep_tag) {
+        constexpr bool D = decltype(deep_tag)::value;
+        if (formula == 7)
+          hipLaunchKernelGGL((k_aux<T, 7, D>), grid, dim3(kBlock), 0, s, sc, b, band_first, sb, stats);
+        else if (formula == 8)
+          hipLaunchKernelGGL((k_aux<T, 8, D>), grid, dim3(kBlock), 0, s, sc, b, band_first, sb, stats);
+        else
+          hipLaunchKernelGGL((k_aux<T, 2, D>), grid, dim3(kBlock), 0, s, sc, b, band_first, sb, stats);
+      };
+      if (deep) aux(std::true_type{});
+      else aux(std::false_type{});
+    }
+  }
+  if (ev_ao0) {
+    hipError_t e = hipEventRecord(ev_ao0, s);
+    if (e != hipSuccess) return e;
+  }
+  if (sbuf.slow_ao) {
+    // plain scenes (no primitives, limits, interior mode, iteration
+    // threshold, pre-folds or Julia constant) take a variant without those
+    // branches and the scene constants they keep live
+    if (deep) aok(std::true_type{}, std::false_type{});
+    else if (sbuf.plain && !generic) aok(std::false_type{}, std::true_type{});
+    else aok(std::false_type{}, std::false_type{});
+  }
+  if (ev_ao1) {
+    hipError_t e = hipEventRecord(ev_ao1, s);
+    if (e != hipSuccess) return e;
+  }
+  hipLaunchKernelGGL((k_compose<T, T>), grid, dim3(kBlock), 0, s, sc, b, ao, sb);
+  return hipGetLastError();
+}
+#endif
+
+#if MBR_UNIT(2)
+template hipError_t shade_run<double>(const DevScene *, const BandBufs &, int, AODev, ShadeBufs, int,
+                                      unsigned long long *, hipStream_t, hipEvent_t, hipEvent_t);
+#endif
+#if MBR_UNIT(3)
+template hipError_t shade_run<float>(const DevScene *, const BandBufs &, int, AODev, ShadeBufs, int,
+                                     unsigned long long *, hipStream_t, hipEvent_t, hipEvent_t);
+#endif
+
+#if MBR_UNIT(4)
+hipError_t launch_shade(int precision, const DevScene *sc, const BandBufs &b, int band_first, AODev ao,
+                        ShadeBufs sbuf, int persist_blocks, unsigned long long *stats, hipStream_t s,
+                        hipEvent_t ev_ao0, hipEvent_t ev_ao1) {
   // generic formulas in FP32: FP32_FIXUP without aux lights (the host keeps
   // other generic scenes in FP64)
-  if (formula_generic(formula) && (precision > 1 || (precision == 1 && sbuf.lights))) return hipErrorInvalidValue;
-  if (precision == 0) return run(double{});
-  return run(float{});
+  if (formula_generic(sbuf.formula) && (precision > 1 || (precision == 1 && sbuf.lights))) return hipErrorInvalidValue;
+  if (precision == 0) return shade_run<double>(sc, b, band_first, ao, sbuf, persist_blocks, stats, s, ev_ao0, ev_ao1);
+  return shade_run<float>(sc, b, band_first, ao, sbuf, persist_blocks, stats, s, ev_ao0, ev_ao1);
 }
 
 hipError_t launch_finish(int precision, const DevScene *sc, const BandBufs &b, int band_first, int band_rays,
@@ -1865,5 +1908,6 @@ hipError_t launch_finish(int precision, const DevScene *sc, const BandBufs &b, i
   }
   return hipGetLastError();
 }
+#endif  // finish
 
 }  // namespace mbr
