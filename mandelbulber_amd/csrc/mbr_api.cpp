@@ -941,6 +941,7 @@ int prepare_scene(mbr_ctx *c, const mbr_scene *scene_in, const mbr_texture *ligh
   d.plain = d.fd.limits == 0 && d.fd.only_plane == 0 && d.fd.interior == 0 && d.fd.iter_thresh == 0 &&
             !d.fd.prim_plane && !d.fd.prim_box && !d.fd.prim_ibox && !d.fd.prim_sphere && !d.fd.prim_isphere &&
             !d.fd.prim_water && !d.fd.tglad_fold && !d.fd.sph_fold && !d.fd.julia_mode && !d.fd.ifs_fold;
+  if (d.plain) d.plain = s.formula == 8 && !d.fd.mb_rot_on && !d.fd.mb_main_rot ? kUnrotated : kPlain;
   return MBR_OK;
 }
 
@@ -1233,8 +1234,9 @@ int enqueue_band(mbr_ctx *c, Slot &sl, const ShadeBufs &sbuf, int precision, con
   if (e) HIPCHECK(c, hipEventRecord(e[0], st));
   HIPCHECK(c, launch_march(precision, d_sc, b, (int)band_first, band_rays, formula, host.plain, persist, d_stats, st,
                            sbuf.ip8 != 0));
-  HIPCHECK(c, launch_march_fix(precision, d_sc, b, (int)band_first, formula, persist / 2, d_stats, st,
-                               sbuf.ip8 != 0));
+  if (precision == MBR_PREC_FP32_MARCH)
+    HIPCHECK(c, launch_march_fix(d_sc, b, (int)band_first, formula, host.plain, persist, d_stats, st,
+                                 sbuf.ip8 != 0));
   if (e) HIPCHECK(c, hipEventRecord(e[1], st));
   HIPCHECK(c, launch_shade(precision, d_sc, b, (int)band_first, ao, sbuf, persist, d_stats, st,
                            e ? e[4] : nullptr, e ? e[5] : nullptr));
@@ -1380,7 +1382,6 @@ int enqueue_frame_refl(mbr_ctx *c, std::vector<Slot *> &lv, const DevScene *d_sc
     if (e) HIPCHECK(c, hipEventRecord(e[0], st));
     HIPCHECK(c, launch_march(MBR_PREC_FP64, d_sc, b0, (int)band_first, band_rays, formula, host.plain, persist,
                              c->d_stats, st));
-    HIPCHECK(c, launch_march_fix(MBR_PREC_FP64, d_sc, b0, (int)band_first, formula, persist / 2, c->d_stats, st));
     for (int k = 1; k < n_levels; k++) {
       BandBufs &bk = lv[(size_t)k]->band;
       HIPCHECK(c, launch_band_reset(bk, st));
@@ -2303,8 +2304,6 @@ int run_adjoint(mbr_ctx *c, const mbr_render_opts *opts, const float *const grad
       HIPCHECK(c, launch_band_reset(sl.band, st));
       HIPCHECK(c, launch_march(MBR_PREC_FP64, c->d_sc, sl.band, (int)band_first, band_rays, s.formula,
                                c->host_sc.plain, persist, c->d_stats, st));
-      HIPCHECK(c, launch_march_fix(MBR_PREC_FP64, c->d_sc, sl.band, (int)band_first, s.formula, persist / 2,
-                                   c->d_stats, st));
       HIPCHECK(c, launch_adjoint(c->d_sc, sl.band, (int)band_first, band_rays, p, gR, gG, gB,
                                  jac ? nullptr : c->d_grad, skipped, jac, persist, st));
     }

@@ -147,12 +147,22 @@ MBR_HD uint32_t mix32(uint32_t x) {
 
 // Counter-based stand-in for Random(1000) (src/common_math.cpp:25-32) at
 // one march step: an integer in [0, 1000].
-MBR_HD uint32_t jitter_draw(uint32_t seed, uint32_t frame, uint32_t pixel, uint32_t step) {
+// jitter_ray holds what the steps of one ray share.
+MBR_HD uint32_t jitter_ray(uint32_t seed, uint32_t frame, uint32_t pixel) {
   uint32_t h = mix32(seed ^ 0x9e3779b9U);
   h = mix32(h ^ frame);
-  h = mix32(h ^ pixel);
-  h = mix32(h ^ step);
-  return h % 1001U;
+  return mix32(h ^ pixel);
+}
+MBR_HD uint32_t jitter_draw(uint32_t ray, uint32_t step) { return mix32(ray ^ step) % 1001U; }
+MBR_HD uint32_t jitter_draw(uint32_t seed, uint32_t frame, uint32_t pixel, uint32_t step) {
+  return jitter_draw(jitter_ray(seed, frame, pixel), step);
+}
+// The step's factor 1 - draw / 10000, the quotient by its reciprocal and one
+// correction (equal to the division for all 1001 draws) instead of the FP64
+// division sequence.
+MBR_HD double jitter_factor(uint32_t draw) {
+  const double d = (double)draw, q = d * 1e-4;
+  return 1.0 - __builtin_fma(__builtin_fma(-q, 10000.0, d), 1e-4, q);
 }
 
 // double -> int as the reference's x86-64 build converts it: values out of

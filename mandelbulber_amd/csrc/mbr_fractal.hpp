@@ -776,7 +776,14 @@ struct DEIter {
 
 // IP: the Mandelbulb's integer power when the caller knows it at compile
 // time (8, the standard bulb), else 0 (read from f.ipow).
-template <class T, int F, bool P = false, bool A = (sizeof(T) < 8), int IP = 0>
+// P: what the caller knows of the scene: kOptions nothing, kPlain that no
+// optional term is on (primitives, limits, interior mode, iteration
+// threshold, pre-folds, Julia constant), kUnrotated (Mandelbox) in addition
+// that its folds and its main rotation are not rotated.  The 19 rotation
+// matrices otherwise fill the scalar registers of every kernel that holds
+// the iteration (380-450 spills into vector lanes, read back in every pass).
+enum : int { kOptions = 0, kPlain = 1, kUnrotated = 2 };
+template <class T, int F, int P = 0, bool A = (sizeof(T) < 8), int IP = 0>
 MBR_HD void de_begin(const FractalK<T> &f, V3<T> p, DEIter<T> &s) {
   s.z = p;
   s.c = (!P && f.julia_mode) ? ld3(f.julia) : p * f.constant_factor;
@@ -793,11 +800,32 @@ MBR_HD void de_begin(const FractalK<T> &f, V3<T> p, DEIter<T> &s) {
   }
 }
 
-// One loop pass.  Returns true when the call has finished; `dist` is then
-// the return value of Compute<normal> (0 when the orbit stayed bounded for
-// N iterations) and s.L the reference's iteration counter.
-template <class T, int F, bool P = false, bool A = (sizeof(T) < 8), int IP = 0>
-MBR_HD bool de_iter(const FractalK<T> &f, DEIter<T> &s, int N, T &dist) {
+// !(|z| <= R) of the folding formulas' escape test from q = |z|^2, for R =
+// 1000 or 1024, without the square root: an FP64 root and its refinement are
+// about as long as a whole Menger iteration.  FP64 roots are correctly
+// rounded, so |z| <= R exactly when q is at most the largest double whose
+// root rounds to R.  FP32 roots are the hardware's (1 ulp): inside a band of
+// 2^-20 about R^2 the root itself decides.  NaN counts as escaped.
+template <int R>
+MBR_HD bool beyond(double q) {
+  static_assert(R == 1000 || R == 1024, "");
+  return !(q <= (R == 1000 ? 0x1.e848p+19 : 0x1.0000000000001p+20));
+}
+template <int R>
+MBR_HD bool beyond(float q) {
+  constexpr float R2 = (float)R * R, lo = R2 * (1.0f - 0x1p-20f), hi = R2 * (1.0f + 0x1p-20f);
+  bool e = !(q <= hi);
+  if (q > lo && q <= hi) e = !(Math<float>::sqrt(q) <= (float)R);
+  return e;
+}
+
+// One loop pass.  Returns true when the call has finished: the orbit escaped
+// (s.L < N, the reference's iteration counter) or stayed bounded for N
+// iterations (s.L == N).  The distance is left to de_escape_distance, so that
+// the persistent kernels form it for the lanes that finished together instead
+// of in every pass.
+template <class T, int F, int P = 0, bool A = (sizeof(T) < 8), int IP = 0>
+MBR_HD bool de_iter(const FractalK<T> &f, DEIter<T> &s, int N) {
   using M = Math<T>;
   V3<T> z = s.z;
   T r = s.r;
@@ -812,6 +840,7 @@ MBR_HD bool de_iter(const FractalK<T> &f, DEIter<T> &s, int N, T &dist) {
     r = length(z);
   }
   if ((!P && f.sph_fold)) {
+    if (F == 7 || F == 8) r = length(z);  // they keep no radius
     T r2 = r * r;
     if (r2 < f.sph_mR2) { z = z * f.sph_factor1; s.aux *= f.sph_factor1; }
     else if (r2 < f.sph_fR2) { T tf2 = fdiv(f.sph_fR2, r2); z = z * tf2; s.aux *= tf2; }
@@ -858,14 +887,11 @@ MBR_HD bool de_iter(const FractalK<T> &f, DEIter<T> &s, int N, T &dist) {
         const T zr2 = z.x * z.x + z.y * z.y + z.z * z.z;
         s.inv_r = fast_rsq(zr2);
         r = zr2 * s.inv_r;
-        esc = !(r <= f.bailout);
-        if (esc) dist = T(0.5) * r * fast_ln(r) * fast_rcp(s.aux);
         s.z = z;
         s.r = r;
-        if (esc) return true;
+        if (!(r <= f.bailout)) return true;
         s.L++;
-        if (s.L >= N) { dist = 0; return true; }
-        return false;
+        return s.L >= N;
       }
       T ure = off_axis ? rho2 * inv_rho * inv_r : T(0);
       T uim = z.z * inv_r;
@@ -897,14 +923,11 @@ MBR_HD bool de_iter(const FractalK<T> &f, DEIter<T> &s, int N, T &dist) {
       const T r2 = z.x * z.x + z.y * z.y + z.z * z.z;
       s.inv_r = fast_rsq(r2);
       r = r2 * s.inv_r;
-      esc = !(r <= f.bailout);
-      if (esc) dist = T(0.5) * r * fast_ln(r) * fast_rcp(s.aux);
       s.z = z;
       s.r = r;
-      if (esc) return true;
+      if (!(r <= f.bailout)) return true;
       s.L++;
-      if (s.L >= N) { dist = 0; return true; }
-      return false;
+      return s.L >= N;
     }
   }
   if constexpr (F == 2) {  // trig_optim
@@ -919,8 +942,8 @@ MBR_HD bool de_iter(const FractalK<T> &f, DEIter<T> &s, int N, T &dist) {
     rp *= r;
     z = V3<T>{cth * M::cos(ph), cth * M::sin(ph), M::sin(th)} * rp + s.c;
     r = length(z);
+    s.r = r;
     esc = !(r <= f.bailout);
-    if (esc) dist = T(0.5) * r * M::log(r) / s.aux;
   } else if constexpr (F == 7) {  // menger_sponge
     T temp;
     z.x = M::fabs(z.x); z.y = M::fabs(z.y); z.z = M::fabs(z.z);
@@ -930,13 +953,11 @@ MBR_HD bool de_iter(const FractalK<T> &f, DEIter<T> &s, int N, T &dist) {
     z = z * T(3);
     z.x -= T(2); z.y -= T(2);
     if (z.z > T(1)) z.z -= T(2);
-    r = length(z);
     s.aux *= T(3);
-    esc = !(r <= T(1000));
-    if (esc) dist = fdiv(r - T(2), s.aux);
+    esc = beyond<1000>(dot(z, z));
   } else {  // tglad (Mandelbox)
     const T lim = f.mb_limit, val = f.mb_value;
-    if (f.mb_rot_on) {
+    if (P != kUnrotated && f.mb_rot_on) {
       bool lockout = false;
       z = rot9(f.mb_rot[0][0], z);
       if (z.x > lim) { z.x = val - z.x; lockout = true; }
@@ -972,19 +993,27 @@ MBR_HD bool de_iter(const FractalK<T> &f, DEIter<T> &s, int N, T &dist) {
     if (r2 < f.mb_mR2) { z = z * f.mb_factor1; s.aux *= f.mb_factor1; }
     else if (r2 < f.mb_fR2) { T tf2 = fdiv(f.mb_fR2, r2); z = z * tf2; s.aux *= tf2; }
     z = z - ld3(f.mb_offset);
-    if (f.mb_main_rot) z = mat_apply(f.mb_main, z);
+    if (P != kUnrotated && f.mb_main_rot) z = mat_apply(f.mb_main, z);
     z = z * f.mb_scale + s.c;
     s.aux = s.aux * f.mb_abs_scale + T(1);
-    r = length(z);
-    esc = !(r <= T(1024));
-    if (esc) dist = fdiv(r, M::fabs(s.aux));
+    esc = beyond<1024>(dot(z, z));
   }
   s.z = z;
-  s.r = r;
   if (esc) return true;
   s.L++;
-  if (s.L >= N) { dist = 0; return true; }
-  return false;
+  return s.L >= N;
+}
+
+// Compute<normal>'s return value for an orbit that escaped.
+template <class T, int F, bool A = (sizeof(T) < 8), int IP = 0>
+MBR_HD T de_escape_distance(const FractalK<T> &f, const DEIter<T> &s) {
+  using M = Math<T>;
+  if constexpr (F == 7) return fdiv(length(s.z) - T(2), s.aux);
+  if constexpr (F == 8) return fdiv(length(s.z), M::fabs(s.aux));
+  if constexpr (F == 2 && A) {
+    if (IP || f.ipow) return T(0.5) * s.r * fast_ln(s.r) * fast_rcp(s.aux);
+  }
+  return T(0.5) * s.r * M::log(s.r) / s.aux;
 }
 
 // CalculateDistance (src/fractal.cpp:1245-1448), analytic branch, split into
@@ -998,7 +1027,7 @@ struct DECall {
   T limitBox;
 };
 
-template <class T, bool P = false>
+template <class T, int P = 0>
 MBR_HD T de_finish(const FractalK<T> &f, V3<T> point, T distance, int L, bool fractal, int N, int minN,
                    bool normalMode, T detailSize, T limitBoxDist, DEInfo &info) {
   info.object = OBJ_FRACTAL;
@@ -1069,7 +1098,7 @@ __attribute__((noinline)) __host__ __device__ T compute_generic(const FractalK<T
 
 // Not inlined: the body (five orbit runs over every generic formula) would
 // otherwise be copied into each of the shaders' distance-estimate sites.
-template <class T, bool P = false>
+template <class T, int P = 0>
 __attribute__((noinline)) __host__ __device__ T calc_distance_generic(const FractalK<T> &f, V3<T> point, T detailSize, int N, int minN, bool normalMode,
                                DEInfo &info) {
 #pragma clang fp contract(off)
@@ -1120,8 +1149,9 @@ __attribute__((noinline)) __host__ __device__ T calc_distance_generic(const Frac
   return dist;
 }
 
-// Start one CalculateDistance; true when it finished without iterating.
-template <class T, int F, bool P = false, bool A = (sizeof(T) < 8), int IP = 0>
+// Start one CalculateDistance; true when it finished without iterating (never
+// in a plain scene: mbr_set_scene accepts N > 0 only).
+template <class T, int F, int P = 0, bool A = (sizeof(T) < 8), int IP = 0>
 MBR_HD bool de_call_begin(const FractalK<T> &f, V3<T> point, T detailSize, int N, int minN, bool normalMode,
                           DECall<T> &call, T &dist, DEInfo &info) {
   if constexpr (F == 0) {
@@ -1149,32 +1179,36 @@ MBR_HD bool de_call_begin(const FractalK<T> &f, V3<T> point, T detailSize, int N
     return true;
   }
   de_begin<T, F, P, A, IP>(f, point, call.it);
-  if (N <= 0) {
+  if (!P && N <= 0) {
     dist = de_finish<T, P>(f, point, T(0), 0, true, N, minN, normalMode, detailSize, call.limitBox, info);
     return true;
   }
   return false;
 }
 
-// Advance one iteration; true when the call finished (dist, info valid).
-template <class T, int F, bool P = false, bool A = (sizeof(T) < 8), int IP = 0>
-MBR_HD bool de_call_step(const FractalK<T> &f, DECall<T> &call, T detailSize, int N, int minN, bool normalMode,
-                         T &dist, DEInfo &info) {
-  T raw = 0;
-  if (!de_iter<T, F, P, A, IP>(f, call.it, N, raw)) return false;
-  dist = de_finish<T, P>(f, call.p, raw, call.it.L, true, N, minN, normalMode, detailSize, call.limitBox, info);
-  return true;
+// Advance one iteration; true when the call finished (de_call_end then gives
+// its distance and info).
+template <class T, int F, int P = 0, bool A = (sizeof(T) < 8), int IP = 0>
+MBR_HD bool de_call_step(const FractalK<T> &f, DECall<T> &call, int N) {
+  return de_iter<T, F, P, A, IP>(f, call.it, N);
 }
 
-template <class T, int F, bool A = (sizeof(T) < 8), int IP = 0>
+template <class T, int F, int P = 0, bool A = (sizeof(T) < 8), int IP = 0>
+MBR_HD T de_call_end(const FractalK<T> &f, const DECall<T> &call, T detailSize, int N, int minN, bool normalMode,
+                     DEInfo &info) {
+  const T raw = call.it.L < N ? de_escape_distance<T, F, A, IP>(f, call.it) : T(0);
+  return de_finish<T, P>(f, call.p, raw, call.it.L, true, N, minN, normalMode, detailSize, call.limitBox, info);
+}
+
+template <class T, int F, bool A = (sizeof(T) < 8), int IP = 0, int P = 0>
 MBR_HD T calc_distance_f(const FractalK<T> &f, V3<T> point, T detailSize, int N, int minN, bool normalMode,
                          DEInfo &info) {
   DECall<T> call;
   T dist = 0;
-  if (de_call_begin<T, F, false, A, IP>(f, point, detailSize, N, minN, normalMode, call, dist, info)) return dist;
-  while (!de_call_step<T, F, false, A, IP>(f, call, detailSize, N, minN, normalMode, dist, info)) {
+  if (de_call_begin<T, F, P, A, IP>(f, point, detailSize, N, minN, normalMode, call, dist, info)) return dist;
+  while (!de_call_step<T, F, P, A, IP>(f, call, N)) {
   }
-  return dist;
+  return de_call_end<T, F, P, A, IP>(f, call, detailSize, N, minN, normalMode, info);
 }
 
 // Distance estimate at an FP64 point for an FP32 caller (camera-relative
@@ -1203,10 +1237,10 @@ MBR_HD bool de_call_begin_p64(const FractalK<double> &fd, const FractalK<float> 
   }
   const double cm = length(c64.it.c);
   for (;;) {
-    const double zm = c64.it.r;
+    const double zm = F == 2 ? c64.it.r : length(c64.it.z);
     if (Math<double>::fabs(c64.it.aux) * (double)detail >= kMixedSwitch * (zm > cm ? zm : cm)) break;
-    if (de_call_step<double, F>(fd, c64, (double)detail, N, minN, normalMode, d64, info)) {
-      dist = (float)d64;
+    if (de_call_step<double, F>(fd, c64, N)) {
+      dist = (float)de_call_end<double, F>(fd, c64, (double)detail, N, minN, normalMode, info);
       return true;
     }
   }
@@ -1242,9 +1276,9 @@ MBR_HD T calc_distance_p64(const FractalK<double> &fd, const FractalK<T> &f, V3<
     DECall<float> call;
     float dist = 0;
     if (de_call_begin_p64<F>(fd, f, point, detailSize, N, minN, normalMode, call, dist, info)) return dist;
-    while (!de_call_step<float, F>(f, call, detailSize, N, minN, normalMode, dist, info)) {
+    while (!de_call_step<float, F>(f, call, N)) {
     }
-    return dist;
+    return de_call_end<float, F>(f, call, detailSize, N, minN, normalMode, info);
   }
 }
 

@@ -156,154 +156,58 @@ struct RayState {
 
 enum : int { SO_CONTINUE = 0, SO_MISS = 1, SO_HANDOFF = 2 };
 
-// Refl: a reflected ray, whose thresholds start from s.thr0
-// (distThreshInit, src/Render3D.cpp:92, :102-109); primary rays start from 0.
-template <bool Refl = false>
-__device__ __forceinline__ void march_before_de(const DevScene &sc, V3<double> start, V3<double> dir, RayState &s) {
-#pragma clang fp contract(off)
+// What every step reads of the scene, held in registers: the kernels' stores
+// keep the compiler from hoisting the loads out of their loops, and a step of a
+// primary ray has fewer than two formula iterations to hide them behind.
+struct MarchK {
+  double resolution, persp, quality, DE_factor, far, below;
+  int constant_thresh, wide, jitter;
+};
+__device__ __forceinline__ MarchK march_k(const DevScene &sc) {
   const ShadeK<double> &k = sc.sd;
+  return MarchK{k.resolution, k.persp, k.quality, k.DE_factor, sc.view_distance_max, sc.interior ? 0.8 : 0.5,
+                sc.constant_thresh, sc.persp_type == 1 || sc.persp_type == 2, sc.jitter_mode};
+}
+
+// The threshold at a distance along the ray; a quality of 1 needs no division.
+// thr0: 0, or a reflected ray's initial threshold (distThreshInit,
+// src/Render3D.cpp:92, :102-109).
+__device__ __forceinline__ double march_thr(const MarchK &m, double scan, double thr0) {
+#pragma clang fp contract(off)
+  if (m.constant_thresh) return m.quality;
+  double t = scan * m.resolution * m.persp;
+  if (m.quality != 1.0) t = t / m.quality;
+  return t + thr0;
+}
+
+__device__ __forceinline__ void march_before_de(const MarchK &m, V3<double> start, V3<double> dir, RayState &s) {
+#pragma clang fp contract(off)
   s.point = start + dir * s.scan;
-  s.thr = sc.constant_thresh ? k.quality : s.scan * k.resolution * k.persp / k.quality + (Refl ? s.thr0 : 0.0);
-  if (sc.persp_type == 1 || sc.persp_type == 2) s.thr *= kPi;
+  s.thr = march_thr(m, s.scan, s.thr0);
+  if (m.wide) s.thr *= kPi;
 }
 
 // obj_it: the estimate's object type in the low 3 bits, its iteration count
 // (CalculateDistance's itersOut) above them.
-template <class T, class RT>
-__device__ __forceinline__ int march_after_de(const DevScene &sc, RayState &s, double d, int obj_it, uint32_t pixel,
-                                              const RecPlanes<RT> &rec) {
+__device__ __forceinline__ int march_after_de(const MarchK &m, RayState &s, double d, int obj_it, uint32_t ray_hash,
+                                              const RecPlanes<float> &rec) {
 #pragma clang fp contract(off)
-  const ShadeK<double> &k = sc.sd;
   s.object = obj_it & 7;
   const double dist = d > 3.0 ? 3.0 : d;
-  double err = 0.0;
-  if constexpr (sizeof(T) < 8) {
-    // s.drift holds the variance of the scan deviation
-    const double pmax = fmax(fabs(s.point.x), fmax(fabs(s.point.y), fabs(s.point.z)));
-    err = 1e-6 * fabs(d) + 6e-8 * pmax;
-    if (dist < 1.001 * s.thr || dist - s.thr < 4.0 * sqrt(s.drift + err * err)) return SO_HANDOFF;
-  } else {
-    if (dist < s.thr) return SO_HANDOFF;
-  }
-  const double jf = sc.jitter_mode ? 1.0 - jitter_draw(sc.jitter_seed, sc.frame_no, pixel, (uint32_t)s.i) / 10000.0 : 1.0;
+  // s.drift holds the variance of the scan deviation
+  const double pmax = fmax(fabs(s.point.x), fmax(fabs(s.point.y), fabs(s.point.z)));
+  const double err = 1e-6 * fabs(d) + 6e-8 * pmax;
+  if (dist < 1.001 * s.thr || dist - s.thr < 4.0 * sqrt(s.drift + err * err)) return SO_HANDOFF;
+  const double jf = m.jitter ? jitter_factor(jitter_draw(ray_hash, (uint32_t)s.i)) : 1.0;
   const double old_step = s.step;
-  s.step = (dist - (sc.interior ? 0.8 : 0.5) * s.thr) * k.DE_factor * jf;
+  s.step = (dist - m.below * s.thr) * m.DE_factor * jf;
   rec.put(s.i, old_step, d, s.thr, obj_it >> 3);
   s.scan += s.step;
-  s.drift += (err * k.DE_factor) * (err * k.DE_factor);
+  s.drift += (err * m.DE_factor) * (err * m.DE_factor);
   s.dist = dist;
   s.i++;
-  if (s.scan > sc.view_distance_max || s.i >= 10000) return SO_MISS;
+  if (s.scan > m.far || s.i >= 10000) return SO_MISS;
   return SO_CONTINUE;
-}
-
-// The reference loop from step s.i on, in FP64, then the binary search
-// (src/Render3D.cpp:145-183).  Sets `ambiguous` when a decision lies within
-// the drift margin of its threshold (see the hand-over rule above).
-template <class RT, int F, bool Refl = false, int IP = 0>
-__device__ void march_continue_f64(const DevScene &sc, V3<double> start, V3<double> dir, uint32_t pixel,
-                                   const RecPlanes<RT> &rec, RayState s, MarchOut &o, LaneCount &cnt,
-                                   bool &ambiguous) {
-#pragma clang fp contract(off)
-  // trig-free integer-power iteration where the records are FP32, as in
-  // k_march
-  constexpr bool kAlg = sizeof(RT) < 8 || IP != 0;
-  const ShadeK<double> &k = sc.sd;
-  const double search_limit = 1.0 - 0.01 * k.quality;
-  const double margin = 4.0 * sqrt(s.drift);  // s.drift: variance of the FP32 scan deviation
-  bool found = false, missed = false;
-  double dist = 0.0, detail = 0.0;
-  double prev_dist = s.dist, prev_scan = s.scan - s.step;  // the step before s.i
-  bool have_prev = s.i > 0;
-  ambiguous = false;
-  for (; s.i < 10000; s.i++) {
-    march_before_de<Refl>(sc, start, dir, s);
-    detail = s.thr;
-    DEInfo info;
-    dist = calc_distance_f<double, F, kAlg, IP>(sc.fd, s.point, detail, sc.N, sc.minN, false, info);
-    cnt.add(info);
-    s.object = info.object;
-    const double dist_raw = dist;
-    if (dist > 3.0) dist = 3.0;
-    if (fabs(dist - s.thr) < margin) ambiguous = true;
-    if (dist < s.thr) {
-      if (dist < 0.1 * s.thr) missed = true;
-      found = true;
-      break;
-    }
-    const double jf = sc.jitter_mode ? 1.0 - jitter_draw(sc.jitter_seed, sc.frame_no, pixel, (uint32_t)s.i) / 10000.0 : 1.0;
-    const double old_step = s.step;
-    s.step = (dist - (sc.interior ? 0.8 : 0.5) * s.thr) * k.DE_factor * jf;
-    rec.put(s.i, old_step, dist_raw, s.thr, info.iters);
-    prev_dist = dist;
-    prev_scan = s.scan;
-    have_prev = true;
-    s.scan += s.step;
-    if (s.scan > sc.view_distance_max) { s.i++; break; }
-  }
-  double distThresh = s.thr, scan = s.scan;
-  V3<double> point = s.point;
-  int object = s.object;
-  if (found) {
-    double step = s.step * 0.5;
-    for (int j = 0; j < 20; j++) {
-      if (step > 5e-6 * scan &&
-          (fabs(dist - distThresh) < margin || fabs(dist - distThresh * search_limit) < margin))
-        ambiguous = true;
-      if (dist < distThresh && dist > distThresh * search_limit) break;
-      prev_dist = dist;
-      prev_scan = scan;
-      have_prev = true;
-      if (dist > distThresh) { scan += step; point = start + dir * scan; }
-      else if (dist < distThresh * search_limit) { scan -= step; point = start + dir * scan; }
-      distThresh = sc.constant_thresh ? k.quality : scan * k.resolution * k.persp / k.quality + (Refl ? s.thr0 : 0.0);
-      DEInfo bi;
-      dist = calc_distance_f<double, F, kAlg, IP>(sc.fd, point, detail, sc.N, sc.minN, false, bi);
-      cnt.add(bi);
-      object = bi.object;
-      step *= 0.5;
-    }
-    if (ambiguous && have_prev) {
-      const double g = fabs(dist - prev_dist) / fmax(fabs(scan - prev_scan), 1e-300);
-      const double W = (0.01 * k.quality * distThresh + 2.0 * margin) / fmax(g, 1e-12);
-      ambiguous = W > kRedoTol * scan;
-    }
-    if (sc.hit_refine && !sc.constant_thresh) {
-      // Newton steps on F(t) = dist(t) - c0 thr(t), c0 the middle of the
-      // band, with a central-difference slope; each step at most one
-      // threshold long
-      const double c0 = 1.0 - 0.005 * k.quality;
-      const double kthr = k.resolution * k.persp / k.quality;
-      double t = scan, f = dist - c0 * kthr * t;
-      for (int it = 0; it < 8 && fabs(f) > 1e-13 * kthr * t; it++) {
-        const double eps = 1e-3 * kthr * t;
-        DEInfo bi;
-        const double dp = calc_distance_f<double, F, kAlg, IP>(sc.fd, start + dir * (t + eps), detail, sc.N, sc.minN, false, bi);
-        const double dm = calc_distance_f<double, F, kAlg, IP>(sc.fd, start + dir * (t - eps), detail, sc.N, sc.minN, false, bi);
-        const double g = (dp - dm) / (2.0 * eps) - c0 * kthr;
-        if (!(fabs(g) > 0.0)) break;
-        double dt = -f / g;
-        const double lim = kthr * t;
-        dt = dt > lim ? lim : (dt < -lim ? -lim : dt);
-        t += dt;
-        dist = calc_distance_f<double, F, kAlg, IP>(sc.fd, start + dir * t, detail, sc.N, sc.minN, false, bi);
-        cnt.add(bi);
-        object = bi.object;
-        f = dist - c0 * kthr * t;
-      }
-      scan = t;
-      point = start + dir * scan;
-      distThresh = scan * kthr;
-    }
-  }
-  o.point = point;
-  o.scan = scan;
-  o.distThresh = distThresh;
-  o.dist = dist;
-  o.buffCount = s.i;
-  o.object = object;
-  o.found = found;
-  o.missed = missed;
 }
 
 __device__ __forceinline__ RayState ray_start_state(const DevScene &sc) {
@@ -393,9 +297,11 @@ enum : int { MS_NEED = 0, MS_ITER = 1, MS_DONE = 2, MS_EXHAUSTED = 3 };
 constexpr int kMarchIters = MBR_MARCH_ITERS;
 
 // IP: the integer power of the Mandelbulb when fixed at compile time (8).
-template <class T, class RT, int F, bool Plain, int IP>
+template <int F, int Plain, int IP>
 __device__ __forceinline__ void march_body(const DevScene *__restrict__ scp, BandBufs b, int band_first,
                                            int band_rays, unsigned long long *stats) {
+  using T = float;
+  using RT = float;
   // integer-power Mandelbulb iterations without inverse trig wherever the
   // records are FP32; the FP64 mode keeps the trigonometric form
   constexpr bool kAlg = sizeof(RT) < 8 || IP != 0;
@@ -410,26 +316,25 @@ __device__ __forceinline__ void march_body(const DevScene *__restrict__ scp, Ban
   const unsigned long long lt_mask = (lane == 0) ? 0ull : (~0ull >> (64 - lane));
   const V3<double> start = v3<double>(sc.start[0], sc.start[1], sc.start[2]);
 
+  const MarchK m = march_k(sc);
   int state = MS_NEED;
   int r = 0;
-  uint32_t pixel = 0;
+  uint32_t ray_hash = 0;
   V3<double> dir = v3<double>(0, 0, 0);
   RayState s = ray_start_state(sc);
   DECall<T> call;
   T dist = 0;
   int object = OBJ_FRACTAL;
+  bool early = false;  // the estimate ended in begin_de, without iterating
   LaneCount cnt = {0, 0};
-  int missed = 0;
 
   auto begin_de = [&]() {
-    march_before_de(sc, start, dir, s);
+    march_before_de(m, start, dir, s);
     DEInfo info;
-    state = MS_ITER;
-    if (de_call_begin<T, F, Plain, kAlg, IP>(f, cvt<T>(s.point), (T)s.thr, N, minN, false, call, dist, info)) {
-      state = MS_DONE;
-      object = info.object | (info.iters << 3);
-      cnt.de_calls += 1;
-    }
+    const V3<T> p = cvt<T>(s.point);
+    early = de_call_begin<T, F, Plain, kAlg, IP>(f, p, (T)s.thr, N, minN, false, call, dist, info);
+    state = early ? MS_DONE : MS_ITER;
+    if (early) object = info.object | (info.iters << 3);
   };
 
   for (;;) {
@@ -457,7 +362,7 @@ __device__ __forceinline__ void march_body(const DevScene *__restrict__ scp, Ban
           // a cancelled band's remaining rays take the empty record of a
           // cut ray, so later kernels read defined (if meaningless) values
           const bool cut = stop || view_vector(sc, x, y, dir);
-          pixel = sc.pixel_base + (uint32_t)p;
+          ray_hash = jitter_ray(sc.jitter_seed, sc.frame_no, sc.pixel_base + (uint32_t)p);
           s = ray_start_state(sc);
           if (cut) {
             MarchOut o;
@@ -473,24 +378,24 @@ __device__ __forceinline__ void march_body(const DevScene *__restrict__ scp, Ban
     }
 
     if (state == MS_ITER) {
-      DEInfo info;
       bool fin = false;
 #pragma unroll
-      for (int k = 0; k < kMarchIters && !fin; k++)
-        fin = de_call_step<T, F, Plain, kAlg, IP>(f, call, (T)s.thr, N, minN, false, dist, info);
-      if (fin) {
-        state = MS_DONE;
-        object = info.object | (info.iters << 3);
-        cnt.de_calls += 1;
-        cnt.iterations += (uint32_t)info.work;
-      }
+      for (int k = 0; k < kMarchIters && !fin; k++) fin = de_call_step<T, F, Plain, kAlg, IP>(f, call, N);
+      if (fin) state = MS_DONE;
     }
 
     const unsigned long long m_done2 = __ballot(state == MS_DONE);
     const unsigned long long m_iter2 = __ballot(state == MS_ITER);
     const int n_done2 = __popcll(m_done2), n_iter2 = __popcll(m_iter2);
     if (n_done2 && (4 * n_done2 >= n_done2 + n_iter2 || n_iter2 == 0) && state == MS_DONE) {
-      const int out = march_after_de<T, RT>(sc, s, (double)dist, object, pixel, ray_records<RT>(b, r, stats));
+      cnt.de_calls += 1;
+      if (!early) {
+        DEInfo info;
+        dist = de_call_end<T, F, Plain, kAlg, IP>(f, call, (T)s.thr, N, minN, false, info);
+        object = info.object | (info.iters << 3);
+        cnt.iterations += (uint32_t)info.work;
+      }
+      const int out = march_after_de(m, s, (double)dist, object, ray_hash, ray_records<RT>(b, r, stats));
       if (out == SO_CONTINUE) {
         begin_de();
       } else if (out == SO_MISS) {
@@ -521,52 +426,327 @@ __device__ __forceinline__ void march_body(const DevScene *__restrict__ scp, Ban
   v[ST_MARCH_DE] = cnt.de_calls;
   v[ST_MARCH_ITERS] = cnt.iterations;
   flush_stats(stats, v);
-  (void)missed;
 }
 
-template <class T, class RT, int F, bool Plain, int IP = 0>
+template <int F, int Plain, int IP>
 __global__ void __launch_bounds__(kBlock) k_march(const DevScene *__restrict__ scp, BandBufs b, int band_first,
                                                   int band_rays, unsigned long long *stats) {
-  march_body<T, RT, F, Plain, IP>(scp, b, band_first, band_rays, stats);
+  march_body<F, Plain, IP>(scp, b, band_first, band_rays, stats);
 }
 
 
-// FP64 continuation of the handed-over rays: one lane per ray, a grid-stride
-// loop over the hand-over list whose length the march left in the band
-// counters.
-template <class RT, int F, int IP = 0>
-__global__ void __launch_bounds__(kBlock) k_march_fix(const DevScene *__restrict__ scp, BandBufs b, int band_first,
-                                                      unsigned long long *stats) {
+// ---------------------------------------------------------- FP64 march
+// RayMarching (src/Render3D.cpp:79-199) in FP64, march, binary search and
+// (hit_refine) root refinement, one ray per lane and one distance estimate
+// at a time: every lane is in one phase of its own ray, and when its estimate
+// completes the phase's rule picks the next point or ends the ray, so lanes of
+// one wave march, search and start new rays side by side.
+//
+// One kernel for all FP64 rays.  As two kernels (march, then a lane-per-ray
+// loop over the hits for the search) the search took as long as its slowest
+// lane per wave at 25-30% active lanes and 256 registers with up to 1500 bytes
+// of scratch, ran every hit's last estimate twice, and a frame waited for the
+// slowest ray of each kernel in turn.
+//   kRays  the band's primary rays from their start (FP64 march modes)
+//   kHand  rays the FP32 march handed over, from the step it stopped at; those
+//          whose result FP32 error could have changed are listed for kRedo
+//   kRedo  the listed rays from their start
+//   kRefl  a reflection level's rays, each with its own start and threshold
+enum : int { kRays = 0, kHand = 1, kRedo = 2, kRefl = 3 };
+enum : int { PH_MARCH = 0, PH_SEARCH = 1, PH_PLUS = 2, PH_MINUS = 3, PH_ROOT = 4 };
+
+// IP: the integer power of the Mandelbulb when fixed at compile time (8).
+template <class RT, int F, int Plain, int IP, int Src>
+__device__ __forceinline__ void march64_body(const DevScene *__restrict__ scp, BandBufs b, int band_first,
+                                             int band_rays, int lane_cap, unsigned long long *stats) {
+#pragma clang fp contract(off)
+  // integer-power Mandelbulb iterations without inverse trig wherever the
+  // records are FP32; the FP64 mode keeps the trigonometric form
+  constexpr bool kAlg = sizeof(RT) < 8 || IP != 0;
   const DevScene &sc = *scp;
-  const long long n_hand = (long long)b.counters[CNT_HAND];
+  // the power-8 variants read a few formula constants in every iteration: a
+  // local copy keeps them in registers (the pass's stores and atomics keep
+  // the compiler from hoisting loads of the scene block out of the loop)
+  const FractalK<double> f_local = (Plain && IP) ? sc.fd : FractalK<double>{};
+  const FractalK<double> &f = (Plain && IP) ? f_local : sc.fd;
+  const MarchK m = march_k(sc);
+  const int N = sc.N, minN = sc.minN;
+  const int lane = __lane_id();
+  const unsigned long long lt_mask = (lane == 0) ? 0ull : (~0ull >> (64 - lane));
+  const long long n_items = Src == kRays ? (long long)band_rays
+                                         : (long long)b.counters[Src == kRedo ? CNT_REDO : CNT_HAND];
+  unsigned long long *const queue = &b.counters[Src == kRays ? CNT_RAYQ : Src == kRedo ? CNT_REDOQ : CNT_HANDQ];
+  const double search_limit = 1.0 - 0.01 * m.quality;
+  const bool hit_refine = sc.hit_refine != 0;
+  const double c0 = 1.0 - 0.005 * m.quality;
+  const double kthr = m.resolution * m.persp / m.quality;
+
+  int state = lane < lane_cap ? MS_NEED : MS_EXHAUSTED;
+  int phase = PH_MARCH;
+  int r = 0, j = 0;
+  uint32_t ray_hash = 0;
+  V3<double> start = v3<double>(sc.start[0], sc.start[1], sc.start[2]);
+  V3<double> dir = v3<double>(0, 0, 0);
+  RayState s = ray_start_state(sc);
+  DECall<double> call;
+  // the estimate, the threshold of the search, its step (the refinement: the
+  // estimate ahead of the root)
+  double dist = 0, thr = 0, step = 0;
+  double prev_dist = 0, prev_scan = 0, margin = 0;
+  bool early = false, ambiguous = false, have_prev = false, below = false;
+  int early_obj = 0;  // object and iterations << 3 of an early estimate
   LaneCount cnt = {0, 0};
   unsigned long long hits = 0, missed = 0, redo = 0;
-  const V3<double> start = v3<double>(sc.start[0], sc.start[1], sc.start[2]);
-  for (long long h = (long long)blockIdx.x * kBlock + threadIdx.x; h < n_hand; h += (long long)gridDim.x * kBlock) {
-    const int r = b.hand_ray[h];
-    const int p = band_first + r;
-    const int x = p % sc.width, y = p / sc.width;
-    V3<double> dir;
-    view_vector(sc, x, y, dir);
-    const uint32_t pixel = sc.pixel_base + (uint32_t)p;
-    RayState s = ray_start_state(sc);
-    s.i = b.hand_i[h];
-    s.scan = b.hand_scan[h];
-    s.step = b.hand_step[h];
-    s.drift = b.hand_drift[h];
-    s.dist = b.hand_dist[h];
-    const RecPlanes<RT> rec = ray_records<RT>(b, r, stats);
+
+  // start the estimate at distance t along the ray (detail size s.thr)
+  auto begin_de = [&](double t) {
+#pragma clang fp contract(off)
+    const V3<double> p = start + dir * t;
+    DEInfo info;
+    early = de_call_begin<double, F, Plain, kAlg, IP>(f, p, s.thr, N, minN, false, call, dist, info);
+    state = early ? MS_DONE : MS_ITER;
+    if (early) {
+      early_obj = info.object | (info.iters << 3);
+      cnt.iterations += (uint32_t)info.work;
+    }
+  };
+  // step s.i of the march
+  auto begin_march = [&]() {
+#pragma clang fp contract(off)
+    march_before_de(m, start, dir, s);
+    thr = s.thr;
+    phase = PH_MARCH;
+    begin_de(s.scan);
+  };
+  auto finish = [&](bool found) {
+#pragma clang fp contract(off)
     MarchOut o;
-    bool ambiguous = false;
-    march_continue_f64<RT, F, false, IP>(sc, start, dir, pixel, rec, s, o, cnt, ambiguous);
-    if (ambiguous) {
-      // re-marched from the start by k_march_redo
-      b.redo_list[atomicAdd(&b.counters[CNT_REDO], 1ull)] = r;
-      redo++;
-    } else {
-      write_ray(b, r, o);
-      hits += o.found;
-      missed += o.missed;
+    o.point = start + dir * s.scan;
+    if (!found) o.point = s.point;  // the last estimate's
+    o.scan = s.scan;
+    o.distThresh = thr;
+    o.dist = found ? dist : s.dist;
+    o.buffCount = s.i;
+    o.object = s.object;
+    o.found = found;
+    o.missed = false;
+    write_ray(b, r, o);
+    hits += found;
+    missed += found && below;
+    state = MS_NEED;
+  };
+  // The next point of the binary search from the estimate `dist` at s.scan,
+  // or true at its end (src/Render3D.cpp:163-183).
+  auto search = [&]() -> bool {
+#pragma clang fp contract(off)
+    bool end = j >= 20;
+    if (!end) {
+      if constexpr (Src == kHand) {
+        if (step > 5e-6 * s.scan && (fabs(dist - thr) < margin || fabs(dist - thr * search_limit) < margin))
+          ambiguous = true;
+      }
+      end = dist < thr && dist > thr * search_limit;
+    }
+    if (!end) {
+      if constexpr (Src == kHand) {
+        prev_dist = dist;
+        prev_scan = s.scan;
+        have_prev = true;
+      }
+      if (dist > thr) s.scan += step;
+      else if (dist < thr * search_limit) s.scan -= step;
+      thr = march_thr(m, s.scan, s.thr0);
+      step *= 0.5;
+      j++;
+      phase = PH_SEARCH;
+      begin_de(s.scan);
+      return false;
+    }
+    if constexpr (Src == kHand) {
+      if (ambiguous && have_prev) {
+        const double g = fabs(dist - prev_dist) / fmax(fabs(s.scan - prev_scan), 1e-300);
+        const double W = (0.01 * m.quality * thr + 2.0 * margin) / fmax(g, 1e-12);
+        ambiguous = W > kRedoTol * s.scan;
+      }
+    }
+    j = 0;
+    return true;
+  };
+  // Newton steps on F(t) = dist(t) - c0 thr(t), c0 the middle of the band,
+  // with a central-difference slope; each step at most one threshold long; true when settled
+  auto refine = [&]() -> bool {
+#pragma clang fp contract(off)
+    const double f0 = dist - c0 * kthr * s.scan;
+    if (j < 8 && fabs(f0) > 1e-13 * kthr * s.scan) {
+      const double eps = 1e-3 * kthr * s.scan;
+      prev_dist = dist;
+      phase = PH_PLUS;
+      begin_de(s.scan + eps);
+      return false;
+    }
+    thr = s.scan * kthr;
+    return true;
+  };
+
+  for (;;) {
+    const unsigned long long m_need = __ballot(state == MS_NEED);
+    const unsigned long long m_iter = __ballot(state == MS_ITER);
+    const unsigned long long m_done = __ballot(state == MS_DONE);
+    if (!(m_need | m_iter | m_done)) break;
+    const int n_need = __popcll(m_need), n_iter = __popcll(m_iter), n_done = __popcll(m_done);
+
+    if (n_need && (4 * n_need >= n_need + n_iter + n_done || n_iter + n_done == 0)) {
+      unsigned long long base = 0;
+      int stop = 0;
+      if (lane == 0) {
+        if constexpr (Src == kRays) base = take_work(b, queue, (unsigned long long)n_need, 12, stop);
+        else base = atomicAdd(queue, (unsigned long long)n_need);
+      }
+      base = __shfl(base, 0);
+      stop = __shfl(stop, 0);
+      if (state == MS_NEED) {
+        const unsigned long long mine = base + (unsigned long long)__popcll(m_need & lt_mask);
+        if (mine >= (unsigned long long)n_items) {
+          state = MS_EXHAUSTED;
+        } else {
+          r = Src == kRays ? (int)mine : Src == kRedo ? b.redo_list[mine] : b.hand_ray[mine];
+          s = ray_start_state(sc);
+          ray_hash = jitter_ray(sc.jitter_seed, sc.frame_no, sc.pixel_base + (uint32_t)(band_first + r));
+          bool cut_ray = false;
+          if constexpr (Src == kRefl) {
+            b.ovf_off[r] = -1;
+            start = v3<double>(b.ray_o[3 * (long long)r], b.ray_o[3 * (long long)r + 1], b.ray_o[3 * (long long)r + 2]);
+            dir = v3<double>(b.ray_d[3 * (long long)r], b.ray_d[3 * (long long)r + 1], b.ray_d[3 * (long long)r + 2]);
+            s.thr0 = b.ray_t0[r];
+          } else {
+            const int p = band_first + r;
+            // a cancelled band's remaining rays take the empty record of a
+            // cut ray, so later kernels read defined (if meaningless) values
+            cut_ray = view_vector(sc, p % sc.width, p / sc.width, dir);
+            if constexpr (Src == kRays) {
+              b.ovf_off[r] = -1;
+              cut_ray = cut_ray || stop;
+            } else {
+              cut_ray = false;  // the march handed it over
+            }
+          }
+          if constexpr (Src == kHand) {
+            s.i = b.hand_i[mine];
+            s.scan = b.hand_scan[mine];
+            s.step = b.hand_step[mine];
+            s.drift = b.hand_drift[mine];
+            s.dist = b.hand_dist[mine];
+            margin = 4.0 * sqrt(s.drift);  // s.drift: variance of the FP32 scan deviation
+            prev_dist = s.dist;
+            prev_scan = s.scan - s.step;  // the step before s.i
+            have_prev = s.i > 0;
+            ambiguous = false;
+          }
+          if (cut_ray) {
+            MarchOut o;
+            o.point = v3<double>(0, 0, 0);
+            o.scan = 0; o.distThresh = 0; o.dist = 0; o.buffCount = 0; o.object = OBJ_FRACTAL;
+            o.found = false; o.missed = false;
+            write_ray(b, r, o);
+          } else {
+            begin_march();
+          }
+        }
+      }
+    }
+
+    if (state == MS_ITER) {
+      bool fin = false;
+#pragma unroll
+      for (int q = 0; q < kMarchIters && !fin; q++) fin = de_call_step<double, F, Plain, kAlg, IP>(f, call, N);
+      if (fin) state = MS_DONE;
+    }
+
+    const unsigned long long m_done2 = __ballot(state == MS_DONE);
+    const unsigned long long m_iter2 = __ballot(state == MS_ITER);
+    const int n_done2 = __popcll(m_done2), n_iter2 = __popcll(m_iter2);
+    if (n_done2 && (4 * n_done2 >= n_done2 + n_iter2 || n_iter2 == 0) && state == MS_DONE) {
+      int obj_it = early_obj;
+      if (!early) {
+        DEInfo info;
+        dist = de_call_end<double, F, Plain, kAlg, IP>(f, call, s.thr, N, minN, false, info);
+        obj_it = info.object | (info.iters << 3);
+        cnt.iterations += (uint32_t)info.work;
+      }
+      cnt.de_calls += 1;
+      bool found = false, settled = false;
+      if (phase != PH_PLUS && phase != PH_MINUS) s.object = obj_it & 7;
+      if (phase == PH_MARCH) {
+        const double raw = dist;
+        if (dist > 3.0) dist = 3.0;
+        if constexpr (Src == kHand) {
+          if (fabs(dist - s.thr) < margin) ambiguous = true;
+        }
+        if (dist < s.thr) {
+          if constexpr (Src == kRays) {
+            // the call counters count this estimate for the march and for the
+            // search that starts from it
+            cnt.de_calls += 1;
+            if (!early) cnt.iterations += (uint32_t)(call.it.L < N ? call.it.L + 1 : N);
+          }
+          below = dist < 0.1 * s.thr;
+          step = s.step * 0.5;
+          j = 0;
+          found = search();
+        } else {
+          const double jf = m.jitter ? jitter_factor(jitter_draw(ray_hash, (uint32_t)s.i)) : 1.0;
+          const double old_step = s.step;
+          s.step = (dist - m.below * s.thr) * m.DE_factor * jf;
+          ray_records<RT>(b, r, stats).put(s.i, old_step, raw, s.thr, obj_it >> 3);
+          if constexpr (Src == kHand) {
+            prev_dist = dist;
+            prev_scan = s.scan;
+            have_prev = true;
+          }
+          s.scan += s.step;
+          s.dist = dist;
+          s.i++;
+          if (s.scan > m.far || s.i >= 10000) finish(false);
+          else begin_march();
+        }
+      } else if (phase == PH_SEARCH) {
+        found = search();
+      } else if (phase == PH_PLUS) {
+        step = dist;
+        phase = PH_MINUS;
+        const double eps = 1e-3 * kthr * s.scan;
+        begin_de(s.scan - eps);
+      } else if (phase == PH_MINUS) {
+        const double eps = 1e-3 * kthr * s.scan;
+        const double g = (step - dist) / (2.0 * eps) - c0 * kthr;
+        const double f0 = prev_dist - c0 * kthr * s.scan;
+        if (!(fabs(g) > 0.0)) {
+          dist = prev_dist;
+          thr = s.scan * kthr;
+          settled = true;
+        } else {
+          double dt = -f0 / g;
+          const double lim = kthr * s.scan;
+          dt = dt > lim ? lim : (dt < -lim ? -lim : dt);
+          s.scan += dt;
+          j++;
+          phase = PH_ROOT;
+          begin_de(s.scan);
+        }
+      } else {
+        settled = refine();
+      }
+      if (found) settled = hit_refine && !m.constant_thresh ? refine() : true;
+      if (settled) {
+        if (Src == kHand && ambiguous) {
+          // marched again from the start (kRedo)
+          b.redo_list[atomicAdd(&b.counters[CNT_REDO], 1ull)] = r;
+          redo++;
+          state = MS_NEED;
+        } else {
+          finish(true);
+        }
+      }
     }
   }
   unsigned long long v[ST_COUNT] = {0};
@@ -578,41 +758,13 @@ __global__ void __launch_bounds__(kBlock) k_march_fix(const DevScene *__restrict
   flush_stats(stats, v);
 }
 
-// FP64 march from the start of the rays k_march_fix listed (FP32_MARCH rays
-// whose result FP32 error could have changed).  A kernel of its own: with
-// the redo as a second inlined pass of the march loop inside k_march_fix,
-// the gfx950 build returned found = false for some lanes whose rays were
-// found, depending on which rays shared a wave (the Mandelbox FP32_MARCH
-// parity test covers it).
-template <class RT, int F>
-__global__ void __launch_bounds__(kBlock) k_march_redo(const DevScene *__restrict__ scp, BandBufs b, int band_first,
-                                                       unsigned long long *stats) {
-  const DevScene &sc = *scp;
-  const long long n_redo = (long long)b.counters[CNT_REDO];
-  LaneCount cnt = {0, 0};
-  unsigned long long hits = 0, missed = 0;
-  const V3<double> start = v3<double>(sc.start[0], sc.start[1], sc.start[2]);
-  for (long long h = (long long)blockIdx.x * kBlock + threadIdx.x; h < n_redo; h += (long long)gridDim.x * kBlock) {
-    const int r = b.redo_list[h];
-    const int p = band_first + r;
-    const int x = p % sc.width, y = p / sc.width;
-    V3<double> dir;
-    view_vector(sc, x, y, dir);
-    const uint32_t pixel = sc.pixel_base + (uint32_t)p;
-    const RecPlanes<RT> rec = ray_records<RT>(b, r, stats);
-    MarchOut o;
-    bool unused = false;
-    march_continue_f64<RT, F>(sc, start, dir, pixel, rec, ray_start_state(sc), o, cnt, unused);
-    write_ray(b, r, o);
-    hits += o.found;
-    missed += o.missed;
-  }
-  unsigned long long v[ST_COUNT] = {0};
-  v[ST_MARCH_DE] = cnt.de_calls;
-  v[ST_MARCH_ITERS] = cnt.iterations;
-  v[ST_HITS] = hits;
-  v[ST_MISSED] = missed;
-  flush_stats(stats, v);
+// lane_cap: lanes of a wave that take rays (a small band spreads over more
+// waves, whose passes then wait for fewer lanes)
+template <class RT, int F, int Plain, int IP, int Src>
+__global__ void __launch_bounds__(kBlock, Plain && (F != 2 || IP) ? 4 : 1)
+    k_march64(const DevScene *__restrict__ scp, BandBufs b, int band_first, int band_rays, int lane_cap,
+              unsigned long long *stats) {
+  march64_body<RT, F, Plain, IP, Src>(scp, b, band_first, band_rays, lane_cap, stats);
 }
 
 template <class T>
@@ -817,7 +969,7 @@ struct AOPolicy {
   static constexpr int need_div = f64 ? MBR_AO64_NEED_DIV : MBR_AO_NEED_DIV;
 };
 
-template <class T, int F, bool Deep, bool Plain, int IP = 0>
+template <class T, int F, bool Deep, int Plain, int IP = 0>
 __device__ __forceinline__ void ao_body(const DevScene *__restrict__ scp, BandBufs b, AODev ao, SurfBufs<T> sb,
                                         unsigned long long *stats) {
   const DevScene &sc = *scp;
@@ -848,6 +1000,7 @@ __device__ __forceinline__ void ao_body(const DevScene *__restrict__ scp, BandBu
   T r = 0, start_dist = 0, end_dist = 1, detail = 0, thr_f = 0;
   T dist = 0;
   int mi = 0, guard = 0;
+  bool early = false;  // the estimate ended in begin_de, without iterating
   DECall<T> call;
   LaneCount cnt = {0, 0};
   unsigned long long ao_steps = 0;
@@ -855,23 +1008,18 @@ __device__ __forceinline__ void ao_body(const DevScene *__restrict__ scp, BandBu
   // start the distance estimate at P + dir * r; DONE when no iteration runs
   auto begin_de = [&]() {
     DEInfo info;
-    state = AO_ITER;
-    bool done;
+    const V3<T> p = P + dir * r;
     if constexpr (Deep && sizeof(T) < 8) {
       if (deep)
-        done = de_call_begin_p64<F>(sc.fd, f, P64 + cvt<double>(dir) * (double)r, detail, N, minN, false, call, dist,
-                                    info);
+        early = de_call_begin_p64<F>(sc.fd, f, P64 + cvt<double>(dir) * (double)r, detail, N, minN, false, call, dist,
+                                     info);
       else
-        done = de_call_begin<T, F, Plain, kAlg, IP>(f, P + dir * r, detail, N, minN, false, call, dist,
-                                                               info);
+        early = de_call_begin<T, F, Plain, kAlg, IP>(f, p, detail, N, minN, false, call, dist, info);
     } else {
-      done = de_call_begin<T, F, Plain, kAlg, IP>(f, P + dir * r, detail, N, minN, false, call, dist, info);
+      early = de_call_begin<T, F, Plain, kAlg, IP>(f, p, detail, N, minN, false, call, dist, info);
     }
-    if (done) {
-      state = AO_DONE;
-      mi = info.max_iter;
-      cnt.de_calls += 1;
-    }
+    state = early ? AO_DONE : AO_ITER;
+    if (early) mi = info.max_iter;
   };
 
   for (;;) {
@@ -938,23 +1086,24 @@ __device__ __forceinline__ void ao_body(const DevScene *__restrict__ scp, BandBu
     }
 
     if (state == AO_ITER) {
-      DEInfo info;
       bool fin = false;
 #pragma unroll
       for (int k = 0; k < AOPolicy<T>::iters && !fin; k++)
-        fin = de_call_step<T, F, Plain, kAlg, IP>(f, call, detail, N, minN, false, dist, info);
-      if (fin) {
-        state = AO_DONE;
-        mi = info.max_iter;
-        cnt.de_calls += 1;
-        cnt.iterations += (uint32_t)info.work;
-      }
+        fin = de_call_step<T, F, Plain, kAlg, IP>(f, call, N);
+      if (fin) state = AO_DONE;
     }
 
     const unsigned long long m_done2 = __ballot(state == AO_DONE);
     const unsigned long long m_iter2 = __ballot(state == AO_ITER);
     const int n_done2 = __popcll(m_done2), n_iter2 = __popcll(m_iter2);
     if (n_done2 && (AOPolicy<T>::done_div * n_done2 >= n_done2 + n_iter2 || n_iter2 == 0) && state == AO_DONE) {
+      cnt.de_calls += 1;
+      if (!early) {
+        DEInfo info;
+        dist = de_call_end<T, F, Plain, kAlg, IP>(f, call, detail, N, minN, false, info);
+        mi = info.max_iter;
+        cnt.iterations += (uint32_t)info.work;
+      }
       // one step of the AO ray (src/shaders.cpp:625-662)
       ao_steps++;
       if (dist < thr_f || mi) {
@@ -983,18 +1132,18 @@ __device__ __forceinline__ void ao_body(const DevScene *__restrict__ scp, BandBu
   flush_stats(stats, v);
 }
 
-template <class T, int F, bool Deep, bool Plain, int IP = 0>
+template <class T, int F, bool Deep, int Plain, int IP = 0>
 __global__ void __launch_bounds__(kBlock) k_ao(const DevScene *__restrict__ scp, BandBufs b, AODev ao,
                                                SurfBufs<T> sb, unsigned long long *stats) {
   ao_body<T, F, Deep, Plain, IP>(scp, b, ao, sb, stats);
 }
 
 // The FP32 plain variant (the benchmarked AO pass) held to 6 waves per SIMD.
-template <class T, int F, int IP = 0>
+template <class T, int F, int Plain, int IP>
 __global__ void __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(6, 8)))
     k_ao_f32_plain(const DevScene *__restrict__ scp, BandBufs b, AODev ao, SurfBufs<T> sb,
                    unsigned long long *stats) {
-  ao_body<T, F, false, true, IP>(scp, b, ao, sb, stats);
+  ao_body<T, F, false, Plain, IP>(scp, b, ao, sb, stats);
 }
 
 template <class T, class RT>
@@ -1397,41 +1546,6 @@ __global__ void __launch_bounds__(kBlock) k_refl_setup(const DevScene *__restric
   flush_stats(stats, v);
 }
 
-// The FP64 march (RayMarching with its binary search) of a reflection
-// level's rays, with the same step jitter as the pixel's primary ray.
-template <int F>
-__global__ void __launch_bounds__(kBlock) k_refl_march(const DevScene *__restrict__ scp, BandBufs b, int band_first,
-                                                       unsigned long long *stats) {
-  const DevScene &sc = *scp;
-  const long long n_rays = (long long)b.counters[CNT_HAND];
-  LaneCount cnt = {0, 0};
-  unsigned long long hits = 0, missed = 0;
-  for (long long h = (long long)blockIdx.x * kBlock + threadIdx.x; h < n_rays; h += (long long)gridDim.x * kBlock) {
-    const int r = b.hand_ray[h];
-    b.ovf_off[r] = -1;
-    const V3<double> start = v3<double>(b.ray_o[3 * (long long)r], b.ray_o[3 * (long long)r + 1],
-                                        b.ray_o[3 * (long long)r + 2]);
-    const V3<double> dir = v3<double>(b.ray_d[3 * (long long)r], b.ray_d[3 * (long long)r + 1],
-                                      b.ray_d[3 * (long long)r + 2]);
-    const uint32_t pixel = sc.pixel_base + (uint32_t)(band_first + r);
-    RayState s = ray_start_state(sc);
-    s.thr0 = b.ray_t0[r];
-    MarchOut o;
-    bool ambiguous = false;
-    march_continue_f64<double, F, true>(sc, start, dir, pixel, ray_records<double>(b, r, stats), s, o, cnt,
-                                        ambiguous);
-    write_ray(b, r, o);
-    hits += o.found;
-    missed += o.missed;
-  }
-  unsigned long long v[ST_COUNT] = {0};
-  v[ST_MARCH_DE] = cnt.de_calls;
-  v[ST_MARCH_ITERS] = cnt.iterations;
-  v[ST_HITS] = hits;
-  v[ST_MISSED] = missed;
-  flush_stats(stats, v);
-}
-
 // Per pixel: the levels from the last one reached down to the primary ray
 // (src/Render3D.cpp:501-571): each shaded surface (or background) blended
 // with the next level's result by its reflection coefficient, then that
@@ -1558,6 +1672,38 @@ __global__ void __launch_bounds__(kBlock) k_refl_finish(const DevScene *__restri
 }
 
 // ---------------------------------------------------------------- launch
+// Calls go(F, Plain, IP) (as integral constants) with the compiled variant of
+// a scene: the formula's kernels (0: generic), without the optional terms of
+// the distance estimate where the scene has none, and with the Mandelbulb's
+// power 8 fixed where the trig-free iteration is wanted (ip8).
+template <class Go>
+static inline void march_variant(int formula, int plain, bool ip8, Go go) {
+  std::integral_constant<int, 0> z;
+  std::integral_constant<int, 2> f2;
+  std::integral_constant<int, 7> f7;
+  std::integral_constant<int, 8> f8;
+  std::integral_constant<int, kPlain> yes;
+  std::integral_constant<int, kOptions> no;
+  std::integral_constant<int, kUnrotated> box;
+  if (formula_generic(formula)) return go(z, no, z);
+  if (plain) {
+    if (formula == 7) return go(f7, yes, z);
+    if (formula == 8) return plain == kUnrotated ? go(f8, box, z) : go(f8, yes, z);
+    return ip8 ? go(f2, yes, f8) : go(f2, yes, z);
+  }
+  if (formula == 7) return go(f7, no, z);
+  if (formula == 8) return go(f8, no, z);
+  return ip8 ? go(f2, no, f8) : go(f2, no, z);
+}
+
+// Lanes per wave of a march over n rays: a band with fewer than 64 rays for
+// each of the two waves per SIMD that the FP64 units need to stay busy spreads
+// over that many waves, at least 4 rays each.
+static inline int march_lanes(int n, int persist_blocks) {
+  const int waves = std::max(1, persist_blocks);  // 8 workgroups per CU: two waves per SIMD
+  return std::min(64, std::max(4, (n + waves - 1) / waves));
+}
+
 static inline dim3 grid_for(int n) { return dim3((unsigned)((n + kBlock - 1) / kBlock)); }
 
 #if MBR_UNIT(5)
@@ -1585,13 +1731,17 @@ hipError_t launch_refl_march(const DevScene *sc, const BandBufs &next, int band_
                              unsigned long long *stats, hipStream_t s) {
   const dim3 grid((unsigned)std::max(1, blocks));
   if (formula_generic(formula))
-    hipLaunchKernelGGL((k_refl_march<0>), grid, dim3(kBlock), 0, s, sc, next, band_first, stats);
+    hipLaunchKernelGGL((k_march64<double, 0, 0, 0, kRefl>), grid, dim3(kBlock), 0, s, sc, next, band_first, 0, 64,
+                       stats);
   else if (formula == 7)
-    hipLaunchKernelGGL((k_refl_march<7>), grid, dim3(kBlock), 0, s, sc, next, band_first, stats);
+    hipLaunchKernelGGL((k_march64<double, 7, 0, 0, kRefl>), grid, dim3(kBlock), 0, s, sc, next, band_first, 0, 64,
+                       stats);
   else if (formula == 8)
-    hipLaunchKernelGGL((k_refl_march<8>), grid, dim3(kBlock), 0, s, sc, next, band_first, stats);
+    hipLaunchKernelGGL((k_march64<double, 8, 0, 0, kRefl>), grid, dim3(kBlock), 0, s, sc, next, band_first, 0, 64,
+                       stats);
   else
-    hipLaunchKernelGGL((k_refl_march<2>), grid, dim3(kBlock), 0, s, sc, next, band_first, stats);
+    hipLaunchKernelGGL((k_march64<double, 2, 0, 0, kRefl>), grid, dim3(kBlock), 0, s, sc, next, band_first, 0, 64,
+                       stats);
   return hipGetLastError();
 }
 
@@ -1629,83 +1779,50 @@ hipError_t launch_march(int precision, const DevScene *sc, const BandBufs &b, in
   // generic formulas: FP64, or the FP64 march of FP32_FIXUP (FP32 records)
   if (formula_generic(formula) && precision > 1) return hipErrorInvalidValue;
   const dim3 grid((unsigned)std::max(1, persist_blocks));
-  auto run = [&](auto tag, auto rtag) {
-    using T = decltype(tag);
-    using RT = decltype(rtag);
-    auto go = [&](auto plain_tag) {
-      constexpr bool Pl = decltype(plain_tag)::value;
-      if constexpr (Pl) {
-        // the caller sets ip8 only where the trig-free iteration is wanted
-        if (formula == 2 && ip8) {
-          hipLaunchKernelGGL((k_march<T, RT, 2, true, 8>), grid, dim3(kBlock), 0, s, sc, b, band_first, band_rays,
-                             stats);
-          return;
-        }
-      }
-      if (formula == 7)
-        hipLaunchKernelGGL((k_march<T, RT, 7, Pl>), grid, dim3(kBlock), 0, s, sc, b, band_first, band_rays, stats);
-      else if (formula == 8)
-        hipLaunchKernelGGL((k_march<T, RT, 8, Pl>), grid, dim3(kBlock), 0, s, sc, b, band_first, band_rays, stats);
-      else
-        hipLaunchKernelGGL((k_march<T, RT, 2, Pl>), grid, dim3(kBlock), 0, s, sc, b, band_first, band_rays, stats);
+  if (precision == 2) {
+    auto go = [&](auto f_tag, auto plain_tag, auto ip_tag) {
+      constexpr int F = decltype(f_tag)::value;
+      if constexpr (F != 0)
+        hipLaunchKernelGGL((k_march<F, decltype(plain_tag)::value, decltype(ip_tag)::value>), grid, dim3(kBlock), 0,
+                           s, sc, b, band_first, band_rays, stats);
     };
-    if (formula_generic(formula)) {
-      if constexpr (std::is_same<T, double>::value)
-        hipLaunchKernelGGL((k_march<double, RT, 0, false>), grid, dim3(kBlock), 0, s, sc, b, band_first, band_rays,
-                           stats);
-      return;
-    }
-    if (plain) go(std::true_type{});
-    else go(std::false_type{});
-  };
-  if (precision == 0) run(double{}, double{});
-  else if (precision == 1) run(double{}, float{});
-  else run(float{}, float{});
-  return hipGetLastError();
-}
-
-#endif  // march
-
-#if MBR_UNIT(1)
-hipError_t launch_march_fix(int precision, const DevScene *sc, const BandBufs &b, int band_first, int formula,
-                            int persist_blocks, unsigned long long *stats, hipStream_t s, bool ip8) {
-  const dim3 grid((unsigned)std::max(1, persist_blocks));
-  if (formula_generic(formula) && precision > 1) return hipErrorInvalidValue;
-  if (formula_generic(formula)) {
-    if (precision == 0)
-      hipLaunchKernelGGL((k_march_fix<double, 0>), grid, dim3(kBlock), 0, s, sc, b, band_first, stats);
-    else
-      hipLaunchKernelGGL((k_march_fix<float, 0>), grid, dim3(kBlock), 0, s, sc, b, band_first, stats);
+    march_variant(formula, plain, ip8, go);
     return hipGetLastError();
   }
+  const int lanes = march_lanes(band_rays, persist_blocks);
   auto run = [&](auto rtag) {
     using RT = decltype(rtag);
-    if (formula == 7)
-      hipLaunchKernelGGL((k_march_fix<RT, 7>), grid, dim3(kBlock), 0, s, sc, b, band_first, stats);
-    else if (formula == 8)
-      hipLaunchKernelGGL((k_march_fix<RT, 8>), grid, dim3(kBlock), 0, s, sc, b, band_first, stats);
-    else {
-      bool done = false;
-      if (ip8) {
-        hipLaunchKernelGGL((k_march_fix<RT, 2, 8>), grid, dim3(kBlock), 0, s, sc, b, band_first, stats);
-        done = true;
-      }
-      if (!done) hipLaunchKernelGGL((k_march_fix<RT, 2>), grid, dim3(kBlock), 0, s, sc, b, band_first, stats);
-    }
-    if (precision == 2) {
-      if (formula == 7)
-        hipLaunchKernelGGL((k_march_redo<RT, 7>), grid, dim3(kBlock), 0, s, sc, b, band_first, stats);
-      else if (formula == 8)
-        hipLaunchKernelGGL((k_march_redo<RT, 8>), grid, dim3(kBlock), 0, s, sc, b, band_first, stats);
-      else
-        hipLaunchKernelGGL((k_march_redo<RT, 2>), grid, dim3(kBlock), 0, s, sc, b, band_first, stats);
-    }
+    auto go = [&](auto f_tag, auto plain_tag, auto ip_tag) {
+      hipLaunchKernelGGL((k_march64<RT, decltype(f_tag)::value, decltype(plain_tag)::value, decltype(ip_tag)::value,
+                                    kRays>),
+                         grid, dim3(kBlock), 0, s, sc, b, band_first, band_rays, lanes, stats);
+    };
+    march_variant(formula, plain, ip8, go);
   };
   if (precision == 0) run(double{});
   else run(float{});
   return hipGetLastError();
 }
+#endif  // march
 
+#if MBR_UNIT(1)
+hipError_t launch_march_fix(const DevScene *sc, const BandBufs &b, int band_first, int formula, int plain,
+                            int persist_blocks, unsigned long long *stats, hipStream_t s, bool ip8) {
+  if (formula_generic(formula)) return hipErrorInvalidValue;
+  const dim3 grid((unsigned)std::max(1, persist_blocks));
+  auto hand = [&](auto f_tag, auto plain_tag, auto ip_tag) {
+    constexpr int F = decltype(f_tag)::value, IP = decltype(ip_tag)::value;
+    constexpr int Pl = decltype(plain_tag)::value;
+    if constexpr (F != 0) {
+      hipLaunchKernelGGL((k_march64<float, F, Pl, IP, kHand>), grid, dim3(kBlock), 0, s, sc, b, band_first, 0, 64,
+                         stats);
+      hipLaunchKernelGGL((k_march64<float, F, Pl, IP, kRedo>), grid, dim3(kBlock), 0, s, sc, b, band_first, 0, 64,
+                         stats);
+    }
+  };
+  march_variant(formula, plain, ip8, hand);
+  return hipGetLastError();
+}
 #endif  // continuation
 
 #if MBR_UNIT(4)
@@ -1768,38 +1885,18 @@ hipError_t shade_run(const DevScene *sc, const BandBufs &b, int band_first, AODe
     else
       hipLaunchKernelGGL((k_surface<T, 2, D>), grid, dim3(kBlock), 0, s, sc, b, band_first, sb, stats);
   };
-  auto aok = [&](auto deep_tag, auto plain_tag) {
+  // plain scenes take a variant without the optional terms' branches (and the
+  // scene constants they keep live); FP32 deep-zoom scenes the one that starts
+  // estimates in FP64
+  auto aok = [&](auto deep_tag, auto f_tag, auto plain_tag, auto ip_tag) {
     constexpr bool D = decltype(deep_tag)::value;
-    constexpr bool Pl = decltype(plain_tag)::value;
-    if constexpr (!D && Pl && std::is_same<T, float>::value) {
-      if (formula == 7)
-        hipLaunchKernelGGL((k_ao_f32_plain<T, 7>), grid, dim3(kBlock), 0, s, sc, b, ao, sb, stats);
-      else if (formula == 8)
-        hipLaunchKernelGGL((k_ao_f32_plain<T, 8>), grid, dim3(kBlock), 0, s, sc, b, ao, sb, stats);
-      else if (sbuf.ip8)
-        hipLaunchKernelGGL((k_ao_f32_plain<T, 2, 8>), grid, dim3(kBlock), 0, s, sc, b, ao, sb, stats);
-      else
-        hipLaunchKernelGGL((k_ao_f32_plain<T, 2>), grid, dim3(kBlock), 0, s, sc, b, ao, sb, stats);
-      return;
-    }
-    if constexpr (!D && !Pl) {
-      if (generic) {
-        hipLaunchKernelGGL((k_ao<T, 0, false, false>), grid, dim3(kBlock), 0, s, sc, b, ao, sb, stats);
-        return;
-      }
-    }
-    if constexpr (!D && Pl && std::is_same<T, double>::value) {
-      if (formula == 2 && sbuf.ip8) {  // FP64_DEMOIVRE
-        hipLaunchKernelGGL((k_ao<T, 2, false, true, 8>), grid, dim3(kBlock), 0, s, sc, b, ao, sb, stats);
-        return;
-      }
-    }
-    if (formula == 7)
-      hipLaunchKernelGGL((k_ao<T, 7, D, Pl>), grid, dim3(kBlock), 0, s, sc, b, ao, sb, stats);
-    else if (formula == 8)
-      hipLaunchKernelGGL((k_ao<T, 8, D, Pl>), grid, dim3(kBlock), 0, s, sc, b, ao, sb, stats);
+    constexpr int F = decltype(f_tag)::value, Pl = decltype(plain_tag)::value, IP = decltype(ip_tag)::value;
+    if constexpr (!D && Pl && std::is_same<T, float>::value)
+      hipLaunchKernelGGL((k_ao_f32_plain<T, F, Pl, IP>), grid, dim3(kBlock), 0, s, sc, b, ao, sb, stats);
+    else if constexpr (Pl)
+      hipLaunchKernelGGL((k_ao<T, F, D, Pl, IP>), grid, dim3(kBlock), 0, s, sc, b, ao, sb, stats);
     else
-      hipLaunchKernelGGL((k_ao<T, 2, D, Pl>), grid, dim3(kBlock), 0, s, sc, b, ao, sb, stats);
+      hipLaunchKernelGGL((k_ao<T, F, D, Pl>), grid, dim3(kBlock), 0, s, sc, b, ao, sb, stats);
   };
   // deep-zoom variants only for FP32 shading of scenes that need them
   const bool deep = sbuf.deep && sizeof(T) < 8 && !generic;
@@ -1828,12 +1925,13 @@ hipError_t shade_run(const DevScene *sc, const BandBufs &b, int band_first, AODe
     if (e != hipSuccess) return e;
   }
   if (sbuf.slow_ao) {
-    // plain scenes (no primitives, limits, interior mode, iteration
-    // threshold, pre-folds or Julia constant) take a variant without those
-    // branches and the scene constants they keep live
-    if (deep) aok(std::true_type{}, std::false_type{});
-    else if (sbuf.plain && !generic) aok(std::false_type{}, std::true_type{});
-    else aok(std::false_type{}, std::false_type{});
+    if (deep)
+      march_variant(formula, 0, false, [&](auto f, auto, auto) {
+        constexpr int F = decltype(f)::value;
+        if constexpr (F != 0) aok(std::true_type{}, f, std::integral_constant<int, kOptions>{}, std::integral_constant<int, 0>{});
+      });
+    else
+      march_variant(formula, sbuf.plain, sbuf.ip8, [&](auto f, auto pl, auto ip) { aok(std::false_type{}, f, pl, ip); });
   }
   if (ev_ao1) {
     hipError_t e = hipEventRecord(ev_ao1, s);

@@ -21,9 +21,10 @@ enum StatIdx {
 // Band counters (BandBufs::counters), zeroed on the device at band start:
 // hits appended, rays handed to the FP64 continuation, primary-ray queue,
 // overflow runs handed out, AO work queue, rays listed for the FP64 redo,
-// overflow chunks.
+// overflow chunks, the queues over the handed-over and the redo rays.
 enum CounterIdx {
-  CNT_HITS = 0, CNT_HAND = 1, CNT_RAYQ = 2, CNT_DIRS = 3, CNT_AOQ = 4, CNT_REDO = 5, CNT_CHUNKS = 6, CNT_COUNT = 8
+  CNT_HITS = 0, CNT_HAND = 1, CNT_RAYQ = 2, CNT_DIRS = 3, CNT_AOQ = 4, CNT_REDO = 5, CNT_CHUNKS = 6,
+  CNT_HANDQ = 7, CNT_REDOQ = 8, CNT_COUNT = 16
 };
 
 // Formulas of the render core; the generic ones (no kernels of their own)
@@ -111,7 +112,9 @@ hipError_t launch_zero(unsigned long long *p, int n, hipStream_t s);
 hipError_t launch_march(int precision, const DevScene *sc, const BandBufs &b, int band_first, int band_rays,
                         int formula, int plain, int persist_blocks, unsigned long long *stats, hipStream_t s,
                         bool ip8 = false);
-hipError_t launch_march_fix(int precision, const DevScene *sc, const BandBufs &b, int band_first, int formula,
+// FP32_MARCH only: the FP64 continuation of the rays the FP32 march handed
+// over, and the FP64 march of those it lists for a redo
+hipError_t launch_march_fix(const DevScene *sc, const BandBufs &b, int band_first, int formula, int plain,
                             int persist_blocks, unsigned long long *stats, hipStream_t s, bool ip8 = false);
 // Buffers of the shading launches (element type T = the path's precision).
 struct ShadeBufs {
