@@ -1215,6 +1215,9 @@ ShadeBufs frame_shade_bufs(Slot &sl, const DevScene &host, int formula, bool tri
   sbuf.aux = sl.sh_aux;
   sbuf.n = b.cap;
   sbuf.slow_ao = host.ao && !host.fast_ao;
+  sbuf.env = host.env_map;
+  sbuf.fast_ao_on = host.ao && host.fast_ao;
+  sbuf.shadow_fx = host.shadow && host.shadow_fx;
   sbuf.deep = host.deep;
   sbuf.plain = host.plain;
   sbuf.formula = formula;
@@ -1325,6 +1328,9 @@ ShadeBufs shade_bufs(Slot &sl, const DevScene &host, int formula) {
   sbuf.aux = sl.sh_aux;
   sbuf.n = sl.band.cap;
   sbuf.slow_ao = host.ao && !host.fast_ao;
+  sbuf.env = host.env_map;
+  sbuf.fast_ao_on = host.ao && host.fast_ao;
+  sbuf.shadow_fx = host.shadow && host.shadow_fx;
   sbuf.deep = 0;
   sbuf.plain = host.plain;
   sbuf.formula = formula;

@@ -109,10 +109,20 @@ MBR_HD void rotate_right(T *m, bool &ident, int axis, T angle) {
   ident = false;
 }
 
+// P: what the caller knows of the scene: kOptions nothing, kPlain that no
+// optional term is on (primitives, limits, interior mode, iteration
+// threshold, pre-folds, Julia constant), kUnrotated (Mandelbox) in addition
+// that its folds and its main rotation are not rotated.  The 19 rotation
+// matrices otherwise fill the scalar registers of every kernel that holds
+// the iteration (380-450 spills into vector lanes, read back in every pass).
+enum : int { kOptions = 0, kPlain = 1, kUnrotated = 2 };
+
 // G: the formulas of the generic path are compiled in (always in FP64; in
 // FP32 for the FP32 shading of the analytic generic formulas, whose kernels
 // ask for them, so that the FP32 kernels of formulas 2, 7 and 8 stay small).
-template <class T, int Mode, bool G = (sizeof(T) == 8)>
+// FF: the formula when the caller was compiled for one (then without G and
+// without hybrids), P what it knows of the scene.
+template <class T, int Mode, bool G = (sizeof(T) == 8), int FF = 0, int P = 0>
 MBR_HD T compute(const FractalK<T> &f, V3<T> z, int N, int *iter_count) {
 #pragma clang fp contract(off)
   using M = Math<T>;
@@ -128,14 +138,14 @@ MBR_HD T compute(const FractalK<T> &f, V3<T> z, int N, int *iter_count) {
   T tgladDE = 1;
   T tgladColor = 1;
   T orbitTrapTotal = 0;  // the fake lights' orbit-trap sum
-  V3<T> constant = f.julia_mode ? ld3(f.julia) : z * f.constant_factor;  // aexion rewrites it
+  V3<T> constant = (!P && f.julia_mode) ? ld3(f.julia) : z * f.constant_factor;  // aexion rewrites it
   T r = length_nc(z);
   T min = Mode == MODE_COLOURING ? T(3.0e38) : T(0);  // min radius of the orbit (1e200 in FP64)
   if (Mode == MODE_COLOURING && sizeof(T) == 8) min = T(1e200);
 
   for (L = 0; L < N; L++) {
-    int af = f.formula;  // the formula of this iteration (the hybrid sequence's, src/fractal.cpp:88-96)
-    if constexpr (sizeof(T) == 8) {
+    int af = FF ? FF : f.formula;  // the formula of this iteration (the hybrid sequence's, src/fractal.cpp:88-96)
+    if constexpr (sizeof(T) == 8 && FF == 0) {
       if (f.formula == 12) {
         // the sequence has N entries; longer runs (normals at 5N, colouring
         // at 10N) stay on its last entry (src/fractal.cpp:92-93)
@@ -170,7 +180,7 @@ MBR_HD T compute(const FractalK<T> &f, V3<T> z, int N, int *iter_count) {
         r = length_nc(z);
       }
     }
-    if (f.tglad_fold) {
+    if (!P && f.tglad_fold) {
       const T lim = f.fold_limit, val = f.fold_value;
       if (z.x > lim) { z.x = val - z.x; tgladColor *= T(0.9); }
       else if (z.x < -lim) { z.x = -val - z.x; tgladColor *= T(0.9); }
@@ -180,7 +190,7 @@ MBR_HD T compute(const FractalK<T> &f, V3<T> z, int N, int *iter_count) {
       else if (z.z < -lim) { z.z = -val - z.z; tgladColor *= T(0.9); }
       r = length_nc(z);
     }
-    if (f.sph_fold) {
+    if (!P && f.sph_fold) {
       T r2 = r * r;
       if (r2 < f.sph_mR2) { z = z * f.sph_factor1; tgladDE *= f.sph_factor1; tgladColor += 1; }
       else if (r2 < f.sph_fR2) { T tf2 = f.sph_fR2 / r2; z = z * tf2; tgladDE *= tf2; tgladColor += 10; }
@@ -212,7 +222,7 @@ MBR_HD T compute(const FractalK<T> &f, V3<T> z, int N, int *iter_count) {
       tgladDE *= T(3);
     } else if (af == 8) {  // tglad (Mandelbox)
       const T lim = f.mb_limit, val = f.mb_value;
-      if (f.mb_rot_on) {
+      if (P != kUnrotated && f.mb_rot_on) {
         bool lockout = false;
         z = rot9(f.mb_rot[0][0], z);
         if (z.x > lim) { z.x = val - z.x; tgladColor += f.mb_col_X; lockout = true; }
@@ -248,7 +258,7 @@ MBR_HD T compute(const FractalK<T> &f, V3<T> z, int N, int *iter_count) {
       if (r2 < f.mb_mR2) { z = z * f.mb_factor1; tgladDE *= f.mb_factor1; tgladColor += f.mb_col_Sp1; }
       else if (r2 < f.mb_fR2) { T tf2 = f.mb_fR2 / r2; z = z * tf2; tgladDE *= tf2; tgladColor += f.mb_col_Sp2; }
       z = z - ld3(f.mb_offset);
-      if (f.mb_main_rot) z = mat_apply(f.mb_main, z);
+      if (P != kUnrotated && f.mb_main_rot) z = mat_apply(f.mb_main, z);
       z = z * mscale + constant;
       tgladDE = tgladDE * mabs + T(1);
       r = length_nc(z);
@@ -671,7 +681,7 @@ MBR_HD T compute(const FractalK<T> &f, V3<T> z, int N, int *iter_count) {
         if (esc) { distance = T(0.5) * r * M::log(r) / r_dz; break; }
       } else if (Mode == MODE_COLOURING) {
         distance = length_nc(z);
-        if (f.only_plane) {
+        if (!P && f.only_plane) {
           if (!(distance <= T(1e15))) {
             distance = (T(L) - M::log(M::log(r) / M::log(T(N))) / M::log(p)) / T(100);
             break;
@@ -691,14 +701,14 @@ MBR_HD T compute(const FractalK<T> &f, V3<T> z, int N, int *iter_count) {
   }
   if (Mode == MODE_DELTA1 || Mode == MODE_DELTA2) return r;
   if (Mode == MODE_ORBIT_TRAP) return distance;
-  if (f.formula == 12) {  // hybrid colouring (src/fractal.cpp:1218-1229)
+  if (FF == 0 && f.formula == 12) {  // hybrid colouring (src/fractal.cpp:1218-1229)
     if (min > T(100)) min = T(100);
     if (distance > T(20)) distance = T(20);
     if (tgladColor > T(1000)) tgladColor = T(1000);
     return distance * T(5000) + tgladColor * T(100) + min * T(1000);
   }
-  if (formula_box_group(f.formula)) return tgladColor * T(100) + length_nc(z) * f.mb_col_R;
-  if (formula_menger_group(f.formula)) return min * T(1000);
+  if (formula_box_group(FF ? FF : f.formula)) return tgladColor * T(100) + length_nc(z) * f.mb_col_R;
+  if (formula_menger_group(FF ? FF : f.formula)) return min * T(1000);
   return distance * T(5000);
 }
 
@@ -776,13 +786,7 @@ struct DEIter {
 
 // IP: the Mandelbulb's integer power when the caller knows it at compile
 // time (8, the standard bulb), else 0 (read from f.ipow).
-// P: what the caller knows of the scene: kOptions nothing, kPlain that no
-// optional term is on (primitives, limits, interior mode, iteration
-// threshold, pre-folds, Julia constant), kUnrotated (Mandelbox) in addition
-// that its folds and its main rotation are not rotated.  The 19 rotation
-// matrices otherwise fill the scalar registers of every kernel that holds
-// the iteration (380-450 spills into vector lanes, read back in every pass).
-enum : int { kOptions = 0, kPlain = 1, kUnrotated = 2 };
+// P: kOptions, kPlain or kUnrotated.
 template <class T, int F, int P = 0, bool A = (sizeof(T) < 8), int IP = 0>
 MBR_HD void de_begin(const FractalK<T> &f, V3<T> p, DEIter<T> &s) {
   s.z = p;

@@ -288,6 +288,77 @@ __device__ __forceinline__ unsigned long long take_work(const BandBufs &b, unsig
   return v & (kStopBit - 1);
 }
 
+// Lanes of a wave that take items, for n items over the launch's waves: few
+// items spread over half of the waves, at least 4 each, so that a wave's
+// passes wait for fewer lanes.
+__device__ __forceinline__ int item_lanes(long long n) {
+  const long long half = (long long)gridDim.x * (kBlock / 128);
+  const long long per = (n + half - 1) / half;
+  return per >= 64 ? 64 : per < 4 ? 4 : (int)per;
+}
+
+// A wave's share of the band's n items (rays, hits): its first `lanes` items by
+// its number, then runs taken from a counter shared by all waves.  Adds to one
+// address pass at about 13 ns each on MI355X, whichever wave sends them: with
+// an add for every hand-out, 8192 waves spent 100 us just to find a small
+// frame's queue empty, so an item costs no add where there are lanes for all,
+// and a run grows with what is left (up to 4 waves' worth, and so that every
+// wave of the launch can still take 4 runs).
+struct WaveQueue {
+  unsigned long long *queue;
+  long long n, cur, end, shared;  // shared: first item handed out by the counter
+  int waves;
+  bool dry, stopped;
+
+  __device__ __forceinline__ WaveQueue(unsigned long long *queue_, long long n_, int lanes) {
+    queue = queue_;
+    n = n_;
+    stopped = false;
+    waves = (int)gridDim.x * (kBlock / 64);
+    // workgroups first, so that few items spread over the CUs
+    const long long w = (long long)__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)) * gridDim.x + blockIdx.x;
+    cur = w * lanes;
+    end = cur + lanes;
+    shared = (long long)waves * lanes;
+    if (cur > n) cur = n;
+    if (end > n) end = n;
+    dry = shared >= n;
+  }
+  // For the whole wave: lane `rank` of `need` lanes gets its item, or -1.
+  // Poll: the items are rays whose hand-out polls the cancel flag (take_work);
+  // stop is then set once the band was stopped.
+  template <bool Poll>
+  __device__ __forceinline__ long long take(const BandBufs &b, int rank, int need, int poll_shift, int &stop) {
+    const int have = (int)(end - cur < need ? end - cur : need);
+    long long mine = rank < have ? cur + rank : -1;
+    cur += have;
+    if (have < need && !dry) {
+      const long long left = n - end;
+      const long long fair = left / (4ll * waves);
+      const long long run = fair < need - have ? need - have : fair > 256 ? 256 : fair;
+      unsigned long long base = 0;
+      if (__lane_id() == 0) {
+        if constexpr (Poll) base = take_work(b, queue, (unsigned long long)run, poll_shift, stop);
+        else base = atomicAdd(queue, (unsigned long long)run);
+      }
+      base = __shfl(base, 0);
+      if constexpr (Poll) stop = __shfl(stop, 0);
+      const long long first = shared + (long long)base;
+      cur = first + (need - have);
+      end = first + run;
+      if (end >= n) {
+        dry = first >= n;
+        end = n;
+      }
+      if (cur > end) cur = end;
+      if (rank >= have && rank < need && first + (rank - have) < n) mine = first + (rank - have);
+      if constexpr (Poll) stopped = stop != 0;
+    }
+    if constexpr (Poll) stop = stopped;
+    return mine;
+  }
+};
+
 // Persistent march: one primary ray per lane, up to kMarchIters formula
 // iterations per pass, lane states and amortised bookkeeping as in k_ao.
 enum : int { MS_NEED = 0, MS_ITER = 1, MS_DONE = 2, MS_EXHAUSTED = 3 };
@@ -306,18 +377,17 @@ __device__ __forceinline__ void march_body(const DevScene *__restrict__ scp, Ban
   // records are FP32; the FP64 mode keeps the trigonometric form
   constexpr bool kAlg = sizeof(RT) < 8 || IP != 0;
   const DevScene &sc = *scp;
-  // the power-8 variants read a few formula constants in every iteration: a
-  // local copy keeps them in registers (the pass's stores and atomics keep
-  // the compiler from hoisting loads of the scene block out of the loop)
-  const FractalK<T> f_local = (Plain && IP) ? sc.frac<T>() : FractalK<T>{};
-  const FractalK<T> &f = (Plain && IP) ? f_local : sc.frac<T>();
+  const FractalK<T> f_local = Plain ? sc.frac<T>() : FractalK<T>{};
+  const FractalK<T> &f = Plain ? f_local : sc.frac<T>();  // see k_march64
   const int N = sc.N, minN = sc.minN;
   const int lane = __lane_id();
   const unsigned long long lt_mask = (lane == 0) ? 0ull : (~0ull >> (64 - lane));
   const V3<double> start = v3<double>(sc.start[0], sc.start[1], sc.start[2]);
 
   const MarchK m = march_k(sc);
-  int state = MS_NEED;
+  const int lanes = item_lanes(band_rays);
+  WaveQueue q(&b.counters[CNT_RAYQ], band_rays, lanes);
+  int state = lane < lanes ? MS_NEED : MS_EXHAUSTED;
   int r = 0;
   uint32_t ray_hash = 0;
   V3<double> dir = v3<double>(0, 0, 0);
@@ -345,14 +415,10 @@ __device__ __forceinline__ void march_body(const DevScene *__restrict__ scp, Ban
     const int n_need = __popcll(m_need), n_iter = __popcll(m_iter), n_done = __popcll(m_done);
 
     if (n_need && (4 * n_need >= n_need + n_iter + n_done || n_iter + n_done == 0)) {
-      unsigned long long base = 0;
       int stop = 0;
-      if (lane == 0) base = take_work(b, &b.counters[CNT_RAYQ], (unsigned long long)n_need, 12, stop);
-      base = __shfl(base, 0);
-      stop = __shfl(stop, 0);
+      const long long mine = q.take<true>(b, __popcll(m_need & lt_mask), n_need, 12, stop);
       if (state == MS_NEED) {
-        const unsigned long long mine = base + (unsigned long long)__popcll(m_need & lt_mask);
-        if (mine >= (unsigned long long)band_rays) {
+        if (mine < 0) {
           state = MS_EXHAUSTED;
         } else {
           r = (int)mine;
@@ -458,30 +524,31 @@ enum : int { PH_MARCH = 0, PH_SEARCH = 1, PH_PLUS = 2, PH_MINUS = 3, PH_ROOT = 4
 // IP: the integer power of the Mandelbulb when fixed at compile time (8).
 template <class RT, int F, int Plain, int IP, int Src>
 __device__ __forceinline__ void march64_body(const DevScene *__restrict__ scp, BandBufs b, int band_first,
-                                             int band_rays, int lane_cap, unsigned long long *stats) {
+                                             int band_rays, unsigned long long *stats) {
 #pragma clang fp contract(off)
   // integer-power Mandelbulb iterations without inverse trig wherever the
   // records are FP32; the FP64 mode keeps the trigonometric form
   constexpr bool kAlg = sizeof(RT) < 8 || IP != 0;
   const DevScene &sc = *scp;
-  // the power-8 variants read a few formula constants in every iteration: a
+  // the plain variants read a few formula constants in every iteration: a
   // local copy keeps them in registers (the pass's stores and atomics keep
   // the compiler from hoisting loads of the scene block out of the loop)
-  const FractalK<double> f_local = (Plain && IP) ? sc.fd : FractalK<double>{};
-  const FractalK<double> &f = (Plain && IP) ? f_local : sc.fd;
+  const FractalK<double> f_local = Plain ? sc.fd : FractalK<double>{};
+  const FractalK<double> &f = Plain ? f_local : sc.fd;
   const MarchK m = march_k(sc);
   const int N = sc.N, minN = sc.minN;
   const int lane = __lane_id();
   const unsigned long long lt_mask = (lane == 0) ? 0ull : (~0ull >> (64 - lane));
   const long long n_items = Src == kRays ? (long long)band_rays
                                          : (long long)b.counters[Src == kRedo ? CNT_REDO : CNT_HAND];
-  unsigned long long *const queue = &b.counters[Src == kRays ? CNT_RAYQ : Src == kRedo ? CNT_REDOQ : CNT_HANDQ];
+  const int lanes = item_lanes(n_items);
+  WaveQueue q(&b.counters[Src == kRays ? CNT_RAYQ : Src == kRedo ? CNT_REDOQ : CNT_HANDQ], n_items, lanes);
   const double search_limit = 1.0 - 0.01 * m.quality;
   const bool hit_refine = sc.hit_refine != 0;
   const double c0 = 1.0 - 0.005 * m.quality;
   const double kthr = m.resolution * m.persp / m.quality;
 
-  int state = lane < lane_cap ? MS_NEED : MS_EXHAUSTED;
+  int state = lane < lanes ? MS_NEED : MS_EXHAUSTED;
   int phase = PH_MARCH;
   int r = 0, j = 0;
   uint32_t ray_hash = 0;
@@ -520,6 +587,13 @@ __device__ __forceinline__ void march64_body(const DevScene *__restrict__ scp, B
   };
   auto finish = [&](bool found) {
 #pragma clang fp contract(off)
+    if (Src == kHand && ambiguous) {
+      // marched again from the start (kRedo)
+      b.redo_list[atomicAdd(&b.counters[CNT_REDO], 1ull)] = r;
+      redo++;
+      state = MS_NEED;
+      return;
+    }
     MarchOut o;
     o.point = start + dir * s.scan;
     if (!found) o.point = s.point;  // the last estimate's
@@ -596,17 +670,10 @@ __device__ __forceinline__ void march64_body(const DevScene *__restrict__ scp, B
     const int n_need = __popcll(m_need), n_iter = __popcll(m_iter), n_done = __popcll(m_done);
 
     if (n_need && (4 * n_need >= n_need + n_iter + n_done || n_iter + n_done == 0)) {
-      unsigned long long base = 0;
       int stop = 0;
-      if (lane == 0) {
-        if constexpr (Src == kRays) base = take_work(b, queue, (unsigned long long)n_need, 12, stop);
-        else base = atomicAdd(queue, (unsigned long long)n_need);
-      }
-      base = __shfl(base, 0);
-      stop = __shfl(stop, 0);
+      const long long mine = q.take<Src == kRays>(b, __popcll(m_need & lt_mask), n_need, 12, stop);
       if (state == MS_NEED) {
-        const unsigned long long mine = base + (unsigned long long)__popcll(m_need & lt_mask);
-        if (mine >= (unsigned long long)n_items) {
+        if (mine < 0) {
           state = MS_EXHAUSTED;
         } else {
           r = Src == kRays ? (int)mine : Src == kRedo ? b.redo_list[mine] : b.hand_ray[mine];
@@ -658,7 +725,7 @@ __device__ __forceinline__ void march64_body(const DevScene *__restrict__ scp, B
     if (state == MS_ITER) {
       bool fin = false;
 #pragma unroll
-      for (int q = 0; q < kMarchIters && !fin; q++) fin = de_call_step<double, F, Plain, kAlg, IP>(f, call, N);
+      for (int it = 0; it < kMarchIters && !fin; it++) fin = de_call_step<double, F, Plain, kAlg, IP>(f, call, N);
       if (fin) state = MS_DONE;
     }
 
@@ -737,16 +804,7 @@ __device__ __forceinline__ void march64_body(const DevScene *__restrict__ scp, B
         settled = refine();
       }
       if (found) settled = hit_refine && !m.constant_thresh ? refine() : true;
-      if (settled) {
-        if (Src == kHand && ambiguous) {
-          // marched again from the start (kRedo)
-          b.redo_list[atomicAdd(&b.counters[CNT_REDO], 1ull)] = r;
-          redo++;
-          state = MS_NEED;
-        } else {
-          finish(true);
-        }
-      }
+      if (settled) finish(true);
     }
   }
   unsigned long long v[ST_COUNT] = {0};
@@ -758,13 +816,11 @@ __device__ __forceinline__ void march64_body(const DevScene *__restrict__ scp, B
   flush_stats(stats, v);
 }
 
-// lane_cap: lanes of a wave that take rays (a small band spreads over more
-// waves, whose passes then wait for fewer lanes)
 template <class RT, int F, int Plain, int IP, int Src>
 __global__ void __launch_bounds__(kBlock, Plain && (F != 2 || IP) ? 4 : 1)
-    k_march64(const DevScene *__restrict__ scp, BandBufs b, int band_first, int band_rays, int lane_cap,
+    k_march64(const DevScene *__restrict__ scp, BandBufs b, int band_first, int band_rays,
               unsigned long long *stats) {
-  march64_body<RT, F, Plain, IP, Src>(scp, b, band_first, band_rays, lane_cap, stats);
+  march64_body<RT, F, Plain, IP, Src>(scp, b, band_first, band_rays, stats);
 }
 
 template <class T>
@@ -805,67 +861,533 @@ __device__ __forceinline__ V3<double> ray_dir(const DevScene &sc, const BandBufs
   return dir;
 }
 
-template <class T, int F, bool Deep>
-__global__ void __launch_bounds__(kBlock) k_surface(const DevScene *__restrict__ scp, BandBufs b, int band_first,
-                                                    SurfBufs<T> sb, unsigned long long *stats) {
+// Writes the hit's colour planes and its 8-bit colour.
+template <class T>
+__device__ __forceinline__ void put_colour(const BandBufs &b, const SurfBufs<T> &sb, int r, long long tid,
+                                           RGBT<T> colour) {
+  const long long n = sb.n;
+  sb.col[0 * n + tid] = colour.R;
+  sb.col[1 * n + tid] = colour.G;
+  sb.col[2 * n + tid] = colour.B;
+  b.col_r[r] = x86_d2u8((double)colour.R * 255);
+  b.col_g[r] = x86_d2u8((double)colour.G * 255);
+  b.col_b[r] = x86_d2u8((double)colour.B * 255);
+}
+
+// ObjectShader's diffuse and specular terms of the main light from the hit's
+// normal and shadow.
+template <class T>
+struct Lit {
+  T base[3], spec[3];
+};
+template <class T>
+__device__ __forceinline__ Lit<T> light_hit(const DevScene &sc, const ShaderIn<T> &in, T shadow) {
+  const ShadeK<T> &k = sc.shade<T>();
+  Lit<T> o;
+  T sh = dot(in.normal, in.light);
+  if (sh < 0) sh = 0;
+  const T shade = k.direct_light * ((T(1) - k.shading) + k.shading * sh);
+  V3<T> half = normalize(in.light - in.view);
+  T shade2 = dot(in.normal, half);
+  if (shade2 < T(0)) shade2 = 0;
+  shade2 = Math<T>::pow(shade2, T(30));
+  if (shade2 > T(15)) shade2 = 15;
+  const T specular = shade2 * k.specular;
+  for (int c = 0; c < 3; c++) {
+    o.base[c] = k.main_light[c] * shade * shadow;
+    o.spec[c] = k.main_light[c] * specular * shadow;
+  }
+  return o;
+}
+
+// Stores them, and what the later shaders read of the hit.
+template <class T>
+__device__ __forceinline__ void put_lit(const DevScene &sc, const ShaderIn<T> &in, const Lit<T> &o, long long tid,
+                                        const SurfBufs<T> &sb) {
+  const long long n = sb.n;
+  for (int c = 0; c < 3; c++) {
+    sb.base[c * n + tid] = o.base[c];
+    sb.spec[c * n + tid] = o.spec[c];
+  }
+  if constexpr (sizeof(T) == 8) {
+    if (sc.env_map) {
+      // environment mapping x reflect (ObjectShader, src/shaders.cpp:73-80);
+      // k_compose multiplies it by the AO
+      double e[3];
+      env_mapping(sc, cvt<double>(in.normal), cvt<double>(in.view), e);
+      for (int c = 0; c < 3; c++) sb.aux[(6 + c) * n + tid] = (T)(e[c] * sc.reflect);
+    }
+  }
+  if (sc.n_lights > 0 || sc.fake_lights) {
+    // k_aux shades the aux (and fake) lights from the normal and the
+    // detail size MainShadow left (the aux shadows inherit it)
+    sb.aux[0 * n + tid] = in.normal.x;
+    sb.aux[1 * n + tid] = in.normal.y;
+    sb.aux[2 * n + tid] = in.normal.z;
+    sb.aux[3 * n + tid] = in.detail;
+  }
+}
+
+// The generic formulas' surface shading, one lane per hit (their estimates
+// run whole, so there is nothing to interleave).
+template <class T>
+__global__ void __launch_bounds__(kBlock) k_surface_generic(const DevScene *__restrict__ scp, BandBufs b,
+                                                            int band_first, SurfBufs<T> sb,
+                                                            unsigned long long *stats) {
   const DevScene &sc = *scp;
   const long long n_hits = (long long)b.counters[CNT_HITS];
   LaneCount cnt = {0, 0};
   for (long long tid = (long long)blockIdx.x * kBlock + threadIdx.x; tid < n_hits;
        tid += (long long)gridDim.x * kBlock) {
     const int r = b.hit_list[tid];
-    const V3<double> dir = ray_dir(sc, b, band_first, r);
-    const ShadeK<T> &k = sc.shade<T>();
     ShaderIn<T> in;
     load_hit(sc, b, r, in);
-    in.view = cvt<T>(dir);
-    in.normal = normals<T, F, Deep>(sc, in, cnt);
-    T sh = dot(in.normal, in.light);
-    if (sh < 0) sh = 0;
-    const T shade = k.direct_light * ((T(1) - k.shading) + k.shading * sh);
+    in.view = cvt<T>(ray_dir(sc, b, band_first, r));
+    in.normal = normals<T, 0, false>(sc, in, cnt);
     T shadow = 1;
-    if (sc.shadow) shadow = main_shadow<T, F, Deep>(sc, in, cnt);
-    V3<T> half = normalize(in.light - in.view);
-    T shade2 = dot(in.normal, half);
-    if (shade2 < T(0)) shade2 = 0;
-    shade2 = Math<T>::pow(shade2, T(30));
-    if (shade2 > T(15)) shade2 = 15;
-    const T specular = shade2 * k.specular;
-    RGBT<T> colour = surface_colour<T, Deep, sizeof(T) == 8 || F == 0>(sc, in, cnt);
-    const long long n = sb.n;
-    for (int c = 0; c < 3; c++) {
-      sb.base[c * n + tid] = k.main_light[c] * shade * shadow;
-      sb.spec[c * n + tid] = k.main_light[c] * specular * shadow;
-    }
-    sb.col[0 * n + tid] = colour.R;
-    sb.col[1 * n + tid] = colour.G;
-    sb.col[2 * n + tid] = colour.B;
-    if (sc.ao && sc.fast_ao) sb.fast_ao[tid] = fast_ao2<T, F, Deep>(sc, in, cnt);
-    // AmbientOcclusion estimates with the detail size calcParam holds when
-    // it runs: MainShadow's last threshold, float-rounded (src/shaders.cpp:
-    // 510-522), when there are shadows; the slow AO pass reads it from here
-    if (sc.ao && !sc.fast_ao) sb.fast_ao[tid] = in.detail;
-    if constexpr (sizeof(T) == 8) {
-      if (sc.env_map) {
-        // environment mapping x reflect (ObjectShader, src/shaders.cpp:73-80);
-        // k_compose multiplies it by the AO
-        double e[3];
-        env_mapping(sc, cvt<double>(in.normal), cvt<double>(in.view), e);
-        for (int c = 0; c < 3; c++) sb.aux[(6 + c) * n + tid] = (T)(e[c] * sc.reflect);
-      }
-    }
-    if (sc.n_lights > 0 || sc.fake_lights) {
-      // k_aux shades the aux (and fake) lights from the normal and the
-      // detail size MainShadow left (the aux shadows inherit it)
-      sb.aux[0 * n + tid] = in.normal.x;
-      sb.aux[1 * n + tid] = in.normal.y;
-      sb.aux[2 * n + tid] = in.normal.z;
-      sb.aux[3 * n + tid] = in.detail;
-    }
-    b.col_r[r] = x86_d2u8((double)colour.R * 255);
-    b.col_g[r] = x86_d2u8((double)colour.G * 255);
-    b.col_b[r] = x86_d2u8((double)colour.B * 255);
+    if (sc.shadow) shadow = main_shadow<T, 0, false>(sc, in, cnt);
+    const RGBT<T> colour = surface_colour<T, false, true>(sc, in, cnt);
+    put_lit<T>(sc, in, light_hit<T>(sc, in, shadow), tid, sb);
+    put_colour(b, sb, r, tid, colour);
+    if (sc.ao && sc.fast_ao) sb.fast_ao[tid] = fast_ao2<T, 0, false>(sc, in, cnt);
+    else if (sc.ao) sb.fast_ao[tid] = in.detail;
   }
+  unsigned long long v[ST_COUNT] = {0};
+  v[ST_SHADE_DE] = cnt.de_calls;
+  v[ST_SHADE_ITERS] = cnt.iterations;
+  flush_stats(stats, v);
+}
+
+// A distance estimate of the surface shaders at a hit's point plus an offset
+// (de_at), as a resumable state.  Deep: an FP32 estimate whose detail is below
+// FP32 resolution at its point runs whole in FP64 (calc_distance_p64).
+template <class T, int F, bool Deep, int P, int IP>
+struct HitDE {
+  static constexpr bool kDeep = Deep && sizeof(T) < 8;
+  static constexpr bool kAlg = sizeof(T) < 8;
+  struct None {};
+  DECall<T> c;
+  std::conditional_t<kDeep, DECall<double>, None> c64;
+  bool in64 = false;
+
+  // true when it ended without iterating (dist and info are then set)
+  __device__ __forceinline__ bool begin(const FractalK<double> &fd, const FractalK<T> &f, V3<T> point, V3<double> point64,
+                                        V3<T> off, T detail, int N, int minN, bool normalMode, T &dist,
+                                        DEInfo &info) {
+    if constexpr (kDeep) {
+      const V3<double> p = point64 + cvt<double>(off);
+      const V3<float> pf = cvt<float>(p);
+      const float cmax = length(pf) * (f.julia_mode ? 0.0f : (f.constant_factor > 1.0f ? f.constant_factor : 1.0f));
+      const float zc = f.julia_mode ? length(ld3(f.julia)) : cmax;
+      in64 = (double)detail < kMixedSwitch * (double)(length(pf) > zc ? length(pf) : zc);
+      if (in64) {
+        double d = 0.0;
+        const bool e = de_call_begin<double, F, P>(fd, p, (double)detail, N, minN, normalMode, c64, d, info);
+        dist = (T)d;
+        return e;
+      }
+      return de_call_begin<T, F, P, kAlg, IP>(f, pf, detail, N, minN, normalMode, c, dist, info);
+    } else {
+      return de_call_begin<T, F, P, kAlg, IP>(f, point + off, detail, N, minN, normalMode, c, dist, info);
+    }
+  }
+  __device__ __forceinline__ bool step(const FractalK<double> &fd, const FractalK<T> &f, int N) {
+    if constexpr (kDeep) {
+      if (in64) return de_call_step<double, F, P>(fd, c64, N);
+    }
+    return de_call_step<T, F, P, kAlg, IP>(f, c, N);
+  }
+  __device__ __forceinline__ T end(const FractalK<double> &fd, const FractalK<T> &f, T detail, int N, int minN,
+                                   bool normalMode, DEInfo &info) {
+    if constexpr (kDeep) {
+      if (in64) return (T)de_call_end<double, F, P>(fd, c64, (double)detail, N, minN, normalMode, info);
+    }
+    return de_call_end<T, F, P, kAlg, IP>(f, c, detail, N, minN, normalMode, info);
+  }
+};
+
+// The lanes of a wave over a queue of items, one distance estimate per lane
+// and step (the scheme of k_march64): a lane is NEED (wants an item), ITER
+// (its estimate is running), DONE (its estimate is complete, its item's next
+// step pending) or EXHAUSTED.  fetch(rank, n): lanes in NEED take the items
+// after the first n; step(): one formula iteration; done(): the item's next
+// step.
+template <int Iters, class Fetch, class Step, class Done>
+__device__ __forceinline__ void lane_loop(int &state, Fetch fetch, Step step, Done done) {
+  const int lane = __lane_id();
+  const unsigned long long lt_mask = (lane == 0) ? 0ull : (~0ull >> (64 - lane));
+  for (;;) {
+    const unsigned long long m_need = __ballot(state == MS_NEED);
+    const unsigned long long m_iter = __ballot(state == MS_ITER);
+    const unsigned long long m_done = __ballot(state == MS_DONE);
+    if (!(m_need | m_iter | m_done)) break;
+    const int n_need = __popcll(m_need), n_iter = __popcll(m_iter), n_done = __popcll(m_done);
+    if (n_need && (4 * n_need >= n_need + n_iter + n_done || n_iter + n_done == 0))
+      fetch(__popcll(m_need & lt_mask), n_need);
+    if (state == MS_ITER) {
+      bool fin = false;
+      for (int q = 0; q < Iters && !fin; q++) fin = step();
+      if (fin) state = MS_DONE;
+    }
+    const unsigned long long m_done2 = __ballot(state == MS_DONE);
+    const unsigned long long m_iter2 = __ballot(state == MS_ITER);
+    const int n_done2 = __popcll(m_done2), n_iter2 = __popcll(m_iter2);
+    if (n_done2 && (4 * n_done2 >= n_done2 + n_iter2 || n_iter2 == 0) && state == MS_DONE) done();
+  }
+}
+
+
+// Surface shading of the hits (ObjectShader's estimates) as three kinds of
+// items that depend on the hit's march alone and run side by side: the shadow
+// ray (MainShadow, chained estimates), the normal's four estimates (one item
+// each; slowShading's 11^3 chained as one) and the colouring orbit.  A wave
+// works through the shadow rays, then the normals, then the colours; waves
+// whose lanes still follow long rays leave the rest of the queues to others.
+// One lane per hit instead ran them one after the other at 20-27% active
+// lanes and 11-13% VALU busy, and the deep-zoom variant at one wave per SIMD
+// (256 + 107 registers).  hit_lit forms the shade from the results: estimates in sb.base and sb.spec[0], the shadow factor in sb.spec[1], the detail size
+// MainShadow leaves in sb.fast_ao.
+enum : int { HIT_SHADOW = 1, HIT_NORMAL = 2, HIT_COLOUR = 4 };
+template <class T, int F, bool Deep, int P>
+struct HitPolicy {
+  static constexpr bool trig64 = sizeof(T) == 8 && F == 2;
+  static constexpr int iters = trig64 ? 2 : 4;
+  // waves per SIMD asked of the compiler
+  static constexpr int waves = P == kOptions ? 1 : trig64 || (Deep && F == 2) ? 2 : sizeof(T) == 8 || Deep ? 4 : 6;
+};
+
+template <class T, int F, bool Deep, int P, int IP>
+__global__ void __launch_bounds__(kBlock, (HitPolicy<T, F, Deep, P>::waves))
+    k_hits(const DevScene *__restrict__ scp, BandBufs b, SurfBufs<T> sb, int kinds, unsigned long long *stats) {
+  const DevScene &sc = *scp;
+  const FractalK<T> f_local = P ? sc.frac<T>() : FractalK<T>{};
+  const FractalK<T> &f = P ? f_local : sc.frac<T>();  // see k_march64
+  constexpr bool kLocal64 = P && Deep && sizeof(T) < 8;
+  const FractalK<double> fd_local = kLocal64 ? sc.fd : FractalK<double>{};
+  const FractalK<double> &fd = kLocal64 ? fd_local : sc.fd;
+  const ShadeK<T> &k = sc.shade<T>();
+  constexpr int kIters = HitPolicy<T, F, Deep, P>::iters;
+  const long long n_hits = (long long)b.counters[CNT_HITS];
+  const long long n = sb.n;
+  const int lane = __lane_id();
+  LaneCount cnt = {0, 0};
+
+  if ((kinds & HIT_SHADOW) && sc.shadow) {
+    const V3<T> light = v3<T>(k.light[0], k.light[1], k.light[2]);
+    const T DE_factor = sc.shadow_fx ? T(1) : k.DE_factor;
+    const int N = sc.N, minN = sc.minN, soft = sc.bsoft, fx = sc.shadow_fx, penetrating = sc.penetrating;
+    const int iter_fog = sc.iter_fog;
+    const T soft_range = k.soft_range;
+    const int lanes = item_lanes(n_hits);
+    WaveQueue queue(&b.counters[CNT_SHADOWQ], n_hits, lanes);
+    int state = lane < lanes ? MS_NEED : MS_EXHAUSTED;
+    long long tid = 0;
+    V3<T> point = v3<T>(0, 0, 0);
+    V3<double> point64 = v3<double>(0, 0, 0);
+    T i = 0, factor = 0, hit_thr = 0, thr = 0, dist = 0, shadowTemp = 1, maxSoft = 0;
+    int guard = 0, early_it = 0;
+    bool early = false;
+    HitDE<T, F, Deep, P, IP> call;
+    auto finish = [&]() {
+      sb.spec[n + tid] = soft ? (T(1) - maxSoft) : shadowTemp;
+      sb.fast_ao[tid] = thr;  // the detail size MainShadow leaves, for the AO
+      state = MS_NEED;
+    };
+    // the estimate at distance i, or the ray's end
+    auto next = [&]() {
+      if (!(i < factor && guard < kMaxShadeSteps)) {
+        finish();
+        return;
+      }
+      const float dist_thresh = fx ? fx_thresh<T>(sc, point + light * i) : (float)hit_thr;
+      thr = (T)dist_thresh;
+      DEInfo info;
+      early = call.begin(fd, f, point, point64, light * i, thr, N, minN, false, dist, info);
+      state = early ? MS_DONE : MS_ITER;
+      if (early) early_it = info.iters;
+    };
+    lane_loop<kIters>(
+        state,
+        [&](int rank, int n_need) {
+          int stop;
+          const long long mine = queue.take<false>(b, rank, n_need, 0, stop);
+          if (state != MS_NEED) return;
+          if (mine < 0) {
+            state = MS_EXHAUSTED;
+            return;
+          }
+          tid = mine;
+          ShaderIn<T> in;
+          load_hit(sc, b, b.hit_list[tid], in);
+          point = in.point;
+          point64 = in.point64;
+          hit_thr = in.dist_thresh;
+          factor = in.delta / k.resolution;
+          if (!penetrating) factor = k.view_distance_max;
+          dist = hit_thr;
+          thr = hit_thr;
+          i = hit_thr;
+          if (sc.interior) i = hit_thr * DE_factor;
+          shadowTemp = 1;
+          maxSoft = 0;
+          guard = 0;
+          next();
+        },
+        [&]() { return call.step(fd, f, N); },
+        [&]() {
+          int iters = early_it;
+          cnt.de_calls += 1;
+          if (!early) {
+            DEInfo info;
+            dist = call.end(fd, f, thr, N, minN, false, info);
+            iters = info.iters;
+            cnt.iterations += (uint32_t)info.work;
+          }
+          if (soft) {
+            T angle = (dist - thr) / i;
+            if (angle < 0) angle = 0;
+            if (dist < thr) angle = 0;
+            T softShadow = (T(1) - angle / soft_range);
+            if (penetrating) softShadow *= (factor - i) / factor;
+            if (softShadow < 0) softShadow = 0;
+            if (softShadow > maxSoft) maxSoft = softShadow;
+          }
+          if (iter_fog) shadowTemp -= fog_opacity<T>(sc, dist * DE_factor, iters) * (factor - i) / factor;
+          if (dist < thr || shadowTemp < T(0)) {
+            shadowTemp -= (factor - i) / factor;
+            if (!penetrating) shadowTemp = 0;
+            if (shadowTemp < T(0)) shadowTemp = 0;
+            finish();
+            return;
+          }
+          i += dist * DE_factor;
+          guard++;
+          next();
+        });
+  }
+
+  if (kinds & HIT_NORMAL) {
+    const int N5 = sc.N * 5, slow = sc.slow_shading, minN = slow ? sc.minN : 0;
+    const long long n_items = slow ? n_hits : 4 * n_hits;
+    const int lanes = item_lanes(n_items);
+    WaveQueue queue(&b.counters[CNT_NORMALQ], n_items, lanes);
+    int state = lane < lanes ? MS_NEED : MS_EXHAUSTED;
+    long long item = 0;
+    V3<T> point = v3<T>(0, 0, 0), p2 = point, sum = point;
+    V3<double> point64 = v3<double>(0, 0, 0);
+    double px = 0, py = 0, pz = 0;
+    T delta = 0, detail = 0, dist = 0;
+    bool early = false;
+    HitDE<T, F, Deep, P, IP> call;
+    auto begin = [&](V3<T> off) {
+      DEInfo info;
+      early = call.begin(fd, f, point, point64, off, detail, N5, minN, true, dist, info);
+      state = early ? MS_DONE : MS_ITER;
+    };
+    auto stencil = [&]() {
+      p2 = v3<T>((T)px, (T)py, (T)pz);
+      begin(p2 * delta);
+    };
+    lane_loop<kIters>(
+        state,
+        [&](int rank, int n_need) {
+          int stop;
+          const long long mine = queue.take<false>(b, rank, n_need, 0, stop);
+          if (state != MS_NEED) return;
+          if (mine < 0) {
+            state = MS_EXHAUSTED;
+            return;
+          }
+          item = mine;
+          ShaderIn<T> in;
+          load_hit(sc, b, b.hit_list[slow ? item : item >> 2], in);
+          point = in.point;
+          point64 = in.point64;
+          detail = in.detail;
+          delta = in.delta * k.smoothness;
+          if (sc.interior) delta = in.dist_thresh * k.quality * T(0.2) * k.smoothness;
+          if (slow) {
+            sum = v3<T>(0, 0, 0);
+            px = py = pz = -1.0;
+            stencil();
+          } else {
+            const int j = (int)(item & 3);
+            begin(v3<T>(j == 1 ? delta : T(0), j == 2 ? delta : T(0), j == 3 ? delta : T(0)));
+          }
+        },
+        [&]() { return call.step(fd, f, N5); },
+        [&]() {
+          cnt.de_calls += 1;
+          if (!early) {
+            DEInfo info;
+            dist = call.end(fd, f, detail, N5, minN, true, info);
+            cnt.iterations += (uint32_t)info.work;
+          }
+          state = MS_NEED;
+          if (!slow) {
+            const long long j = item & 3, tid = item >> 2;
+            if (j < 3) sb.base[j * n + tid] = dist;
+            else sb.spec[tid] = dist;
+            return;
+          }
+          // the 11^3 stencil with the reference's accumulated loop variables
+          sum = sum + p2 * dist;
+          pz += 0.2;
+          if (!(pz <= 1.0)) { pz = -1.0; py += 0.2; }
+          if (!(py <= 1.0)) { py = -1.0; px += 0.2; }
+          if (px <= 1.0) {
+            stencil();
+            return;
+          }
+          sb.base[item] = sum.x;
+          sb.base[n + item] = sum.y;
+          sb.base[2 * n + item] = sum.z;
+        });
+  }
+
+  if (kinds & HIT_COLOUR) {
+    // whole orbits: their lengths differ little between neighbouring hits
+    const int lanes = item_lanes(n_hits);
+    WaveQueue queue(&b.counters[CNT_COLOURQ], n_hits, lanes);
+    for (;;) {
+      int stop;
+      const long long tid = queue.take<false>(b, lane < lanes ? lane : 64, lanes, 0, stop);
+      if (!__ballot(tid >= 0)) break;
+      if (tid < 0) continue;
+      const int r = b.hit_list[tid];
+      ShaderIn<T> in;
+      load_hit(sc, b, r, in);
+      if (!sc.shadow) sb.fast_ao[tid] = in.detail;
+      else if (Deep && sc.shadow_fx) in.detail = sb.fast_ao[tid];
+      else in.detail = (T)(float)in.detail;
+      put_colour(b, sb, r, tid, surface_colour<T, Deep, false, F, P>(sc, in, cnt));
+    }
+  }
+  unsigned long long v[ST_COUNT] = {0};
+  v[ST_SHADE_DE] = cnt.de_calls;
+  v[ST_SHADE_ITERS] = cnt.iterations;
+  flush_stats(stats, v);
+}
+
+// The normal of hit tid from k_hits's estimates (CalculateNormals).
+template <class T>
+__device__ __forceinline__ V3<T> hit_normal(const DevScene &sc, const SurfBufs<T> &sb, long long tid) {
+  const long long n = sb.n;
+  const T s1 = sb.base[tid], s2 = sb.base[n + tid], s3 = sb.base[2 * n + tid];
+  V3<T> v = v3<T>(s1, s2, s3);
+  if (!sc.slow_shading) {
+    const T s4 = sb.spec[tid];
+    v = v3<T>(s2 - s1, s3 - s1, s4 - s1);
+  }
+  if (v.x == 0 && v.y == 0 && v.z == 0) v.x = 1;
+  else v = normalize(v);
+  return v;
+}
+
+// The lit hit tid from k_hits's results.
+template <class T>
+__device__ __forceinline__ Lit<T> hit_lit(const DevScene &sc, const BandBufs &b, int band_first, const SurfBufs<T> &sb,
+                                          int r, long long tid, ShaderIn<T> &in) {
+  load_hit(sc, b, r, in);
+  in.view = cvt<T>(ray_dir(sc, b, band_first, r));
+  in.normal = hit_normal(sc, sb, tid);
+  return light_hit<T>(sc, in, sc.shadow ? sb.spec[sb.n + tid] : T(1));
+}
+
+// For the shaders that read the lit hits before k_compose (aux and fake
+// lights, environment mapping): replaces k_hits's and k_fast_ao's results.
+template <class T>
+__global__ void __launch_bounds__(kBlock) k_hits_end(const DevScene *__restrict__ scp, BandBufs b, int band_first,
+                                                     SurfBufs<T> sb) {
+  const DevScene &sc = *scp;
+  const long long n_hits = (long long)b.counters[CNT_HITS];
+  for (long long tid = (long long)blockIdx.x * kBlock + threadIdx.x; tid < n_hits;
+       tid += (long long)gridDim.x * kBlock) {
+    ShaderIn<T> in;
+    const Lit<T> o = hit_lit<T>(sc, b, band_first, sb, b.hit_list[tid], tid, in);
+    in.detail = sb.fast_ao[tid];
+    if (sc.ao && sc.fast_ao) sb.fast_ao[tid] = sb.spec[2 * sb.n + tid];
+    put_lit<T>(sc, in, o, tid, sb);
+  }
+}
+
+// FastAmbientOcclusion2 (src/shaders.cpp:585-605): quality^2 - 1 estimates
+// along each hit's normal; the AO in sb.spec[2].
+template <class T, int F, bool Deep, int P, int IP>
+__global__ void __launch_bounds__(kBlock, (HitPolicy<T, F, Deep, P>::waves))
+    k_fast_ao(const DevScene *__restrict__ scp, BandBufs b, SurfBufs<T> sb, unsigned long long *stats) {
+  const DevScene &sc = *scp;
+  const FractalK<T> f_local = P ? sc.frac<T>() : FractalK<T>{};
+  const FractalK<T> &f = P ? f_local : sc.frac<T>();  // see k_march64
+  constexpr bool kLocal64 = P && Deep && sizeof(T) < 8;
+  const FractalK<double> fd_local = kLocal64 ? sc.fd : FractalK<double>{};
+  const FractalK<double> &fd = kLocal64 ? fd_local : sc.fd;
+  const ShadeK<T> &k = sc.shade<T>();
+  const long long n_hits = (long long)b.counters[CNT_HITS];
+  const long long n = sb.n;
+  const int lane = __lane_id();
+  const int N = sc.N, minN = sc.minN, end = sc.ao_quality * sc.ao_quality;
+  const T tune = k.fast_ao_tune;
+  LaneCount cnt = {0, 0};
+  const int lanes = item_lanes(n_hits);
+  WaveQueue queue(&b.counters[CNT_FASTQ], n_hits, lanes);
+  int state = lane < lanes ? MS_NEED : MS_EXHAUSTED;
+  long long tid = 0;
+  V3<T> point = v3<T>(0, 0, 0), normal = point;
+  V3<double> point64 = v3<double>(0, 0, 0);
+  T delta = 0, detail = 0, dist = 0, aoTemp = 0, inv2i = 1, scan = 0;
+  int i = 0;
+  bool early = false;
+  HitDE<T, F, Deep, P, IP> call;
+  auto next = [&]() {
+    if (i >= end) {
+      T ao = T(1) - T(0.2) * aoTemp;
+      if (ao < 0) ao = 0;
+      sb.spec[2 * n + tid] = ao;
+      state = MS_NEED;
+      return;
+    }
+    inv2i *= T(0.5);  // 1/pow(2,i), exact
+    scan = T(i * i) * delta;
+    DEInfo info;
+    early = call.begin(fd, f, point, point64, normal * scan, detail, N, minN, false, dist, info);
+    state = early ? MS_DONE : MS_ITER;
+  };
+  lane_loop<HitPolicy<T, F, Deep, P>::iters>(
+      state,
+      [&](int rank, int n_need) {
+        int stop;
+        const long long mine = queue.take<false>(b, rank, n_need, 0, stop);
+        if (state != MS_NEED) return;
+        if (mine < 0) {
+          state = MS_EXHAUSTED;
+          return;
+        }
+        tid = mine;
+        ShaderIn<T> in;
+        load_hit(sc, b, b.hit_list[tid], in);
+        point = in.point;
+        point64 = in.point64;
+        normal = hit_normal(sc, sb, tid);
+        delta = in.dist_thresh;
+        detail = sb.fast_ao[tid];
+        aoTemp = 0;
+        inv2i = 1;
+        i = 1;
+        next();
+      },
+      [&]() { return call.step(fd, f, N); },
+      [&]() {
+        cnt.de_calls += 1;
+        if (!early) {
+          DEInfo info;
+          dist = call.end(fd, f, detail, N, minN, false, info);
+          cnt.iterations += (uint32_t)info.work;
+        }
+        aoTemp += inv2i * (scan - tune * dist) / delta;
+        i++;
+        next();
+      });
   unsigned long long v[ST_COUNT] = {0};
   v[ST_SHADE_DE] = cnt.de_calls;
   v[ST_SHADE_ITERS] = cnt.iterations;
@@ -976,10 +1498,8 @@ __device__ __forceinline__ void ao_body(const DevScene *__restrict__ scp, BandBu
   // trig-free integer-power iteration in FP32, and in FP64 for the fixed power
   constexpr bool kAlg = sizeof(T) < 8 || IP != 0;
   const long long n_hits = (long long)b.counters[CNT_HITS];
-  unsigned long long *queue = &b.counters[CNT_AOQ];
-  // power-8 variants: the formula constants in registers (as in k_march)
-  const FractalK<T> f_local = (Plain && IP) ? sc.frac<T>() : FractalK<T>{};
-  const FractalK<T> &f = (Plain && IP) ? f_local : sc.frac<T>();
+  const FractalK<T> f_local = Plain ? sc.frac<T>() : FractalK<T>{};
+  const FractalK<T> &f = Plain ? f_local : sc.frac<T>();  // see k_march64
   const ShadeK<T> &k = sc.shade<T>();
   const T *dirs;
   if constexpr (sizeof(T) == 8) dirs = ao.dir_d; else dirs = ao.dir_f;
@@ -988,9 +1508,16 @@ __device__ __forceinline__ void ao_body(const DevScene *__restrict__ scp, BandBu
   const int lane = __lane_id();
   const unsigned long long lt_mask = (lane == 0) ? 0ull : (~0ull >> (64 - lane));
 
-  // wave-uniform cursor: hit wh, next direction wd
-  long long wh = -1;
-  unsigned wd = count;
+  // The wave works through units, each 1 / 2^part_bits of a hit's directions:
+  // whole hits, or parts of at least 16 directions where there are fewer hits
+  // than waves.  Wave-uniform cursor: unit wu (-1 none), next direction wd of it.
+  const int waves = (int)gridDim.x * (kBlock / 64);
+  int part_bits = 0;
+  while ((n_hits << (part_bits + 1)) <= waves && (count >> (part_bits + 1)) >= 16) part_bits++;
+  const unsigned unit = (count + (1u << part_bits) - 1) >> part_bits;
+  WaveQueue queue(&b.counters[CNT_AOQ], n_hits << part_bits, 1);
+  long long wu = -1;
+  unsigned wd = unit;
   int state = AO_NEED;
   long long h_cur = -1;  // hit whose data this lane holds
   unsigned long long item = 0;
@@ -1033,36 +1560,35 @@ __device__ __forceinline__ void ao_body(const DevScene *__restrict__ scp, BandBu
       // hand out the next items to the lanes that need one, in lane order
       const unsigned n = (unsigned)n_need;
       const unsigned off = (unsigned)__popcll(m_need & lt_mask);
-      const unsigned avail = count - wd;
-      long long h = wh;
+      const unsigned avail = unit - wd;
+      long long u = wu;
       unsigned d = wd + off;
       if (n > avail) {
-        // new hits for the lanes beyond this hit's remaining directions
+        // new units for the lanes beyond this one's remaining directions
         const unsigned extra = n - avail;
-        const unsigned khits = (extra + count - 1) / count;
-        unsigned long long base = 0;
-        if (lane == 0) {
-          int stop = 0;
-          base = take_work(b, queue, (unsigned long long)khits, 8, stop);
+        const unsigned more = (extra + unit - 1) / unit;
+        const bool beyond_unit = off >= avail;
+        const unsigned j = beyond_unit ? off - avail : 0u;
+        const unsigned q = unit >= 64 ? 0u : j / unit;  // several units only when they are small
+        int stop = 0;
+        const long long got = queue.take<true>(b, (int)q, (int)more, 8, stop);
+        if (beyond_unit) {
           // cancelled: no further hits (their AO intensities stay unwritten)
-          if (stop) base = (unsigned long long)n_hits;
+          u = stop ? -1 : got;
+          d = j - q * unit;
         }
-        base = __shfl(base, 0);
-        if (off >= avail) {
-          const unsigned j = off - avail;
-          const unsigned q = count >= 64 ? 0u : j / count;  // several hits only when count < 64
-          h = (long long)base + q;
-          d = j - q * count;
-        }
-        wh = (long long)base + (khits - 1);
-        wd = extra - (khits - 1) * count;
+        // the last lane that takes one holds the last unit
+        wu = __shfl(u, 63 - __builtin_clzll(m_need));
+        wd = extra - (more - 1) * unit;
       } else {
         wd += n;
       }
+      d += (unsigned)(u & ((1 << part_bits) - 1)) * unit;
+      const long long h = u >> part_bits;
       if (state == AO_NEED) {
-        if (h >= n_hits) {
+        if (u < 0) {
           state = AO_EXHAUSTED;
-        } else {
+        } else if (d < count) {  // (a hit's last part may be shorter)
           if (h != h_cur) {
             h_cur = h;
             ShaderIn<T> in;
@@ -1146,9 +1672,16 @@ __global__ void __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(6, 
   ao_body<T, F, false, Plain, IP>(scp, b, ao, sb, stats);
 }
 
+// ended: sb.base, sb.spec and sb.fast_ao hold lit hits (k_hits_end, the
+// generic surface kernel); else k_hits's results.
+//
+// A wave composes a run of hits, one per lane; with AmbientOcclusion it first
+// sums the AO intensities of four of them at a time, read coalesced: lane j
+// takes directions j, j + 64, ... in order, then the 64 partial sums are added
+// pairwise (a fixed order, so results are reproducible).
 template <class T, class RT>
-__global__ void __launch_bounds__(kBlock) k_compose(const DevScene *__restrict__ scp, BandBufs b, AODev ao,
-                                                    SurfBufs<T> sb) {
+__global__ void __launch_bounds__(kBlock) k_compose(const DevScene *__restrict__ scp, BandBufs b, int band_first,
+                                                    AODev ao, SurfBufs<T> sb, int ended) {
   const DevScene &sc = *scp;
   const long long n_hits = (long long)b.counters[CNT_HITS];
   const ShadeK<T> &k = sc.shade<T>();
@@ -1156,46 +1689,71 @@ __global__ void __launch_bounds__(kBlock) k_compose(const DevScene *__restrict__
   const int lane = __lane_id();
   const long long wave0 = ((long long)blockIdx.x * kBlock + threadIdx.x) / 64;
   const long long waves = (long long)gridDim.x * (kBlock / 64);
-  // one wave per hit: the lanes read the hit's AO intensities coalesced,
-  // lane j summing directions j, j + 64, ... in order, then the 64 partial
-  // sums are added pairwise (a fixed order, so results are reproducible)
-  for (long long tid = wave0; tid < n_hits; tid += waves) {
-    const int r = b.hit_list[tid];
+  const long long per = (n_hits + waves - 1) / waves;
+  const int run = per >= 64 ? 64 : per < 1 ? 1 : (int)per;
+  const bool slow_ao = sc.ao && !sc.fast_ao;
+  for (long long base = wave0 * run; base < n_hits; base += waves * run) {
+    const int here = n_hits - base < run ? (int)(n_hits - base) : run;
     RGBT<T> amb = {0, 0, 0};
-    if (sc.ao) {
-      if (sc.fast_ao) {
-        const T a = sb.fast_ao[tid];
-        amb = RGBT<T>{a, a, a};
-      } else {
-        const T *it = sb.ao + tid * ao.count;
+    if (slow_ao) {
+      for (int q = 0; q < here; q += 4) {
+        const T *it = sb.ao + (base + q) * ao.count;
+        const int m = here - q < 4 ? here - q : 4;
+        RGBT<T> a[4] = {{0, 0, 0}, {0, 0, 0}, {0, 0, 0}, {0, 0, 0}};
         for (int v = lane; v < ao.count; v += 64) {
-          const T s = it[v];
-          amb.R += s * T(ao.rgb[4 * v + 0]);
-          amb.G += s * T(ao.rgb[4 * v + 1]);
-          amb.B += s * T(ao.rgb[4 * v + 2]);
+          const T cR = T(ao.rgb[4 * v + 0]), cG = T(ao.rgb[4 * v + 1]), cB = T(ao.rgb[4 * v + 2]);
+#pragma unroll
+          for (int u = 0; u < 4; u++) {
+            if (u >= m) break;
+            const T s = it[(long long)u * ao.count + v];
+            a[u].R += s * cR;
+            a[u].G += s * cG;
+            a[u].B += s * cB;
+          }
         }
 #pragma unroll
-        for (int off = 32; off >= 1; off >>= 1) {
-          amb.R += __shfl_xor(amb.R, off);
-          amb.G += __shfl_xor(amb.G, off);
-          amb.B += __shfl_xor(amb.B, off);
+        for (int u = 0; u < 4; u++) {
+#pragma unroll
+          for (int off = 32; off >= 1; off >>= 1) {
+            a[u].R += __shfl_xor(a[u].R, off);
+            a[u].G += __shfl_xor(a[u].G, off);
+            a[u].B += __shfl_xor(a[u].B, off);
+          }
+          if (lane == q + u) amb = a[u];
         }
-        const T den = T(ao.count) * T(256);
-        amb.R /= den;
-        amb.G /= den;
-        amb.B /= den;
       }
+      const T den = T(ao.count) * T(256);
+      amb.R /= den;
+      amb.G /= den;
+      amb.B /= den;
     }
+    if (lane >= here) continue;
+    const long long tid = base + lane;
+    const int r = b.hit_list[tid];
+    Lit<T> lit;
+    if (ended) {
+      for (int c = 0; c < 3; c++) {
+        lit.base[c] = sb.base[c * n + tid];
+        lit.spec[c] = sb.spec[c * n + tid];
+      }
+    } else {
+      ShaderIn<T> in;
+      lit = hit_lit<T>(sc, b, band_first, sb, r, tid, in);
+    }
+    if (sc.ao && sc.fast_ao) {
+      const T a = ended ? sb.fast_ao[tid] : sb.spec[2 * n + tid];
+      amb = RGBT<T>{a, a, a};
+    }
+    const T cR = sb.col[0 * n + tid], cG = sb.col[1 * n + tid], cB = sb.col[2 * n + tid];
     // environment mapping x reflect, times the AO (0 without it)
     RGBT<T> env = {0, 0, 0};
     if (sc.env_map) env = RGBT<T>{sb.aux[6 * n + tid], sb.aux[7 * n + tid], sb.aux[8 * n + tid]};
-    if (lane == 0 && b.sp_r) {
+    if (b.sp_r) {
       // reflections: the object part and the specular part apart
-      const T cR = sb.col[0 * n + tid], cG = sb.col[1 * n + tid], cB = sb.col[2 * n + tid];
-      T oR = env.R * amb.R + (amb.R * k.global_ilum + sb.base[0 * n + tid]) * cR;
-      T oG = env.G * amb.G + (amb.G * k.global_ilum + sb.base[1 * n + tid]) * cG;
-      T oB = env.B * amb.B + (amb.B * k.global_ilum + sb.base[2 * n + tid]) * cB;
-      T sR = sb.spec[0 * n + tid], sG = sb.spec[1 * n + tid], sB = sb.spec[2 * n + tid];
+      T oR = env.R * amb.R + (amb.R * k.global_ilum + lit.base[0]) * cR;
+      T oG = env.G * amb.G + (amb.G * k.global_ilum + lit.base[1]) * cG;
+      T oB = env.B * amb.B + (amb.B * k.global_ilum + lit.base[2]) * cB;
+      T sR = lit.spec[0], sG = lit.spec[1], sB = lit.spec[2];
       if (sc.n_lights > 0 || sc.fake_lights) {
         oR += sb.aux[0 * n + tid] * cR;
         oG += sb.aux[1 * n + tid] * cG;
@@ -1210,28 +1768,22 @@ __global__ void __launch_bounds__(kBlock) k_compose(const DevScene *__restrict__
       ((RT *)b.sp_r)[r] = (RT)sR;
       ((RT *)b.sp_g)[r] = (RT)sG;
       ((RT *)b.sp_b)[r] = (RT)sB;
-    } else if (lane == 0) {
-      const T cR = sb.col[0 * n + tid], cG = sb.col[1 * n + tid], cB = sb.col[2 * n + tid];
-      if (sc.n_lights > 0 || sc.fake_lights) {
-        // (ambient + main light) x colour + aux x colour, then aux specular
-        // + main specular (ObjectShader, src/shaders.cpp:96-108)
-        ((RT *)b.sh_r)[r] = (RT)(((env.R * amb.R + (amb.R * k.global_ilum + sb.base[0 * n + tid]) * cR) +
-                                  sb.aux[0 * n + tid] * cR) +
-                                 (sb.aux[3 * n + tid] + sb.spec[0 * n + tid]));
-        ((RT *)b.sh_g)[r] = (RT)(((env.G * amb.G + (amb.G * k.global_ilum + sb.base[1 * n + tid]) * cG) +
-                                  sb.aux[1 * n + tid] * cG) +
-                                 (sb.aux[4 * n + tid] + sb.spec[1 * n + tid]));
-        ((RT *)b.sh_b)[r] = (RT)(((env.B * amb.B + (amb.B * k.global_ilum + sb.base[2 * n + tid]) * cB) +
-                                  sb.aux[2 * n + tid] * cB) +
-                                 (sb.aux[5 * n + tid] + sb.spec[2 * n + tid]));
-      } else {
-        ((RT *)b.sh_r)[r] =
-            (RT)((env.R * amb.R + (amb.R * k.global_ilum + sb.base[0 * n + tid]) * cR) + sb.spec[0 * n + tid]);
-        ((RT *)b.sh_g)[r] =
-            (RT)((env.G * amb.G + (amb.G * k.global_ilum + sb.base[1 * n + tid]) * cG) + sb.spec[1 * n + tid]);
-        ((RT *)b.sh_b)[r] =
-            (RT)((env.B * amb.B + (amb.B * k.global_ilum + sb.base[2 * n + tid]) * cB) + sb.spec[2 * n + tid]);
-      }
+    } else if (sc.n_lights > 0 || sc.fake_lights) {
+      // (ambient + main light) x colour + aux x colour, then aux specular
+      // + main specular (ObjectShader, src/shaders.cpp:96-108)
+      ((RT *)b.sh_r)[r] = (RT)(((env.R * amb.R + (amb.R * k.global_ilum + lit.base[0]) * cR) +
+                                sb.aux[0 * n + tid] * cR) +
+                               (sb.aux[3 * n + tid] + lit.spec[0]));
+      ((RT *)b.sh_g)[r] = (RT)(((env.G * amb.G + (amb.G * k.global_ilum + lit.base[1]) * cG) +
+                                sb.aux[1 * n + tid] * cG) +
+                               (sb.aux[4 * n + tid] + lit.spec[1]));
+      ((RT *)b.sh_b)[r] = (RT)(((env.B * amb.B + (amb.B * k.global_ilum + lit.base[2]) * cB) +
+                                sb.aux[2 * n + tid] * cB) +
+                               (sb.aux[5 * n + tid] + lit.spec[2]));
+    } else {
+      ((RT *)b.sh_r)[r] = (RT)((env.R * amb.R + (amb.R * k.global_ilum + lit.base[0]) * cR) + lit.spec[0]);
+      ((RT *)b.sh_g)[r] = (RT)((env.G * amb.G + (amb.G * k.global_ilum + lit.base[1]) * cG) + lit.spec[1]);
+      ((RT *)b.sh_b)[r] = (RT)((env.B * amb.B + (amb.B * k.global_ilum + lit.base[2]) * cB) + lit.spec[2]);
     }
   }
 }
@@ -1696,12 +2248,20 @@ static inline void march_variant(int formula, int plain, bool ip8, Go go) {
   return ip8 ? go(f2, no, f8) : go(f2, no, z);
 }
 
-// Lanes per wave of a march over n rays: a band with fewer than 64 rays for
-// each of the two waves per SIMD that the FP64 units need to stay busy spreads
-// over that many waves, at least 4 rays each.
-static inline int march_lanes(int n, int persist_blocks) {
-  const int waves = std::max(1, persist_blocks);  // 8 workgroups per CU: two waves per SIMD
-  return std::min(64, std::max(4, (n + waves - 1) / waves));
+// Launch of a persistent kernel: at most the workgroups that fit the chip at
+// once (and `blocks`, the caller's share), so that no wave starts on its first
+// items only after the others ran out.
+template <auto Kernel, class... A>
+static void launch_resident(int blocks, hipStream_t s, A... args) {
+  static const int resident = [] {
+    int per_cu = 0, dev = 0, cus = 0;
+    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, Kernel, kBlock, 0) != hipSuccess ||
+        hipGetDevice(&dev) != hipSuccess ||
+        hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || per_cu * cus <= 0)
+      return 1 << 20;
+    return per_cu * cus;
+  }();
+  hipLaunchKernelGGL(Kernel, dim3((unsigned)std::max(1, std::min(blocks, resident))), dim3(kBlock), 0, s, args...);
 }
 
 static inline dim3 grid_for(int n) { return dim3((unsigned)((n + kBlock - 1) / kBlock)); }
@@ -1731,17 +2291,13 @@ hipError_t launch_refl_march(const DevScene *sc, const BandBufs &next, int band_
                              unsigned long long *stats, hipStream_t s) {
   const dim3 grid((unsigned)std::max(1, blocks));
   if (formula_generic(formula))
-    hipLaunchKernelGGL((k_march64<double, 0, 0, 0, kRefl>), grid, dim3(kBlock), 0, s, sc, next, band_first, 0, 64,
-                       stats);
+    launch_resident<k_march64<double, 0, 0, 0, kRefl>>(blocks, s, sc, next, band_first, 0, stats);
   else if (formula == 7)
-    hipLaunchKernelGGL((k_march64<double, 7, 0, 0, kRefl>), grid, dim3(kBlock), 0, s, sc, next, band_first, 0, 64,
-                       stats);
+    launch_resident<k_march64<double, 7, 0, 0, kRefl>>(blocks, s, sc, next, band_first, 0, stats);
   else if (formula == 8)
-    hipLaunchKernelGGL((k_march64<double, 8, 0, 0, kRefl>), grid, dim3(kBlock), 0, s, sc, next, band_first, 0, 64,
-                       stats);
+    launch_resident<k_march64<double, 8, 0, 0, kRefl>>(blocks, s, sc, next, band_first, 0, stats);
   else
-    hipLaunchKernelGGL((k_march64<double, 2, 0, 0, kRefl>), grid, dim3(kBlock), 0, s, sc, next, band_first, 0, 64,
-                       stats);
+    launch_resident<k_march64<double, 2, 0, 0, kRefl>>(blocks, s, sc, next, band_first, 0, stats);
   return hipGetLastError();
 }
 
@@ -1783,19 +2339,17 @@ hipError_t launch_march(int precision, const DevScene *sc, const BandBufs &b, in
     auto go = [&](auto f_tag, auto plain_tag, auto ip_tag) {
       constexpr int F = decltype(f_tag)::value;
       if constexpr (F != 0)
-        hipLaunchKernelGGL((k_march<F, decltype(plain_tag)::value, decltype(ip_tag)::value>), grid, dim3(kBlock), 0,
-                           s, sc, b, band_first, band_rays, stats);
+        launch_resident<k_march<F, decltype(plain_tag)::value, decltype(ip_tag)::value>>(persist_blocks, s, sc, b,
+                                                                                         band_first, band_rays, stats);
     };
     march_variant(formula, plain, ip8, go);
     return hipGetLastError();
   }
-  const int lanes = march_lanes(band_rays, persist_blocks);
   auto run = [&](auto rtag) {
     using RT = decltype(rtag);
     auto go = [&](auto f_tag, auto plain_tag, auto ip_tag) {
-      hipLaunchKernelGGL((k_march64<RT, decltype(f_tag)::value, decltype(plain_tag)::value, decltype(ip_tag)::value,
-                                    kRays>),
-                         grid, dim3(kBlock), 0, s, sc, b, band_first, band_rays, lanes, stats);
+      constexpr int F = decltype(f_tag)::value, Pl = decltype(plain_tag)::value, IP = decltype(ip_tag)::value;
+      launch_resident<k_march64<RT, F, Pl, IP, kRays>>(persist_blocks, s, sc, b, band_first, band_rays, stats);
     };
     march_variant(formula, plain, ip8, go);
   };
@@ -1814,10 +2368,8 @@ hipError_t launch_march_fix(const DevScene *sc, const BandBufs &b, int band_firs
     constexpr int F = decltype(f_tag)::value, IP = decltype(ip_tag)::value;
     constexpr int Pl = decltype(plain_tag)::value;
     if constexpr (F != 0) {
-      hipLaunchKernelGGL((k_march64<float, F, Pl, IP, kHand>), grid, dim3(kBlock), 0, s, sc, b, band_first, 0, 64,
-                         stats);
-      hipLaunchKernelGGL((k_march64<float, F, Pl, IP, kRedo>), grid, dim3(kBlock), 0, s, sc, b, band_first, 0, 64,
-                         stats);
+      launch_resident<k_march64<float, F, Pl, IP, kHand>>(persist_blocks, s, sc, b, band_first, 0, stats);
+      launch_resident<k_march64<float, F, Pl, IP, kRedo>>(persist_blocks, s, sc, b, band_first, 0, stats);
     }
   };
   march_variant(formula, plain, ip8, hand);
@@ -1870,20 +2422,27 @@ hipError_t shade_run(const DevScene *sc, const BandBufs &b, int band_first, AODe
   sb.aux = (T *)sbuf.aux;
   sb.n = sbuf.n;
   const bool generic = formula_generic(formula);
-  auto surf = [&](auto deep_tag) {
-    constexpr bool D = decltype(deep_tag)::value;
-    if constexpr (!D) {
-      if (generic) {
-        hipLaunchKernelGGL((k_surface<T, 0, false>), grid, dim3(kBlock), 0, s, sc, b, band_first, sb, stats);
-        return;
+  // deep-zoom variants only for FP32 shading of scenes that need them
+  const bool deep = sbuf.deep && sizeof(T) < 8 && !generic;
+  // the variants of the surface kernels; FP64 shades with the reference's
+  // trigonometric iteration
+  auto variants = [&](auto go) {
+    march_variant(formula, sbuf.plain, sbuf.ip8 && sizeof(T) < 8, [&](auto f_tag, auto plain_tag, auto ip_tag) {
+      if constexpr (decltype(f_tag)::value != 0) {
+        constexpr int IP = sizeof(T) < 8 ? decltype(ip_tag)::value : 0;
+        std::integral_constant<int, IP> ip;
+        if constexpr (sizeof(T) < 8) {
+          if (deep) return go(std::true_type{}, f_tag, plain_tag, ip);
+        }
+        go(std::false_type{}, f_tag, plain_tag, ip);
       }
-    }
-    if (formula == 7)
-      hipLaunchKernelGGL((k_surface<T, 7, D>), grid, dim3(kBlock), 0, s, sc, b, band_first, sb, stats);
-    else if (formula == 8)
-      hipLaunchKernelGGL((k_surface<T, 8, D>), grid, dim3(kBlock), 0, s, sc, b, band_first, sb, stats);
-    else
-      hipLaunchKernelGGL((k_surface<T, 2, D>), grid, dim3(kBlock), 0, s, sc, b, band_first, sb, stats);
+    });
+  };
+  auto hits = [&](int kinds) {
+    variants([&](auto d, auto f, auto pl, auto ip) {
+      constexpr int F = decltype(f)::value, Pl = decltype(pl)::value, IP = decltype(ip)::value;
+      launch_resident<k_hits<T, F, decltype(d)::value, Pl, IP>>(persist_blocks, s, sc, b, sb, kinds, stats);
+    });
   };
   // plain scenes take a variant without the optional terms' branches (and the
   // scene constants they keep live); FP32 deep-zoom scenes the one that starts
@@ -1892,16 +2451,35 @@ hipError_t shade_run(const DevScene *sc, const BandBufs &b, int band_first, AODe
     constexpr bool D = decltype(deep_tag)::value;
     constexpr int F = decltype(f_tag)::value, Pl = decltype(plain_tag)::value, IP = decltype(ip_tag)::value;
     if constexpr (!D && Pl && std::is_same<T, float>::value)
-      hipLaunchKernelGGL((k_ao_f32_plain<T, F, Pl, IP>), grid, dim3(kBlock), 0, s, sc, b, ao, sb, stats);
+      launch_resident<k_ao_f32_plain<T, F, Pl, IP>>(persist_blocks, s, sc, b, ao, sb, stats);
     else if constexpr (Pl)
-      hipLaunchKernelGGL((k_ao<T, F, D, Pl, IP>), grid, dim3(kBlock), 0, s, sc, b, ao, sb, stats);
+      launch_resident<k_ao<T, F, D, Pl, IP>>(persist_blocks, s, sc, b, ao, sb, stats);
     else
-      hipLaunchKernelGGL((k_ao<T, F, D, Pl>), grid, dim3(kBlock), 0, s, sc, b, ao, sb, stats);
+      launch_resident<k_ao<T, F, D, Pl>>(persist_blocks, s, sc, b, ao, sb, stats);
   };
-  // deep-zoom variants only for FP32 shading of scenes that need them
-  const bool deep = sbuf.deep && sizeof(T) < 8 && !generic;
-  if (deep) surf(std::true_type{});
-  else surf(std::false_type{});
+  int ended = 0;
+  if (generic) {
+    hipLaunchKernelGGL((k_surface_generic<T>), grid, dim3(kBlock), 0, s, sc, b, band_first, sb, stats);
+    ended = 1;
+  } else {
+    // the colour of a deep hit under shadow_fx depends on the detail size its
+    // shadow ray left
+    if (deep && sbuf.shadow_fx) {
+      hits(HIT_SHADOW | HIT_NORMAL);
+      hits(HIT_COLOUR);
+    } else {
+      hits(HIT_SHADOW | HIT_NORMAL | HIT_COLOUR);
+    }
+    if (sbuf.fast_ao_on)
+      variants([&](auto d, auto f, auto pl, auto ip) {
+        constexpr int F = decltype(f)::value, Pl = decltype(pl)::value, IP = decltype(ip)::value;
+        launch_resident<k_fast_ao<T, F, decltype(d)::value, Pl, IP>>(persist_blocks, s, sc, b, sb, stats);
+      });
+    if (sbuf.lights || sbuf.env) {
+      hipLaunchKernelGGL((k_hits_end<T>), grid, dim3(kBlock), 0, s, sc, b, band_first, sb);
+      ended = 1;
+    }
+  }
   if (sbuf.lights) {
     if (generic) {
       if constexpr (std::is_same<T, double>::value)
@@ -1937,7 +2515,7 @@ hipError_t shade_run(const DevScene *sc, const BandBufs &b, int band_first, AODe
     hipError_t e = hipEventRecord(ev_ao1, s);
     if (e != hipSuccess) return e;
   }
-  hipLaunchKernelGGL((k_compose<T, T>), grid, dim3(kBlock), 0, s, sc, b, ao, sb);
+  hipLaunchKernelGGL((k_compose<T, T>), grid, dim3(kBlock), 0, s, sc, b, band_first, ao, sb, ended);
   return hipGetLastError();
 }
 #endif

@@ -21,10 +21,12 @@ enum StatIdx {
 // Band counters (BandBufs::counters), zeroed on the device at band start:
 // hits appended, rays handed to the FP64 continuation, primary-ray queue,
 // overflow runs handed out, AO work queue, rays listed for the FP64 redo,
-// overflow chunks, the queues over the handed-over and the redo rays.
+// overflow chunks, the queues over the handed-over and the redo rays and over
+// the hits' shadow rays, normals, colours and fast AO.
 enum CounterIdx {
   CNT_HITS = 0, CNT_HAND = 1, CNT_RAYQ = 2, CNT_DIRS = 3, CNT_AOQ = 4, CNT_REDO = 5, CNT_CHUNKS = 6,
-  CNT_HANDQ = 7, CNT_REDOQ = 8, CNT_COUNT = 16
+  CNT_HANDQ = 7, CNT_REDOQ = 8, CNT_SHADOWQ = 9, CNT_NORMALQ = 10, CNT_COLOURQ = 11, CNT_FASTQ = 12,
+  CNT_COUNT = 16
 };
 
 // Formulas of the render core; the generic ones (no kernels of their own)
@@ -126,7 +128,10 @@ struct ShadeBufs {
   int plain;                    // 1: no primitives, limits, interior, iteration threshold, pre-folds, Julia
   int formula;
   int lights;                   // 1: aux lights take part (k_aux runs after k_surface)
-  int ip8;                      // 1: Mandelbulb of power 8 (AO kernel with the power fixed)
+  int ip8;                      // 1: Mandelbulb of power 8 (kernels with the power fixed)
+  int fast_ao_on;               // 1: FastAmbientOcclusion2 instead of the AmbientOcclusion rays
+  int env;                      // 1: environment mapping
+  int shadow_fx;                // 1: shadow marches take their thresholds from the distance to the eye
 };
 // Shading in three launches: surface (normals, shadow, specular, colour,
 // fast AO), AO rays, composition; ev_ao (when not null) is recorded around

@@ -377,8 +377,8 @@ MBR_HD void index_to_colour(int index, const int (*palette)[3], int out[3]) {
   }
 }
 
-// G: the colouring orbit may be a generic formula's (compute's G)
-template <class T, bool Deep = false, bool G = (sizeof(T) == 8)>
+// G, FF, P: compute's (the colouring orbit may be a generic formula's)
+template <class T, bool Deep = false, bool G = (sizeof(T) == 8), int FF = 0, int P = 0>
 MBR_HD RGBT<T> surface_colour(const DevScene &sc, const ShaderIn<T> &in, LaneCount &cnt) {
   RGBT<T> out;
   const int *pc;
@@ -389,9 +389,9 @@ MBR_HD RGBT<T> surface_colour(const DevScene &sc, const ShaderIn<T> &in, LaneCou
       T cval;
       if (Deep && sizeof(T) < 8 && (double)in.detail < 2.0 * kMixedSwitch * length(in.point64))
         // deep zoom: the FP32 point would merge neighbouring pixels' orbits
-        cval = (T)compute<double, MODE_COLOURING>(sc.fd, in.point64, N10, &L);
+        cval = (T)compute<double, MODE_COLOURING, FF == 0, FF, P>(sc.fd, in.point64, N10, &L);
       else
-        cval = compute<T, MODE_COLOURING, G>(sc.frac<T>(), in.point, N10, &L);
+        cval = compute<T, MODE_COLOURING, G, FF, P>(sc.frac<T>(), in.point, N10, &L);
       cnt.de_calls += 1;
       cnt.iterations += (uint32_t)((L < N10) ? L + 1 : N10);
       int nrCol = x86_d2i(floor((double)cval));

@@ -1,0 +1,53 @@
+"""The surface and AO kernels (k_hits, k_fast_ao, k_ao's split hits) where
+their hand-out can go wrong, against the oracle: frames with fewer hits than a
+wave, ragged ones, AO quality 1 to 3 (several hits per wave) and hits split over
+waves, soft shadows, the chained slowShading stencil, FastAmbientOcclusion2.
+FP64 frames hold the bars of the parity tests for the same arithmetic (equal
+integer planes, 120 dB); FP32_FIXUP frames the parity bars."""
+import pytest
+
+from mandelbulber_amd import _abi, scene
+from metrics import assert_parity, assert_planes_exact, compare
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def renderer():
+    import torch
+    if not torch.cuda.is_available():
+        pytest.fail("GPU tests need a visible GPU")
+    from mandelbulber_amd import Renderer
+    r = Renderer(0)
+    yield r
+    r.close()
+
+
+SOFT = {"shadows_enabled": 1, "shadows_cone_angle": 4, "penetrating_lights": 0}
+FAST = {"ambient_occlusion_enabled": 1, "fast_ambient_occlusion_mode": 1, "ambient_occlusion_quality": 3}
+VIEWS = {"bulb": scene.mandelbulb_plain, "box": lambda w, h: scene.mandelbox_view(w, h, shaded=False),
+         "menger": lambda w, h: scene.menger_view(w, h, shaded=False)}
+
+CASES = [("bulb", 5, 3, dict(SOFT, **FAST)), ("box", 7, 5, dict(SOFT, **FAST)), ("menger", 61, 37, dict(SOFT, **FAST)),
+         ("box", 19, 13, {"slow_shading": 1}), ("menger", 3, 2, {"slow_shading": 1})]
+for _q in (1, 2, 3, 6):
+    CASES.append(("box", 21, 17, {"shadows_enabled": 1, "shadows_cone_angle": 0, "ambient_occlusion_enabled": 1,
+                                  "ambient_occlusion_quality": _q}))
+
+
+@pytest.mark.parametrize("kind,w,h,keys", CASES)
+def test_shaded_hits_match_oracle(renderer, kind, w, h, keys):
+    from oracle import oracle
+    s = VIEWS[kind](w, h)
+    a, b = scene.light_from_seed(5)
+    scene.apply(s, dict(keys, main_light_alfa=a, main_light_beta=b))
+    print(f"[hits] {kind} {w}x{h} {keys}", flush=True)
+    ref, _ = oracle.render(s)
+    renderer.set_scene(s)
+    f64, st = renderer.render(precision=_abi.PREC_FP64)
+    m = compare(f64, ref)
+    print(f"  {st.hits} hits {m}", flush=True)
+    assert st.hits > 0 and m["flips"] == 0 and m["depth_rel_max"] <= 1e-12 and m["psnr_db"] >= 120, m
+    assert_planes_exact(m)
+    fix, _ = renderer.render(precision=_abi.PREC_FP32_FIXUP)
+    assert_parity(compare(fix, ref), label="fixup")
