@@ -941,7 +941,7 @@ int prepare_scene(mbr_ctx *c, const mbr_scene *scene_in, const mbr_texture *ligh
   d.plain = d.fd.limits == 0 && d.fd.only_plane == 0 && d.fd.interior == 0 && d.fd.iter_thresh == 0 &&
             !d.fd.prim_plane && !d.fd.prim_box && !d.fd.prim_ibox && !d.fd.prim_sphere && !d.fd.prim_isphere &&
             !d.fd.prim_water && !d.fd.tglad_fold && !d.fd.sph_fold && !d.fd.julia_mode && !d.fd.ifs_fold;
-  if (d.plain) d.plain = s.formula == 8 && !d.fd.mb_rot_on && !d.fd.mb_main_rot ? kUnrotated : kPlain;
+  if (d.plain) d.plain = s.formula == 8 && standard_box(d.fd) && standard_box(d.ff) ? kStandardBox : kPlain;
   return MBR_OK;
 }
 

@@ -111,11 +111,18 @@ MBR_HD void rotate_right(T *m, bool &ident, int axis, T angle) {
 
 // P: what the caller knows of the scene: kOptions nothing, kPlain that no
 // optional term is on (primitives, limits, interior mode, iteration
-// threshold, pre-folds, Julia constant), kUnrotated (Mandelbox) in addition
-// that its folds and its main rotation are not rotated.  The 19 rotation
-// matrices otherwise fill the scalar registers of every kernel that holds
-// the iteration (380-450 spills into vector lanes, read back in every pass).
-enum : int { kOptions = 0, kPlain = 1, kUnrotated = 2 };
+// threshold, pre-folds, Julia constant), kStandardBox (Mandelbox) in addition
+// that nothing is rotated or offset, the fold value is twice the limit and the
+// fold radii are not tiny (standard_box).  The 19 rotation matrices otherwise
+// fill the scalar registers of every kernel that holds the iteration (380-450
+// spills into vector lanes, read back in every pass).
+enum : int { kOptions = 0, kPlain = 1, kStandardBox = 2 };
+
+template <class T>
+MBR_HD bool standard_box(const FractalK<T> &f) {
+  return !f.mb_rot_on && !f.mb_main_rot && f.mb_offset[0] == 0 && f.mb_offset[1] == 0 && f.mb_offset[2] == 0 &&
+         f.mb_limit >= 0 && f.mb_value == T(2) * f.mb_limit && f.mb_mR2 > T(1e-20) && f.mb_fR2 >= f.mb_mR2;
+}
 
 // G: the formulas of the generic path are compiled in (always in FP64; in
 // FP32 for the FP32 shading of the analytic generic formulas, whose kernels
@@ -222,7 +229,7 @@ MBR_HD T compute(const FractalK<T> &f, V3<T> z, int N, int *iter_count) {
       tgladDE *= T(3);
     } else if (af == 8) {  // tglad (Mandelbox)
       const T lim = f.mb_limit, val = f.mb_value;
-      if (P != kUnrotated && f.mb_rot_on) {
+      if (P != kStandardBox && f.mb_rot_on) {
         bool lockout = false;
         z = rot9(f.mb_rot[0][0], z);
         if (z.x > lim) { z.x = val - z.x; tgladColor += f.mb_col_X; lockout = true; }
@@ -258,7 +265,7 @@ MBR_HD T compute(const FractalK<T> &f, V3<T> z, int N, int *iter_count) {
       if (r2 < f.mb_mR2) { z = z * f.mb_factor1; tgladDE *= f.mb_factor1; tgladColor += f.mb_col_Sp1; }
       else if (r2 < f.mb_fR2) { T tf2 = f.mb_fR2 / r2; z = z * tf2; tgladDE *= tf2; tgladColor += f.mb_col_Sp2; }
       z = z - ld3(f.mb_offset);
-      if (P != kUnrotated && f.mb_main_rot) z = mat_apply(f.mb_main, z);
+      if (P != kStandardBox && f.mb_main_rot) z = mat_apply(f.mb_main, z);
       z = z * mscale + constant;
       tgladDE = tgladDE * mabs + T(1);
       r = length_nc(z);
@@ -786,7 +793,7 @@ struct DEIter {
 
 // IP: the Mandelbulb's integer power when the caller knows it at compile
 // time (8, the standard bulb), else 0 (read from f.ipow).
-// P: kOptions, kPlain or kUnrotated.
+// P: kOptions, kPlain or kStandardBox.
 template <class T, int F, int P = 0, bool A = (sizeof(T) < 8), int IP = 0>
 MBR_HD void de_begin(const FractalK<T> &f, V3<T> p, DEIter<T> &s) {
   s.z = p;
@@ -806,10 +813,10 @@ MBR_HD void de_begin(const FractalK<T> &f, V3<T> p, DEIter<T> &s) {
 
 // !(|z| <= R) of the folding formulas' escape test from q = |z|^2, for R =
 // 1000 or 1024, without the square root: an FP64 root and its refinement are
-// about as long as a whole Menger iteration.  FP64 roots are correctly
-// rounded, so |z| <= R exactly when q is at most the largest double whose
-// root rounds to R.  FP32 roots are the hardware's (1 ulp): inside a band of
-// 2^-20 about R^2 the root itself decides.  NaN counts as escaped.
+// about as long as a whole Menger iteration.  The bound is the largest q whose
+// root is at most R: FP64 roots are correctly rounded; gfx950's v_sqrt_f32
+// gives R for R^2 and the next FP32 value above it and more than R from there
+// on.  NaN counts as escaped.
 template <int R>
 MBR_HD bool beyond(double q) {
   static_assert(R == 1000 || R == 1024, "");
@@ -817,10 +824,33 @@ MBR_HD bool beyond(double q) {
 }
 template <int R>
 MBR_HD bool beyond(float q) {
-  constexpr float R2 = (float)R * R, lo = R2 * (1.0f - 0x1p-20f), hi = R2 * (1.0f + 0x1p-20f);
-  bool e = !(q <= hi);
-  if (q > lo && q <= hi) e = !(Math<float>::sqrt(q) <= (float)R);
-  return e;
+  return !(q <= (R == 1000 ? 0x1.e84802p+19f : 0x1.000002p+20f));
+}
+
+// The larger and the smaller of two values, and z limited to [-lim, lim].
+MBR_HD double larger(double a, double b) { return __builtin_fmax(a, b); }
+MBR_HD double smaller(double a, double b) { return __builtin_fmin(a, b); }
+MBR_HD float larger(float a, float b) { return __builtin_fmaxf(a, b); }
+MBR_HD float smaller(float a, float b) { return __builtin_fminf(a, b); }
+MBR_HD double limited(double z, double lim) { return smaller(larger(z, -lim), lim); }
+MBR_HD float limited(float z, float lim) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  return __builtin_amdgcn_fmed3f(z, -lim, lim);
+#else
+  return smaller(larger(z, -lim), lim);
+#endif
+}
+MBR_HD double fused(double a, double b, double c) { return __builtin_fma(a, b, c); }
+MBR_HD float fused(float a, float b, float c) { return __builtin_fmaf(a, b, c); }
+// sqrt(q) for a radius compared with the sphere fold's (kStandardBox: the fold's
+// squared radii are far above the values FP32 roots would have to rescale)
+MBR_HD double fold_root(double q) { return Math<double>::sqrt(q); }
+MBR_HD float fold_root(float q) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  return __builtin_amdgcn_sqrtf(q);
+#else
+  return Math<float>::sqrt(q);
+#endif
 }
 
 // One loop pass.  Returns true when the call has finished: the orbit escaped
@@ -949,19 +979,37 @@ MBR_HD bool de_iter(const FractalK<T> &f, DEIter<T> &s, int N) {
     s.r = r;
     esc = !(r <= f.bailout);
   } else if constexpr (F == 7) {  // menger_sponge
-    T temp;
-    z.x = M::fabs(z.x); z.y = M::fabs(z.y); z.z = M::fabs(z.z);
-    if (z.x - z.y < 0) { temp = z.y; z.y = z.x; z.x = temp; }
-    if (z.x - z.z < 0) { temp = z.z; z.z = z.x; z.x = temp; }
-    if (z.y - z.z < 0) { temp = z.z; z.z = z.y; z.y = temp; }
+    // |x|, |y|, |z| in descending order: the reference's three conditional
+    // swaps, as maxima and minima (2 instructions each for 4 in FP32, 6 in FP64)
+    const T ax = M::fabs(z.x), ay = M::fabs(z.y), az = M::fabs(z.z);
+    const T hi = larger(ax, ay), lo = smaller(ax, ay);
+    const T mid = smaller(hi, az);
+    z = V3<T>{larger(hi, az), larger(lo, mid), smaller(lo, mid)};
     z = z * T(3);
     z.x -= T(2); z.y -= T(2);
-    if (z.z > T(1)) z.z -= T(2);
+    z.z -= z.z > T(1) ? T(2) : T(0);
     s.aux *= T(3);
     esc = beyond<1000>(dot(z, z));
+  } else if constexpr (P == kStandardBox) {  // tglad (Mandelbox)
+    // The box fold with value = 2 limit is 2 clamp(z) - z, exactly (z where it
+    // lies inside); the sphere fold's factor is 1 outside, and every factor
+    // multiplies z and the derivative without a branch: 42 instead of 75 issue
+    // slots in FP32, where in a full wave all branches are taken anyway.
+    const T lim = f.mb_limit;
+    z = V3<T>{fused(T(2), limited(z.x, lim), -z.x), fused(T(2), limited(z.y, lim), -z.y),
+              fused(T(2), limited(z.z, lim), -z.z)};
+    const T rf = fold_root(dot(z, z));
+    const T r2 = rf * rf;
+    T k = r2 < f.mb_fR2 ? fdiv(f.mb_fR2, r2) : T(1);
+    k = r2 < f.mb_mR2 ? f.mb_factor1 : k;
+    z = z * k;
+    s.aux *= k;
+    z = z * f.mb_scale + s.c;
+    s.aux = s.aux * f.mb_abs_scale + T(1);
+    esc = beyond<1024>(dot(z, z));
   } else {  // tglad (Mandelbox)
     const T lim = f.mb_limit, val = f.mb_value;
-    if (P != kUnrotated && f.mb_rot_on) {
+    if (f.mb_rot_on) {
       bool lockout = false;
       z = rot9(f.mb_rot[0][0], z);
       if (z.x > lim) { z.x = val - z.x; lockout = true; }
@@ -997,7 +1045,7 @@ MBR_HD bool de_iter(const FractalK<T> &f, DEIter<T> &s, int N) {
     if (r2 < f.mb_mR2) { z = z * f.mb_factor1; s.aux *= f.mb_factor1; }
     else if (r2 < f.mb_fR2) { T tf2 = fdiv(f.mb_fR2, r2); z = z * tf2; s.aux *= tf2; }
     z = z - ld3(f.mb_offset);
-    if (P != kUnrotated && f.mb_main_rot) z = mat_apply(f.mb_main, z);
+    if (f.mb_main_rot) z = mat_apply(f.mb_main, z);
     z = z * f.mb_scale + s.c;
     s.aux = s.aux * f.mb_abs_scale + T(1);
     esc = beyond<1024>(dot(z, z));

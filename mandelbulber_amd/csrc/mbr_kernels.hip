@@ -2236,11 +2236,11 @@ static inline void march_variant(int formula, int plain, bool ip8, Go go) {
   std::integral_constant<int, 8> f8;
   std::integral_constant<int, kPlain> yes;
   std::integral_constant<int, kOptions> no;
-  std::integral_constant<int, kUnrotated> box;
+  std::integral_constant<int, kStandardBox> box;
   if (formula_generic(formula)) return go(z, no, z);
   if (plain) {
     if (formula == 7) return go(f7, yes, z);
-    if (formula == 8) return plain == kUnrotated ? go(f8, box, z) : go(f8, yes, z);
+    if (formula == 8) return plain == kStandardBox ? go(f8, box, z) : go(f8, yes, z);
     return ip8 ? go(f2, yes, f8) : go(f2, yes, z);
   }
   if (formula == 7) return go(f7, no, z);
