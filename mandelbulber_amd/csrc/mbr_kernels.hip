@@ -37,6 +37,9 @@ constexpr double kPi = 3.14159265358979323846;
 // re-march of the same ray reuses them.  When the pool is full the record
 // is dropped and ST_POOL_MISS tells the host to grow the pool and render
 // the band again.  All records of one ray are written by one lane.
+constexpr unsigned long long kOneDir = 1ull << 32;
+// fields of a lane's overflow count (misses: one bit)
+constexpr unsigned long long kOvfRay = 1, kOvfChunk = 1ull << 20, kOvfMiss = 1ull << 44;
 template <class RT>
 struct RecPlanes {
   RT *step, *dist, *thr;     // slab planes
@@ -44,10 +47,13 @@ struct RecPlanes {
   int *it, *oit;             // iteration counts (null unless iteration fog is on)
   long long *ovf_off;
   int *dir;
-  unsigned long long *dirs, *chunks, *stats;
+  unsigned long long *pool;  // directories (times kOneDir) and chunks handed out
   long long cap, max_dirs, max_chunks;
   int slab, r;
-  __device__ __forceinline__ void put(int i, double step_v, double dist_v, double thr_v, int iters) const {
+  // ovf counts what the ray's lane adds to the overflow counters of the stats;
+  // an add to a shared counter for each would serialise the waves
+  __device__ __forceinline__ void put(int i, double step_v, double dist_v, double thr_v, int iters,
+                                      unsigned long long &ovf) const {
     long long o;
     RT *st, *di, *th;
     int *itp;
@@ -56,29 +62,36 @@ struct RecPlanes {
       st = step; di = dist; th = thr; itp = it;
     } else {
       long long dj = ovf_off[r];
+      int first = -1;
       if (dj == -1) {
-        const unsigned long long n = atomicAdd(dirs, 1ull);
-        atomicAdd(&stats[ST_OVF_RAYS], 1ull);
-        dj = n < (unsigned long long)max_dirs ? (long long)n : -2;
+        // a directory and the first chunk with one add
+        const unsigned long long n = atomicAdd(pool, kOneDir + 1);
+        ovf += kOvfRay;
+        dj = (long long)(n / kOneDir) < max_dirs ? (long long)(n / kOneDir) : -2;
+        const long long ch = (long long)(n % kOneDir);
+        first = ch < max_chunks ? (int)ch : -2;
         if (dj >= 0)
           for (int k = 0; k < kDirSlots; k++) dir[dj * kDirSlots + k] = -1;
         ovf_off[r] = dj;
       }
       if (dj < 0) {
-        atomicAdd(&stats[ST_POOL_MISS], 1ull);
+        ovf |= kOvfMiss;
         return;
       }
       const int rel = i - slab;
       int *slot = &dir[dj * kDirSlots + rel / kChunk];
-      int ch = *slot;
+      int ch = first != -1 ? first : *slot;
       if (ch == -1) {
-        const unsigned long long n = atomicAdd(chunks, 1ull);
-        atomicAdd(&stats[ST_OVF_CHUNKS], 1ull);
-        ch = n < (unsigned long long)max_chunks ? (int)n : -2;
+        const long long n = (long long)(atomicAdd(pool, 1ull) % kOneDir);
+        ch = n < max_chunks ? (int)n : -2;
+        first = ch;
+      }
+      if (first != -1) {
+        ovf += kOvfChunk;
         *slot = ch;
       }
       if (ch < 0) {
-        atomicAdd(&stats[ST_POOL_MISS], 1ull);
+        ovf |= kOvfMiss;
         return;
       }
       o = (long long)ch * kChunk + rel % kChunk;
@@ -90,6 +103,13 @@ struct RecPlanes {
     if (itp) itp[o] = iters;
   }
 };
+
+// The overflow counts of a lane into its stats.
+__device__ __forceinline__ void add_ovf(unsigned long long (&v)[ST_COUNT], unsigned long long ovf) {
+  v[ST_OVF_RAYS] = ovf % kOvfChunk;
+  v[ST_OVF_CHUNKS] = ovf / kOvfChunk % (kOvfMiss / kOvfChunk);
+  v[ST_POOL_MISS] = ovf / kOvfMiss;
+}
 
 // block-level reduction of per-lane counters into the device stats: LDS
 // atomics inside the workgroup, then one global atomic per counter
@@ -190,7 +210,7 @@ __device__ __forceinline__ void march_before_de(const MarchK &m, V3<double> star
 // obj_it: the estimate's object type in the low 3 bits, its iteration count
 // (CalculateDistance's itersOut) above them.
 __device__ __forceinline__ int march_after_de(const MarchK &m, RayState &s, double d, int obj_it, uint32_t ray_hash,
-                                              const RecPlanes<float> &rec) {
+                                              const RecPlanes<float> &rec, unsigned long long &ovf) {
 #pragma clang fp contract(off)
   s.object = obj_it & 7;
   const double dist = d > 3.0 ? 3.0 : d;
@@ -201,7 +221,7 @@ __device__ __forceinline__ int march_after_de(const MarchK &m, RayState &s, doub
   const double jf = m.jitter ? jitter_factor(jitter_draw(ray_hash, (uint32_t)s.i)) : 1.0;
   const double old_step = s.step;
   s.step = (dist - m.below * s.thr) * m.DE_factor * jf;
-  rec.put(s.i, old_step, d, s.thr, obj_it >> 3);
+  rec.put(s.i, old_step, d, s.thr, obj_it >> 3, ovf);
   s.scan += s.step;
   s.drift += (err * m.DE_factor) * (err * m.DE_factor);
   s.dist = dist;
@@ -224,7 +244,7 @@ __device__ __forceinline__ RayState ray_start_state(const DevScene &sc) {
   return s;
 }
 
-// A ray whose march ended without the FP64 continuation (a miss).
+// The result of a ray's march.
 __device__ __forceinline__ void write_ray(const BandBufs &b, int r, const MarchOut &o) {
   b.found[r] = o.found;
   b.object[r] = (uint8_t)o.object;
@@ -235,14 +255,51 @@ __device__ __forceinline__ void write_ray(const BandBufs &b, int r, const MarchO
   b.px[r] = o.point.x;
   b.py[r] = o.point.y;
   b.pz[r] = o.point.z;
-  if (o.found) {
-    const unsigned long long h = atomicAdd(&b.counters[CNT_HITS], 1ull);
-    b.hit_list[h] = r;
-  }
 }
 
+// Appends to one of the band's lists (hits, hand-overs, redos) through a buffer
+// of the wave in LDS, 64 entries per add to the list's counter: adds to one
+// address pass at about 13 ns each, so one add per hit-finding step block held
+// a 4K frame's march for several ms.  Lists have no order.
+struct WaveListBuf {
+  int entry[kBlock / 64][128];
+  int count[kBlock / 64];
+};
+struct WaveList {
+  WaveListBuf &buf;
+
+  __device__ __forceinline__ explicit WaveList(WaveListBuf &buf_) : buf(buf_) {
+    buf.count[threadIdx.x >> 6] = 0;
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  }
+  // by any lanes
+  __device__ __forceinline__ void append(int r) {
+    const int w = (int)(threadIdx.x >> 6);
+    buf.entry[w][atomicAdd(&buf.count[w], 1)] = r;
+  }
+  // by the whole wave, after at most one append per lane; all: to the last entry
+  __device__ __forceinline__ void flush(int *out, unsigned long long *counter, bool all) {
+    const int lane = __lane_id(), w = (int)(threadIdx.x >> 6);
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    int n = __builtin_amdgcn_readfirstlane(buf.count[w]);
+    while (n >= 64 || (all && n > 0)) {
+      const int m = n < 64 ? n : 64;
+      unsigned long long base = 0;
+      if (lane == 0) base = atomicAdd(counter, (unsigned long long)m);
+      base = __shfl(base, 0);
+      if (lane < m) out[base + lane] = buf.entry[w][lane];
+      const int rest = 64 + lane < n ? buf.entry[w][64 + lane] : 0;
+      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+      if (64 + lane < n) buf.entry[w][lane] = rest;
+      n -= m;
+      buf.count[w] = n;
+      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    }
+  }
+};
+
 template <class RT>
-__device__ __forceinline__ RecPlanes<RT> ray_records(const BandBufs &b, int r, unsigned long long *stats) {
+__device__ __forceinline__ RecPlanes<RT> ray_records(const BandBufs &b, int r) {
   RecPlanes<RT> rec;
   rec.step = (RT *)b.rec_step;
   rec.dist = (RT *)b.rec_dist;
@@ -254,9 +311,7 @@ __device__ __forceinline__ RecPlanes<RT> ray_records(const BandBufs &b, int r, u
   rec.oit = b.ovf_it;
   rec.ovf_off = b.ovf_off;
   rec.dir = b.ovf_dir;
-  rec.dirs = &b.counters[CNT_DIRS];
-  rec.chunks = &b.counters[CNT_CHUNKS];
-  rec.stats = stats;
+  rec.pool = &b.counters[CNT_POOL];
   rec.cap = b.cap;
   rec.max_dirs = b.ovf_dirs;
   rec.max_chunks = b.ovf_chunks;
@@ -385,6 +440,8 @@ __device__ __forceinline__ void march_body(const DevScene *__restrict__ scp, Ban
   const V3<double> start = v3<double>(sc.start[0], sc.start[1], sc.start[2]);
 
   const MarchK m = march_k(sc);
+  __shared__ WaveListBuf hand_buf;
+  WaveList hand(hand_buf);
   const int lanes = item_lanes(band_rays);
   WaveQueue q(&b.counters[CNT_RAYQ], band_rays, lanes);
   int state = lane < lanes ? MS_NEED : MS_EXHAUSTED;
@@ -397,6 +454,7 @@ __device__ __forceinline__ void march_body(const DevScene *__restrict__ scp, Ban
   int object = OBJ_FRACTAL;
   bool early = false;  // the estimate ended in begin_de, without iterating
   LaneCount cnt = {0, 0};
+  unsigned long long ovf = 0;
 
   auto begin_de = [&]() {
     march_before_de(m, start, dir, s);
@@ -452,6 +510,7 @@ __device__ __forceinline__ void march_body(const DevScene *__restrict__ scp, Ban
 
     const unsigned long long m_done2 = __ballot(state == MS_DONE);
     const unsigned long long m_iter2 = __ballot(state == MS_ITER);
+    bool appended = false;
     const int n_done2 = __popcll(m_done2), n_iter2 = __popcll(m_iter2);
     if (n_done2 && (4 * n_done2 >= n_done2 + n_iter2 || n_iter2 == 0) && state == MS_DONE) {
       cnt.de_calls += 1;
@@ -461,7 +520,7 @@ __device__ __forceinline__ void march_body(const DevScene *__restrict__ scp, Ban
         object = info.object | (info.iters << 3);
         cnt.iterations += (uint32_t)info.work;
       }
-      const int out = march_after_de(m, s, (double)dist, object, ray_hash, ray_records<RT>(b, r, stats));
+      const int out = march_after_de(m, s, (double)dist, object, ray_hash, ray_records<RT>(b, r), ovf);
       if (out == SO_CONTINUE) {
         begin_de();
       } else if (out == SO_MISS) {
@@ -477,18 +536,21 @@ __device__ __forceinline__ void march_body(const DevScene *__restrict__ scp, Ban
         write_ray(b, r, o);
         state = MS_NEED;
       } else {
-        const unsigned long long h = atomicAdd(&b.counters[CNT_HAND], 1ull);
-        b.hand_ray[h] = r;
-        b.hand_i[h] = s.i;
-        b.hand_scan[h] = s.scan;
-        b.hand_step[h] = s.step;
-        b.hand_drift[h] = s.drift;
-        b.hand_dist[h] = s.dist;
+        hand.append(r);
+        b.hand_i[r] = s.i;
+        b.hand_scan[r] = s.scan;
+        b.hand_step[r] = s.step;
+        b.hand_drift[r] = s.drift;
+        b.hand_dist[r] = s.dist;
+        appended = true;
         state = MS_NEED;
       }
     }
+    if (__ballot(appended)) hand.flush(b.hand_ray, &b.counters[CNT_HAND], false);
   }
+  hand.flush(b.hand_ray, &b.counters[CNT_HAND], true);
   unsigned long long v[ST_COUNT] = {0};
+  add_ovf(v, ovf);
   v[ST_MARCH_DE] = cnt.de_calls;
   v[ST_MARCH_ITERS] = cnt.iterations;
   flush_stats(stats, v);
@@ -541,6 +603,10 @@ __device__ __forceinline__ void march64_body(const DevScene *__restrict__ scp, B
   const unsigned long long lt_mask = (lane == 0) ? 0ull : (~0ull >> (64 - lane));
   const long long n_items = Src == kRays ? (long long)band_rays
                                          : (long long)b.counters[Src == kRedo ? CNT_REDO : CNT_HAND];
+  __shared__ WaveListBuf hit_buf, redo_buf;  // (the latter's space is kHand's only)
+  WaveList hit_list(hit_buf);
+  WaveList redo_list(Src == kHand ? redo_buf : hit_buf);
+  bool appended = false;
   const int lanes = item_lanes(n_items);
   WaveQueue q(&b.counters[Src == kRays ? CNT_RAYQ : Src == kRedo ? CNT_REDOQ : CNT_HANDQ], n_items, lanes);
   const double search_limit = 1.0 - 0.01 * m.quality;
@@ -563,6 +629,7 @@ __device__ __forceinline__ void march64_body(const DevScene *__restrict__ scp, B
   bool early = false, ambiguous = false, have_prev = false, below = false;
   int early_obj = 0;  // object and iterations << 3 of an early estimate
   LaneCount cnt = {0, 0};
+  unsigned long long ovf = 0;
   unsigned long long hits = 0, missed = 0, redo = 0;
 
   // start the estimate at distance t along the ray (detail size s.thr)
@@ -580,23 +647,25 @@ __device__ __forceinline__ void march64_body(const DevScene *__restrict__ scp, B
   // step s.i of the march
   auto begin_march = [&]() {
 #pragma clang fp contract(off)
-    march_before_de(m, start, dir, s);
+    s.thr = march_thr(m, s.scan, s.thr0);
+    if (m.wide) s.thr *= kPi;
     thr = s.thr;
     phase = PH_MARCH;
     begin_de(s.scan);
   };
-  auto finish = [&](bool found) {
+  // the ray's end; at: its last estimate
+  auto finish = [&](bool found, double at) {
 #pragma clang fp contract(off)
     if (Src == kHand && ambiguous) {
       // marched again from the start (kRedo)
-      b.redo_list[atomicAdd(&b.counters[CNT_REDO], 1ull)] = r;
+      redo_list.append(r);
+      appended = true;
       redo++;
       state = MS_NEED;
       return;
     }
     MarchOut o;
-    o.point = start + dir * s.scan;
-    if (!found) o.point = s.point;  // the last estimate's
+    o.point = start + dir * at;
     o.scan = s.scan;
     o.distThresh = thr;
     o.dist = found ? dist : s.dist;
@@ -605,6 +674,8 @@ __device__ __forceinline__ void march64_body(const DevScene *__restrict__ scp, B
     o.found = found;
     o.missed = false;
     write_ray(b, r, o);
+    if (found) hit_list.append(r);
+    appended |= found;
     hits += found;
     missed += found && below;
     state = MS_NEED;
@@ -698,11 +769,11 @@ __device__ __forceinline__ void march64_body(const DevScene *__restrict__ scp, B
             }
           }
           if constexpr (Src == kHand) {
-            s.i = b.hand_i[mine];
-            s.scan = b.hand_scan[mine];
-            s.step = b.hand_step[mine];
-            s.drift = b.hand_drift[mine];
-            s.dist = b.hand_dist[mine];
+            s.i = b.hand_i[r];
+            s.scan = b.hand_scan[r];
+            s.step = b.hand_step[r];
+            s.drift = b.hand_drift[r];
+            s.dist = b.hand_dist[r];
             margin = 4.0 * sqrt(s.drift);  // s.drift: variance of the FP32 scan deviation
             prev_dist = s.dist;
             prev_scan = s.scan - s.step;  // the step before s.i
@@ -764,16 +835,17 @@ __device__ __forceinline__ void march64_body(const DevScene *__restrict__ scp, B
           const double jf = m.jitter ? jitter_factor(jitter_draw(ray_hash, (uint32_t)s.i)) : 1.0;
           const double old_step = s.step;
           s.step = (dist - m.below * s.thr) * m.DE_factor * jf;
-          ray_records<RT>(b, r, stats).put(s.i, old_step, raw, s.thr, obj_it >> 3);
+          ray_records<RT>(b, r).put(s.i, old_step, raw, s.thr, obj_it >> 3, ovf);
           if constexpr (Src == kHand) {
             prev_dist = dist;
             prev_scan = s.scan;
             have_prev = true;
           }
+          const double at = s.scan;
           s.scan += s.step;
           s.dist = dist;
           s.i++;
-          if (s.scan > m.far || s.i >= 10000) finish(false);
+          if (s.scan > m.far || s.i >= 10000) finish(false, at);
           else begin_march();
         }
       } else if (phase == PH_SEARCH) {
@@ -804,10 +876,18 @@ __device__ __forceinline__ void march64_body(const DevScene *__restrict__ scp, B
         settled = refine();
       }
       if (found) settled = hit_refine && !m.constant_thresh ? refine() : true;
-      if (settled) finish(true);
+      if (settled) finish(true, s.scan);
+    }
+    if (__ballot(appended)) {
+      hit_list.flush(b.hit_list, &b.counters[CNT_HITS], false);
+      if constexpr (Src == kHand) redo_list.flush(b.redo_list, &b.counters[CNT_REDO], false);
+      appended = false;
     }
   }
+  hit_list.flush(b.hit_list, &b.counters[CNT_HITS], true);
+  if constexpr (Src == kHand) redo_list.flush(b.redo_list, &b.counters[CNT_REDO], true);
   unsigned long long v[ST_COUNT] = {0};
+  add_ovf(v, ovf);
   v[ST_MARCH_DE] = cnt.de_calls;
   v[ST_MARCH_ITERS] = cnt.iterations;
   v[ST_HITS] = hits;
@@ -817,7 +897,7 @@ __device__ __forceinline__ void march64_body(const DevScene *__restrict__ scp, B
 }
 
 template <class RT, int F, int Plain, int IP, int Src>
-__global__ void __launch_bounds__(kBlock, Plain && (F != 2 || IP) ? 4 : 1)
+__global__ void __launch_bounds__(kBlock, !Plain ? 1 : F == 2 && !IP ? 2 : 4)
     k_march64(const DevScene *__restrict__ scp, BandBufs b, int band_first, int band_rays,
               unsigned long long *stats) {
   march64_body<RT, F, Plain, IP, Src>(scp, b, band_first, band_rays, stats);

@@ -20,11 +20,11 @@ enum StatIdx {
 
 // Band counters (BandBufs::counters), zeroed on the device at band start:
 // hits appended, rays handed to the FP64 continuation, primary-ray queue,
-// overflow runs handed out, AO work queue, rays listed for the FP64 redo,
-// overflow chunks, the queues over the handed-over and the redo rays and over
+// overflow pool hand-out (directories x 2^32 + chunks), AO work queue, rays
+// listed for the FP64 redo, the queues over the handed-over and the redo rays and over
 // the hits' shadow rays, normals, colours and fast AO.
 enum CounterIdx {
-  CNT_HITS = 0, CNT_HAND = 1, CNT_RAYQ = 2, CNT_DIRS = 3, CNT_AOQ = 4, CNT_REDO = 5, CNT_CHUNKS = 6,
+  CNT_HITS = 0, CNT_HAND = 1, CNT_RAYQ = 2, CNT_POOL = 3, CNT_AOQ = 4, CNT_REDO = 5,
   CNT_HANDQ = 7, CNT_REDOQ = 8, CNT_SHADOWQ = 9, CNT_NORMALQ = 10, CNT_COLOURQ = 11, CNT_FASTQ = 12,
   CNT_COUNT = 16
 };
@@ -65,7 +65,8 @@ struct BandBufs {
   // compaction lists: hits, rays to re-march in FP64
   int *hit_list, *redo_list;
   unsigned long long *counters;          // CNT_* below
-  // rays handed from the march to its FP64 continuation
+  // rays handed from the FP32 march to its FP64 continuation: their list, and
+  // per ray the step it stopped at
   int *hand_ray, *hand_i;
   double *hand_scan, *hand_step, *hand_drift, *hand_dist;
   // overflow pool: ovf_dirs directories of kDirSlots chunk indices,
