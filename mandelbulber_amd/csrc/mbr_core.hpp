@@ -42,6 +42,16 @@ struct Math<double> {
   static MBR_HD double pow(double x, double y) { return ::pow(x, y); }
   static MBR_HD double cos(double x) { return ::cos(x); }
   static MBR_HD double sin(double x) { return ::sin(x); }
+  // one argument reduction for both; the device library's sincos gives the bits
+  // of its sin and cos
+  static MBR_HD void sincos(double x, double &s, double &c) {
+#if defined(__HIP_DEVICE_COMPILE__)
+    ::sincos(x, &s, &c);
+#else
+    s = ::sin(x);
+    c = ::cos(x);
+#endif
+  }
   static MBR_HD double log(double x) { return ::log(x); }
   static MBR_HD double fabs(double x) { return ::fabs(x); }
   static MBR_HD double copysign(double a, double b) { return ::copysign(a, b); }
@@ -57,6 +67,10 @@ struct Math<float> {
   static MBR_HD float pow(float x, float y) { return ::powf(x, y); }
   static MBR_HD float cos(float x) { return ::cosf(x); }
   static MBR_HD float sin(float x) { return ::sinf(x); }
+  static MBR_HD void sincos(float x, float &s, float &c) {
+    s = sin(x);
+    c = cos(x);
+  }
   static MBR_HD float log(float x) { return ::logf(x); }
   static MBR_HD float fabs(float x) { return ::fabsf(x); }
   static MBR_HD float copysign(float a, float b) { return ::copysignf(a, b); }
