@@ -33,11 +33,11 @@
 // 16-bit rounding for the background.  Pixels whose depth or normal is
 // ill-conditioned (grazing hits, degenerate normals) are left out.
 #include "mbr_kernels.hpp"
+#include "mbr_lanes.hpp"
 #include "mbr_shade.hpp"
 
 namespace mbr {
 
-constexpr int kAdjBlock = 256;
 constexpr int kParams = 9;
 constexpr double kTangentMax = 1e5;
 // residual of a refined hit, relative to its threshold, below which it
@@ -49,102 +49,81 @@ struct G4 {
   double v, g[4];
 };
 
-__device__ __forceinline__ G4 gc(double v) { return G4{v, {0, 0, 0, 0}}; }
-__device__ __forceinline__ G4 operator+(const G4 &a, const G4 &b) {
-  return G4{a.v + b.v, {a.g[0] + b.g[0], a.g[1] + b.g[1], a.g[2] + b.g[2], a.g[3] + b.g[3]}};
-}
-__device__ __forceinline__ G4 operator-(const G4 &a, const G4 &b) {
-  return G4{a.v - b.v, {a.g[0] - b.g[0], a.g[1] - b.g[1], a.g[2] - b.g[2], a.g[3] - b.g[3]}};
-}
-__device__ __forceinline__ G4 operator*(const G4 &a, const G4 &b) {
-  G4 r;
-  r.v = a.v * b.v;
-  for (int i = 0; i < 4; i++) r.g[i] = a.g[i] * b.v + a.v * b.g[i];
-  return r;
-}
-__device__ __forceinline__ G4 operator*(const G4 &a, double s) {
-  return G4{a.v * s, {a.g[0] * s, a.g[1] * s, a.g[2] * s, a.g[3] * s}};
-}
-__device__ __forceinline__ G4 operator/(const G4 &a, const G4 &b) {
-  G4 r;
-  r.v = a.v / b.v;
-  const double ib = 1.0 / b.v;
-  for (int i = 0; i < 4; i++) r.g[i] = (a.g[i] - r.v * b.g[i]) * ib;
-  return r;
-}
-// f(a) with f' = fp at a.v
-__device__ __forceinline__ G4 chain(const G4 &a, double fv, double fp) {
-  return G4{fv, {a.g[0] * fp, a.g[1] * fp, a.g[2] * fp, a.g[3] * fp}};
-}
-__device__ __forceinline__ G4 gsqrt(const G4 &a) {
-  const double s = sqrt(a.v);
-  return chain(a, s, s > 0 ? 0.5 / s : 0.0);
-}
-__device__ __forceinline__ G4 gasin(const G4 &a) { return chain(a, asin(a.v), 1.0 / sqrt(1.0 - a.v * a.v)); }
-__device__ __forceinline__ G4 gcos(const G4 &a) { return chain(a, cos(a.v), -sin(a.v)); }
-__device__ __forceinline__ G4 gsin(const G4 &a) { return chain(a, sin(a.v), cos(a.v)); }
-__device__ __forceinline__ G4 glog(const G4 &a) { return chain(a, log(a.v), 1.0 / a.v); }
-__device__ __forceinline__ G4 gatan2(const G4 &y, const G4 &x) {
-  G4 r;
-  r.v = atan2(y.v, x.v);
-  const double den = x.v * x.v + y.v * y.v;
-  const double ix = den > 0 ? x.v / den : 0.0, iy = den > 0 ? y.v / den : 0.0;
-  for (int i = 0; i < 4; i++) r.g[i] = ix * y.g[i] - iy * x.g[i];
-  return r;
-}
-// a^e for a > 0 with both a and e carrying gradients
-__device__ __forceinline__ G4 gpow(const G4 &a, const G4 &e) {
-  G4 r;
-  r.v = pow(a.v, e.v);
-  const double la = log(a.v), da = e.v * r.v / a.v;
-  for (int i = 0; i < 4; i++) r.g[i] = da * a.g[i] + r.v * la * e.g[i];
-  return r;
-}
-
-struct G4V {
-  G4 x, y, z;
-};
-
 // CalculateDistance of the trig_optim Mandelbulb (src/fractal.cpp:211-225,
 // :1151-1157, :1245-1306 for the analytic branch without interior mode,
 // iteration threshold, primitives or limits) with its gradient in (point,
-// power); the branches follow the values, as in the forward.
-__device__ G4 de_grad(const FractalK<double> &f, const V3<double> &p, double power, double detail, int N, int minN) {
-  G4V z = {G4{p.x, {1, 0, 0, 0}}, G4{p.y, {0, 1, 0, 0}}, G4{p.z, {0, 0, 1, 0}}};
-  const G4 pw = G4{power, {0, 0, 0, 1}};
-  const G4 pm1 = pw - gc(1.0);
-  G4V c;
-  if (f.julia_mode) {
-    c = {gc(f.julia[0]), gc(f.julia[1]), gc(f.julia[2])};
-  } else {
-    c = {z.x * f.constant_factor, z.y * f.constant_factor, z.z * f.constant_factor};
-  }
-  G4 r = gsqrt(z.x * z.x + z.y * z.y + z.z * z.z);
-  G4 aux = gc(1.0);
-  G4 dist = gc(0.0);
-  int L = 0;
-  bool esc = false;
-  for (; L < N; L++) {
-    const G4 th0 = gasin(z.z / r);
-    const G4 ph0 = gatan2(z.y, z.x);
-    G4 rp = gpow(r, pm1);
-    const G4 th = th0 * pw, ph = ph0 * pw;
-    const G4 cth = gcos(th);
-    aux = rp * aux * pw + gc(1.0);
-    rp = rp * r;
-    z = {cth * gcos(ph) * rp + c.x, cth * gsin(ph) * rp + c.y, gsin(th) * rp + c.z};
-    r = gsqrt(z.x * z.x + z.y * z.y + z.z * z.z);
-    if (!(r.v <= f.bailout)) {
-      dist = r * glog(r) * 0.5 / aux;
-      esc = true;
-      break;
+// power), as a resumable state; the branches follow the values, as in the
+// forward.  An iteration forms its transcendentals once and carries the four
+// tangent columns of the orbit and of its derivative through their slopes.
+struct GradDE {
+  V3<double> z, c, dz[4];
+  double r, aux, dr[4], daux[4];
+  int L;
+
+  __device__ __forceinline__ void begin(const FractalK<double> &f, V3<double> p) {
+    z = p;
+    c = f.julia_mode ? v3<double>(f.julia[0], f.julia[1], f.julia[2]) : p * f.constant_factor;
+    r = length(z);
+    aux = 1.0;
+    L = 0;
+    for (int i = 0; i < 4; i++) {
+      dz[i] = v3<double>(i == 0, i == 1, i == 2);
+      dr[i] = r > 0 ? dot(z, dz[i]) / r : 0.0;
+      daux[i] = 0.0;
     }
   }
-  if (!esc) dist = gc(0.0);
-  if (dist.v < 0) dist = gc(0.0);
-  if (L < minN && dist.v < detail) dist = gc(detail);
-  return dist;
-}
+  // one iteration; true when the orbit escaped (L < N) or N is reached
+  __device__ __forceinline__ bool step(const FractalK<double> &f, double power, int N) {
+    const double u = z.z / r, th0 = asin(u), ph0 = atan2(z.y, z.x);
+    const double rp = radius_power(f, r), lr = log(r);
+    double sth, cth, sph, cph;
+    sincos(th0 * power, &sth, &cth);
+    sincos(ph0 * power, &sph, &cph);
+    const double dasin = 1.0 / sqrt(1.0 - u * u), ir = 1.0 / r;
+    const double den = z.x * z.x + z.y * z.y;
+    const double ix = den > 0 ? z.x / den : 0.0, iy = den > 0 ? z.y / den : 0.0;
+    const double drp = (power - 1.0) * rp * ir;  // d rp / dr
+    const double R = rp * r;
+    const double k = f.julia_mode ? 0.0 : f.constant_factor;
+    const V3<double> e = v3<double>(cth * cph, cth * sph, sth);
+    const V3<double> zn = e * R + c;
+    const double rn = length(zn), irn = rn > 0 ? 1.0 / rn : 0.0;
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+      const double dp = i == 3 ? 1.0 : 0.0;
+      const double du = (dz[i].z - u * dr[i]) * ir;
+      const double dth = du * dasin * power + th0 * dp;
+      const double dph = (ix * dz[i].y - iy * dz[i].x) * power + ph0 * dp;
+      const double dr1 = drp * dr[i] + rp * lr * dp;
+      daux[i] = (dr1 * aux + rp * daux[i]) * power + rp * aux * dp;
+      const double dR = dr1 * r + rp * dr[i];
+      const V3<double> dn =
+          v3<double>(R * (-sth * cph * dth - e.y * dph) + e.x * dR + (i == 0 ? k : 0.0),
+                     R * (-sth * sph * dth + e.x * dph) + e.y * dR + (i == 1 ? k : 0.0),
+                     R * (cth * dth) + sth * dR + (i == 2 ? k : 0.0));
+      dz[i] = dn;
+      dr[i] = dot(zn, dn) * irn;
+    }
+    aux = rp * aux * power + 1.0;
+    z = zn;
+    r = rn;
+    if (!(r <= f.bailout)) return true;
+    L++;
+    return L >= N;
+  }
+  __device__ __forceinline__ G4 end(double detail, int N, int minN) const {
+    G4 d = {0.0, {0, 0, 0, 0}};
+    if (L < N) {
+      const double lr = log(r);
+      d.v = r * lr * 0.5 / aux;
+      const double ia = 1.0 / aux;
+      for (int i = 0; i < 4; i++) d.g[i] = ((lr + 1.0) * dr[i] * 0.5 - d.v * daux[i]) * ia;
+    }
+    if (d.v < 0) d = G4{0.0, {0, 0, 0, 0}};
+    if (L < minN && d.v < detail) d = G4{detail, {0, 0, 0, 0}};
+    return d;
+  }
+};
 
 // Rotation Rz(a) Rx(b) Ry(g) and its derivatives in a, b, g (row-major).
 __device__ void rot3(double a, double b, double g, double R[9], double dR[3][9]) {
@@ -177,14 +156,97 @@ __device__ __forceinline__ V3<double> dnormalize(const V3<double> &v, const V3<d
   return (dv - u * dot(u, dv)) * (1.0 / l);
 }
 
-template <class RT>
-__global__ void __launch_bounds__(kAdjBlock) k_adjoint(const DevScene *__restrict__ scp, BandBufs b, int band_first,
-                                                       int band_rays, AdjParams P, const float *__restrict__ gR,
-                                                       const float *__restrict__ gG, const float *__restrict__ gB,
-                                                       double *grad, uint8_t *skipped, float *__restrict__ jac) {
+// The estimates with gradients of the band's hits, in planes over the band's
+// rays: value and four slopes of estimate j at [(5 j + i) cap + r], j = 0 at the
+// hit (the implicit equation), 1..4 the normal's stencil.
+__device__ __forceinline__ G4 load_g4(const double *g4, long long cap, int j, int r) {
+  const double *q = g4 + 5 * j * cap + r;
+  return G4{q[0], {q[cap], q[2 * cap], q[3 * cap], q[4 * cap]}};
+}
+
+// Whether the hit's depth has a derivative here.  It is well conditioned where
+// the ray meets the level set D = c0 thr going down it: Ft = dF/dt < 0 with a
+// margin.  Near a grazing tangency Ft -> 0 and dt/dtheta diverges: the refined
+// hit then sits next to a fold of t(theta), where the forward jumps for a small
+// change of theta.  The implicit-function derivative holds at a root of F;
+// where the distance estimate jumps across the binary search's band (its
+// spherical coordinates are singular on the z axis and its preimages) the
+// refinement stops short of a root, and the depth then follows the Newton
+// iterates instead.  Both kinds of hits are left out (and flagged).
+__device__ __forceinline__ bool has_root(const G4 &D, const V3<double> &d, double thr, double c0, double kthr,
+                                         double &Ft) {
+  const V3<double> gD = v3<double>(D.g[0], D.g[1], D.g[2]);
+  Ft = dot(gD, d) - c0 * kthr;
+  return Ft < -0.05 * length(gD) * length(d) && fabs(D.v - c0 * thr) <= kRootTol * thr;
+}
+
+// The hits' estimates, one per lane and item (mbr_lanes.hpp); Stencil: the
+// normal's, of the hits that have a root.  Five estimates after one another per
+// lane, the stencil's with 5 N iterations, left a 512x512 image waiting for the
+// few lanes whose orbits never escape (7.5 ms of 256-register kernel).
+template <bool Stencil>
+__global__ void __launch_bounds__(kBlock, 2)
+    k_adjoint_de(const DevScene *__restrict__ scp, BandBufs b, int band_first, AdjParams P,
+                 const float *__restrict__ gR, const float *__restrict__ gG, const float *__restrict__ gB, bool all,
+                 double *__restrict__ g4) {
+  const DevScene &sc = *scp;
+  const FractalK<double> f = sc.fd;
+  const ShadeK<double> &k = sc.sd;
+  const double kthr = k.resolution * k.persp / k.quality, c0 = 1.0 - 0.005 * k.quality;
+  const long long n_items = (long long)b.counters[CNT_HITS] * (Stencil ? 4 : 1);
+  const int N = Stencil ? sc.N * 5 : sc.N, minN = Stencil ? 0 : sc.minN;
+  const int lanes = item_lanes(n_items);
+  WaveQueue queue(&b.counters[Stencil ? CNT_NORMALQ : CNT_SHADOWQ], n_items, lanes);
+  const int lane = __lane_id();
+  int state = lane < lanes ? MS_NEED : MS_EXHAUSTED;
+  int r = 0, j = 0;
+  double thr = 0;
+  GradDE de;
+  lane_loop<2>(
+      state,
+      [&](int rank, int n_need) {
+        int stop;
+        const long long mine = queue.take<false>(b, rank, n_need, 0, stop);
+        if (state != MS_NEED) return;
+        if (mine < 0) {
+          state = MS_EXHAUSTED;
+          return;
+        }
+        r = b.hit_list[Stencil ? mine >> 2 : mine];
+        j = Stencil ? 1 + (int)(mine & 3) : 0;
+        const int p = band_first + r;
+        if (!all && gR[p] == 0.0f && gG[p] == 0.0f && gB[p] == 0.0f) return;
+        thr = b.thr[r];
+        V3<double> q = v3<double>(b.px[r], b.py[r], b.pz[r]);
+        if constexpr (Stencil) {
+          V3<double> d;
+          view_vector(sc, p % sc.width, p / sc.width, d);
+          double Ft;
+          if (!has_root(load_g4(g4, b.cap, 0, r), d, thr, c0, kthr, Ft)) return;
+          const double delta = thr * k.quality * k.smoothness;
+          q = q + v3<double>(j == 2 ? delta : 0.0, j == 3 ? delta : 0.0, j == 4 ? delta : 0.0);
+        }
+        de.begin(f, q);
+        state = MS_ITER;
+      },
+      [&]() { return de.step(f, P.power, N); },
+      [&]() {
+        const G4 D = de.end(thr, N, minN);
+        double *o = g4 + 5 * j * (long long)b.cap + r;
+        o[0] = D.v;
+        for (int i = 0; i < 4; i++) o[(i + 1) * (long long)b.cap] = D.g[i];
+        state = MS_NEED;
+      });
+}
+
+// Per pixel: the nine tangents of its colour, contracted with the image adjoint.
+__global__ void __launch_bounds__(kBlock) k_adjoint(const DevScene *__restrict__ scp, BandBufs b, int band_first,
+                                                    int band_rays, AdjParams P, const float *__restrict__ gR,
+                                                    const float *__restrict__ gG, const float *__restrict__ gB,
+                                                    double *grad, uint8_t *skipped, float *__restrict__ jac,
+                                                    const double *__restrict__ g4) {
   const DevScene &sc = *scp;
   const ShadeK<double> &k = sc.sd;
-  const FractalK<double> &f = sc.fd;
   double acc[kParams];
   for (int i = 0; i < kParams; i++) acc[i] = 0;
   double R[9], dR[3][9];
@@ -207,8 +269,8 @@ __global__ void __launch_bounds__(kAdjBlock) k_adjoint(const DevScene *__restric
   const double c0 = 1.0 - 0.005 * k.quality;
   const double mlR = k.main_light[0], mlG = k.main_light[1], mlB = k.main_light[2];
 
-  for (long long rr = (long long)blockIdx.x * kAdjBlock + threadIdx.x; rr < band_rays;
-       rr += (long long)gridDim.x * kAdjBlock) {
+  for (long long rr = (long long)blockIdx.x * kBlock + threadIdx.x; rr < band_rays;
+       rr += (long long)gridDim.x * kBlock) {
     const int r = (int)rr;
     const int p = band_first + r;
     const int x = p % sc.width, y = p / sc.width;
@@ -252,21 +314,10 @@ __global__ void __launch_bounds__(kAdjBlock) k_adjoint(const DevScene *__restric
       const V3<double> ph = v3<double>(b.px[r], b.py[r], b.pz[r]);  // the forward's hit point
       const double thr = b.thr[r];
       // the implicit hit
-      const G4 D = de_grad(f, ph, P.power, thr, sc.N, sc.minN);
+      const G4 D = load_g4(g4, b.cap, 0, r);
       const V3<double> gD = v3<double>(D.g[0], D.g[1], D.g[2]);
-      const double Ft = dot(gD, d) - c0 * kthr;
-      // The depth is well conditioned where the ray meets the level set
-      // D = c0 thr going down it: Ft < 0 with a margin.  Near a grazing
-      // tangency Ft -> 0 and dt/dtheta diverges: the refined hit then sits
-      // next to a fold of t(theta), where the forward jumps for a small
-      // change of theta; such pixels are left out (and flagged).
-      // The implicit-function derivative holds at a root of F.  Where the
-      // distance estimate jumps across the binary search's band (its
-      // spherical coordinates are singular on the z axis and its preimages)
-      // the refinement stops short of a root, and the depth then follows
-      // the Newton iterates instead: such hits are left out (and flagged).
-      const bool at_root = fabs(D.v - c0 * thr) <= kRootTol * thr;
-      if (!(Ft < -0.05 * length(gD) * length(d)) || !at_root) {
+      double Ft;
+      if (!has_root(D, d, thr, c0, kthr, Ft)) {
         if (skipped) skipped[p] = 1;
         continue;
       }
@@ -279,12 +330,8 @@ __global__ void __launch_bounds__(kAdjBlock) k_adjoint(const DevScene *__restric
         dp[i] = dO[i] + dd[i] * t + d * dt[i];
       }
       // normal: forward differences of D at N x 5, minN 0
-      const double delta = thr * k.quality * k.smoothness;
-      const int N5 = sc.N * 5;
-      const G4 s1 = de_grad(f, ph, P.power, thr, N5, 0);
-      const G4 s2 = de_grad(f, ph + v3<double>(delta, 0, 0), P.power, thr, N5, 0);
-      const G4 s3 = de_grad(f, ph + v3<double>(0, delta, 0), P.power, thr, N5, 0);
-      const G4 s4 = de_grad(f, ph + v3<double>(0, 0, delta), P.power, thr, N5, 0);
+      const G4 s1 = load_g4(g4, b.cap, 1, r), s2 = load_g4(g4, b.cap, 2, r), s3 = load_g4(g4, b.cap, 3, r),
+               s4 = load_g4(g4, b.cap, 4, r);
       const V3<double> nr = v3<double>(s2.v - s1.v, s3.v - s1.v, s4.v - s1.v);
       const bool zero_n = nr.x == 0 && nr.y == 0 && nr.z == 0;
       const V3<double> n = zero_n ? v3<double>(1, 0, 0) : normalize(nr);
@@ -298,14 +345,19 @@ __global__ void __launch_bounds__(kAdjBlock) k_adjoint(const DevScene *__restric
       const bool spec_live = nh > 0 && s2v < 15.0;
       // colour: the palette index is an integer (derivative zero); the
       // forward's colour, recomputed at the same point
-      ShaderIn<double> in;
-      in.point = ph;
-      in.point64 = ph;
-      in.detail = thr;
-      in.object = b.object[r];
-      LaneCount cnt = {0, 0};
-      const RGBT<double> colour = surface_colour<double>(sc, in, cnt);
-      const double col[3] = {colour.R, colour.G, colour.B};
+      double col[3] = {1.0, 1.0, 1.0};
+      if (sc.coloring) {
+        ShaderIn<double> in;
+        in.point = ph;
+        in.point64 = ph;
+        in.detail = thr;
+        in.object = b.object[r];
+        LaneCount cnt = {0, 0};
+        const RGBT<double> colour = surface_colour<double, false, false, 2>(sc, in, cnt);
+        col[0] = colour.R;
+        col[1] = colour.G;
+        col[2] = colour.B;
+      }
       for (int i = 0; i < kParams; i++) {
         const double ddelta = k.quality * k.smoothness * kthr * dt[i];
         const V3<double> q = dp[i];
@@ -344,7 +396,7 @@ __global__ void __launch_bounds__(kAdjBlock) k_adjoint(const DevScene *__restric
     for (int i = 0; i < kParams; i++) acc[i] += aR * dC[0][i] + aG * dC[1][i] + aB * dC[2][i];
   }
   // block reduction, one atomic per parameter and workgroup
-  __shared__ double red[kParams][kAdjBlock / 64];
+  __shared__ double red[kParams][kBlock / 64];
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   for (int i = 0; i < kParams; i++) {
     double v = acc[i];
@@ -354,7 +406,7 @@ __global__ void __launch_bounds__(kAdjBlock) k_adjoint(const DevScene *__restric
   __syncthreads();
   if (grad && threadIdx.x < kParams) {
     double v = 0;
-    for (int w = 0; w < kAdjBlock / 64; w++) v += red[threadIdx.x][w];
+    for (int w = 0; w < kBlock / 64; w++) v += red[threadIdx.x][w];
     atomicAdd(&grad[threadIdx.x], v);
   }
 }
@@ -363,12 +415,13 @@ hipError_t launch_adjoint(const DevScene *sc, const BandBufs &b, int band_first,
                           const float *gR, const float *gG, const float *gB, double *grad, uint8_t *skipped,
                           float *jac, int blocks, hipStream_t s) {
   if (band_rays <= 0) return hipSuccess;
-  if (b.rec_bytes == 8)
-    hipLaunchKernelGGL((k_adjoint<double>), dim3(std::max(1, blocks)), dim3(kAdjBlock), 0, s, sc, b, band_first,
-                       band_rays, p, gR, gG, gB, grad, skipped, jac);
-  else
-    hipLaunchKernelGGL((k_adjoint<float>), dim3(std::max(1, blocks)), dim3(kAdjBlock), 0, s, sc, b, band_first,
-                       band_rays, p, gR, gG, gB, grad, skipped, jac);
+  if (b.rec_bytes != 8 || b.slab < 25) return hipErrorInvalidValue;
+  // the march's step records are not read any more: their planes hold the estimates
+  double *g4 = (double *)b.rec_step;
+  launch_resident<k_adjoint_de<false>>(blocks, s, sc, b, band_first, p, gR, gG, gB, jac != nullptr, g4);
+  launch_resident<k_adjoint_de<true>>(blocks, s, sc, b, band_first, p, gR, gG, gB, jac != nullptr, g4);
+  hipLaunchKernelGGL(k_adjoint, dim3(std::max(1, std::min(blocks, (band_rays + kBlock - 1) / kBlock))), dim3(kBlock), 0,
+                     s, sc, b, band_first, band_rays, p, gR, gG, gB, grad, skipped, jac, g4);
   return hipGetLastError();
 }
 

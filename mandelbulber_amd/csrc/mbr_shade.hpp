@@ -384,6 +384,10 @@ MBR_HD RGBT<T> surface_colour(const DevScene &sc, const ShaderIn<T> &in, LaneCou
   const int *pc;
   switch (in.object) {
     case OBJ_FRACTAL: {
+      if (!sc.coloring) {  // white, whatever the orbit
+        cnt.de_calls += 1;
+        return RGBT<T>{T(1), T(1), T(1)};
+      }
       int L;
       const int N10 = sc.N * 10;
       T cval;
@@ -396,14 +400,12 @@ MBR_HD RGBT<T> surface_colour(const DevScene &sc, const ShaderIn<T> &in, LaneCou
       cnt.iterations += (uint32_t)((L < N10) ? L + 1 : N10);
       int nrCol = x86_d2i(floor((double)cval));
       nrCol = x86_abs(nrCol) % (248 * 256);
-      int colour[3] = {256, 256, 256};
-      if (sc.coloring) {
-        const ShadeK<T> &k = sc.shade<T>();
-        int color_number;
-        if (nrCol >= 248 * 256) color_number = nrCol;
-        else color_number = x86_d2i((double)(T(nrCol) * k.coloring_speed + T(256) * k.palette_offset)) % 65536;
-        index_to_colour(color_number, sc.palette, colour);
-      }
+      int colour[3];
+      const ShadeK<T> &k = sc.shade<T>();
+      int color_number;
+      if (nrCol >= 248 * 256) color_number = nrCol;
+      else color_number = x86_d2i((double)(T(nrCol) * k.coloring_speed + T(256) * k.palette_offset)) % 65536;
+      index_to_colour(color_number, sc.palette, colour);
       out.R = T(colour[0]) / T(256); out.G = T(colour[1]) / T(256); out.B = T(colour[2]) / T(256);
       return out;
     }
