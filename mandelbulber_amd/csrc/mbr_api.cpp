@@ -1816,6 +1816,8 @@ int mbr_post_ssao(mbr_ctx *c, const mbr_scene *s, const mbr_post_planes *pl, int
   p.aspect = (double)w / h;
   p.fov = s->persp;
   p.intensity = s->global_ilum;
+  p.inv_w = 1.0 / w;
+  p.inv_h = 1.0 / h;
   p.cs = c->d_ssao_tab;
   p.sn = c->d_ssao_tab + q;
   if (on_device) {

@@ -180,6 +180,7 @@ hipError_t launch_refl_finish(const DevScene *sc, const BandBufs *levels, int n_
 struct SsaoParams {
   int width, height, quality, type;  // type: enum mbr_perspective
   double scale, aspect, fov, intensity;
+  double inv_w, inv_h;  // 1 / width, 1 / height
   const double *cs, *sn;
 };
 hipError_t launch_ssao(const SsaoParams &p, const float *z, const uint16_t *opacity, const uint8_t *const colour[3],

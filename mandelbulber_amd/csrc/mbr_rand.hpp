@@ -39,6 +39,17 @@ class GlibcRand {
     b_ = (b_ + 1) % 31;
     return out;
   }
+  // The next kBlock outputs (a multiple of 31, so the ring ends where it began).
+  static constexpr int kBlock = 31 * 64;
+  void block(uint32_t *out) {
+    uint32_t w[31 + kBlock];  // the ring from its oldest word on, then its successors
+    for (int k = 0; k < 31; k++) w[k] = (uint32_t)r_[(f_ + k) % 31];
+    for (int k = 31; k < 31 + kBlock; k++) {
+      w[k] = w[k - 31] + w[k - 3];
+      out[k - 31] = (w[k] >> 1) & 0x7fffffffu;
+    }
+    for (int k = 0; k < 31; k++) r_[(f_ + k) % 31] = (int32_t)w[kBlock + k];
+  }
 
  private:
   int32_t r_[31];
