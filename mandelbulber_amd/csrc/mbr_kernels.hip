@@ -1942,7 +1942,7 @@ __device__ __forceinline__ void finish_body(const DevScene &sc, const BandBufs &
       for (int i = 0; i < n; i++) sum += (double)st[(long long)i * cap + r];
       vray.scan_end = sum;
     }
-    v = volumetric<T>(sc, depth, n, px, alpha, rec, vr, vis, fx);
+    v = volumetric<FX || VIS ? 1 : 4>(sc, depth, n, px, alpha, rec, vr, vis, fx);
   } else {
     // records from the slab on sit in the chunks the ray's directory lists
     // (the host renders a band again when a record found the pool full)
@@ -1970,7 +1970,7 @@ __device__ __forceinline__ void finish_body(const DevScene &sc, const BandBufs &
       }
       vray.scan_end = sum;
     }
-    v = volumetric<T>(sc, depth, n, px, alpha, rec, vr, vis, fx);
+    v = volumetric<FX || VIS ? 1 : 4>(sc, depth, n, px, alpha, rec, vr, vis, fx);
   }
   if (out.rgb[0]) out.rgb[0][p] = (float)v.rgb.R;
   if (out.rgb[1]) out.rgb[1][p] = (float)v.rgb.G;
@@ -2150,7 +2150,7 @@ __global__ void __launch_bounds__(kBlock) k_refl_finish(const DevScene *__restri
         (void)stage; (void)index; (void)p64; (void)thr; (void)step; (void)o; (void)totalOpacity;
       }
     };
-    const VolOut<double> v = volumetric<double>(sc, depth, n, px, alpha, rec, vr, vis, fx);
+    const VolOut<double> v = volumetric<FX || VIS ? 1 : 4>(sc, depth, n, px, alpha, rec, vr, vis, fx);
     result = v.rgb;
     if (ray == 0) {
       opacity0 = v.opacity;

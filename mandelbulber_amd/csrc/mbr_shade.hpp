@@ -635,8 +635,14 @@ struct NoFx {
 // `fx(stage, index, point, threshold, step, out, totalOpacity)` adds the
 // volumetric lights (stage 0, before the fogs) and the iteration fog
 // (stage 1, after them).
-template <class T, class RecFn, class FxFn = NoFx>
-MBR_HD VolOut<T> volumetric(const DevScene &sc, T depth, int stepCount, RGBT<T> px, T alpha, RecFn rec,
+//
+// Records are read by their index, not by their distance from the ray's end:
+// the lanes of a wave then read one row of the step-major planes together,
+// where each from its own last record on they read up to 64 rows at a time
+// (2.8 times the records' bytes fetched on the 1080p power-8 bulb).  Batch
+// records are read before they are used, one latency for all of them.
+template <int Batch, class T, class RecFn, class FxFn = NoFx>
+__device__ __forceinline__ VolOut<T> volumetric(const DevScene &sc, T depth, int stepCount, RGBT<T> px, T alpha, RecFn rec,
                             const VisRay *vr = nullptr, bool vis = false, FxFn fx = NoFx{}) {
   const ShadeK<T> &k = sc.shade<T>();
   VolOut<T> o;
@@ -652,13 +658,11 @@ MBR_HD VolOut<T> volumetric(const DevScene &sc, T depth, int stepCount, RGBT<T> 
   const T glowB = (T(sc.glow1[2]) * glowN + T(sc.glow2[2]) * glow) / T(65536);
   T totalStep = 0;
   double scan = vr ? vr->scan_end : 0.0;
-  for (int index = stepCount - 1; index > 0; index--) {
-    T step, distance, dist_thresh;
-    rec(index, step, distance, dist_thresh);
+  auto record = [&](int index, T step, T distance, T dist_thresh) {
     const double scan_i = scan;  // scan of this record's point
     scan -= (double)step;
     totalStep += step;
-    if (totalStep < dist_thresh * k.quality) continue;
+    if (totalStep < dist_thresh * k.quality) return;
     step = totalStep;
     totalStep = 0;
 
@@ -714,6 +718,21 @@ MBR_HD VolOut<T> volumetric(const DevScene &sc, T depth, int stepCount, RGBT<T> 
     if (totalOpacity > 1.0f) totalOpacity = 1.0f;
     if (o.alpha > T(1)) o.alpha = 1;
     o.opacity = T(totalOpacity);
+  };
+  // the most steps of the wave's rays
+  int most = 0;
+  for (int bit = 1 << 13; bit; bit >>= 1)
+    if (__any(stepCount >= most + bit)) most += bit;
+  for (int top = most - 1; top > 0; top -= Batch) {
+    T step[Batch], distance[Batch], thr[Batch];
+#pragma unroll
+    for (int u = 0; u < Batch; u++) {
+      step[u] = distance[u] = thr[u] = 0;
+      if (top - u > 0 && top - u < stepCount) rec(top - u, step[u], distance[u], thr[u]);
+    }
+#pragma unroll
+    for (int u = 0; u < Batch; u++)
+      if (top - u > 0 && top - u < stepCount) record(top - u, step[u], distance[u], thr[u]);
   }
   return o;
 }
