@@ -1219,6 +1219,7 @@ ShadeBufs frame_shade_bufs(Slot &sl, const DevScene &host, int formula, bool tri
   sbuf.fast_ao_on = host.ao && host.fast_ao;
   sbuf.shadow_fx = host.shadow && host.shadow_fx;
   sbuf.deep = host.deep;
+  sbuf.slow_normals = host.slow_shading;
   sbuf.plain = host.plain;
   sbuf.formula = formula;
   sbuf.lights = host.n_lights > 0 || host.fake_lights;
@@ -1332,6 +1333,7 @@ ShadeBufs shade_bufs(Slot &sl, const DevScene &host, int formula) {
   sbuf.fast_ao_on = host.ao && host.fast_ao;
   sbuf.shadow_fx = host.shadow && host.shadow_fx;
   sbuf.deep = 0;
+  sbuf.slow_normals = host.slow_shading;
   sbuf.plain = host.plain;
   sbuf.formula = formula;
   sbuf.lights = host.n_lights > 0 || host.fake_lights;

@@ -26,6 +26,10 @@ MBR_HD bool formula_analytic(int formula) {
   return formula == 1 || formula == 2 || formula == 7 || formula == 8 || formula == 10 || formula == 17 ||
          formula == 18 || formula == 37;
 }
+// Of these, trig_DE and the kaleidoscopic IFS have kernels of their own (F = 1,
+// 10) for plain scenes; like the generic path their FP32 modes march in FP64
+// and take the normals from FP64 estimates.
+MBR_HD constexpr bool formula_march64(int formula) { return formula == 1 || formula == 10; }
 // termination groups of src/fractal.cpp:1133-1149: Menger-like (r > 1000,
 // (r - 2) / DE) and Mandelbox-like (r > 1024, r / |DE|)
 MBR_HD bool formula_menger_group(int formula) { return formula == 7 || formula == 10; }
@@ -87,7 +91,10 @@ MBR_HD int hybrid_slot(const FractalK<T> &f, int L) {
 template <class T>
 MBR_HD V3<T> angle_vector(T alfa, T beta) {
   using M = Math<T>;
-  return V3<T>{M::cos(beta) * M::cos(alfa), M::cos(beta) * M::sin(alfa), M::sin(beta)};
+  T sa, ca, sb, cb;
+  M::sincos(alfa, sa, ca);
+  M::sincos(beta, sb, cb);
+  return V3<T>{cb * ca, cb * sa, sb};
 }
 
 // m = m * R_axis(angle) (CRotationMatrix::RotateX/Y/Z, src/algebra.cpp:94-143;
@@ -193,7 +200,7 @@ MBR_HD T compute(const FractalK<T> &f, V3<T> z, int N, int *iter_count) {
       // IFS folding mode (src/fractal.cpp:101-127): the kaleidoscopic
       // vectors fold z without their intensities or edges; the scenes that
       // turn it on run the generic kernels
-      if (f.ifs_fold) {
+      if (!P && f.ifs_fold) {
         if (f.ifs_abs[0]) z.x = M::fabs(z.x);
         if (f.ifs_abs[1]) z.y = M::fabs(z.y);
         if (f.ifs_abs[2]) z.z = M::fabs(z.z);
@@ -814,6 +821,7 @@ struct DEIter {
   V3<T> z, c;
   T r, aux;  // aux: r_dz (trig formulas) or tgladDE (folding formulas)
   T inv_r;   // 1/r, kept by the FP32 integer-power Mandelbulb path
+  T th_dz, ph_dz;  // trig_DE: the angles of its derivative vector
   int L;
 };
 
@@ -824,8 +832,9 @@ template <class T, int F, int P = 0, bool A = (sizeof(T) < 8), int IP = 0>
 MBR_HD void de_begin(const FractalK<T> &f, V3<T> p, DEIter<T> &s) {
   s.z = p;
   s.c = (!P && f.julia_mode) ? ld3(f.julia) : p * f.constant_factor;
-  s.r = length(p);
+  s.r = formula_march64(F) ? length_nc(p) : length(p);
   s.aux = 1;
+  if constexpr (F == 1) s.th_dz = s.ph_dz = 0;
   s.L = 0;
   s.inv_r = 0;
   if constexpr (F == 2 && A) {
@@ -879,6 +888,62 @@ MBR_HD float fold_root(float q) {
 #endif
 }
 
+// One iteration of trig_DE (src/fractal.cpp:189-209) or the kaleidoscopic IFS
+// (:837-886), with compute's statements; true when the orbit escaped.
+template <class T, int F>
+MBR_HD bool own_iter(const FractalK<T> &f, DEIter<T> &s) {
+#pragma clang fp contract(off)
+  using M = Math<T>;
+  V3<T> z = s.z;
+  bool esc;
+  if constexpr (F == 1) {
+    const T p = f.power;
+    const T r1 = M::pow(s.r, p - T(1));
+    const T r2 = r1 * s.r;
+    const T th = M::atan2(z.y, z.x);
+    const T ph = -M::atan2(z.z, M::sqrt(z.x * z.x + z.y * z.y));
+    const V3<T> dz = angle_vector((p - T(1)) * th + s.th_dz, (p - T(1)) * ph + s.ph_dz) * (p * r1 * s.aux) +
+                     V3<T>{T(1), T(0), T(0)};
+    s.aux = length_nc(dz);
+    s.th_dz = M::atan2(dz.y, dz.x);
+    s.ph_dz = -M::atan2(dz.z, M::sqrt(dz.x * dz.x + dz.y * dz.y));
+    z = angle_vector(p * th, p * ph) * r2 + s.c;
+    s.r = length_nc(z);
+    esc = s.r > f.bailout;
+  } else {
+    if (f.ifs_abs[0]) z.x = M::fabs(z.x);
+    if (f.ifs_abs[1]) z.y = M::fabs(z.y);
+    if (f.ifs_abs[2]) z.z = M::fabs(z.z);
+    for (int i = 0; i < 9; i++) {
+      if (!f.ifs_en[i]) continue;
+      if (f.ifs_rot_on[i]) z = mat_apply_nc(f.ifs_rot[i], z);
+      const V3<T> dirv = ld3(f.ifs_dir[i]);
+      const T len = dot_nc(z, dirv);
+      if (len < f.ifs_dist[i]) z = z - dirv * (T(2) * (len - f.ifs_dist[i]) * f.ifs_int[i]);
+    }
+    const V3<T> off = ld3(f.ifs_offset);
+    V3<T> zo = z - off;
+    if (f.ifs_main_on) zo = mat_apply_nc(f.ifs_main, zo);
+    z = zo + off;
+    if (f.ifs_edge[0] > 0) z.x = f.ifs_edge[0] - M::fabs(f.ifs_edge[0] - z.x);
+    if (f.ifs_edge[1] > 0) z.y = f.ifs_edge[1] - M::fabs(f.ifs_edge[1] - z.y);
+    if (f.ifs_edge[2] > 0) z.z = f.ifs_edge[2] - M::fabs(f.ifs_edge[2] - z.z);
+    z = z * f.ifs_scale;
+    const T sm1 = f.ifs_scale - T(1);
+    if (f.ifs_menger) {
+      z.x -= off.x * sm1;
+      z.y -= off.y * sm1;
+      if (z.z > T(0.5) * off.z * sm1) z.z -= off.z * sm1;
+    } else {
+      z = z - off * sm1;
+    }
+    s.aux *= f.ifs_scale;
+    esc = beyond<1000>(dot_nc(z, z));
+  }
+  s.z = z;
+  return esc;
+}
+
 // One loop pass.  Returns true when the call has finished: the orbit escaped
 // (s.L < N, the reference's iteration counter) or stayed bounded for N
 // iterations (s.L == N).  The distance is left to de_escape_distance, so that
@@ -887,6 +952,12 @@ MBR_HD float fold_root(float q) {
 template <class T, int F, int P = 0, bool A = (sizeof(T) < 8), int IP = 0>
 MBR_HD bool de_iter(const FractalK<T> &f, DEIter<T> &s, int N) {
   using M = Math<T>;
+  if constexpr (formula_march64(F)) {
+    static_assert(P != kOptions, "plain scenes only");
+    if (own_iter<T, F>(f, s)) return true;
+    s.L++;
+    return s.L >= N;
+  }
   V3<T> z = s.z;
   T r = s.r;
   if ((!P && f.tglad_fold)) {
@@ -1086,6 +1157,7 @@ MBR_HD bool de_iter(const FractalK<T> &f, DEIter<T> &s, int N) {
 template <class T, int F, bool A = (sizeof(T) < 8), int IP = 0>
 MBR_HD T de_escape_distance(const FractalK<T> &f, const DEIter<T> &s) {
   using M = Math<T>;
+  if constexpr (F == 10) return (length_nc(s.z) - T(2)) / s.aux;
   if constexpr (F == 7) return fdiv(length(s.z) - T(2), s.aux);
   if constexpr (F == 8) return fdiv(length(s.z), M::fabs(s.aux));
   if constexpr (F == 2 && A) {

@@ -126,6 +126,7 @@ struct ShadeBufs {
   long long n;                  // hit capacity (plane stride)
   int slow_ao;                  // 1: run the AmbientOcclusion rays
   int deep;                     // 1: FP32 shading starts distance estimates in FP64 where needed
+  int slow_normals;             // the 11^3 normal stencil (slowShading)
   int plain;                    // 1: no primitives, limits, interior, iteration threshold, pre-folds, Julia
   int formula;
   int lights;                   // 1: aux lights take part (k_aux runs after k_surface)

@@ -51,3 +51,37 @@ def test_shaded_hits_match_oracle(renderer, kind, w, h, keys):
     assert_planes_exact(m)
     fix, _ = renderer.render(precision=_abi.PREC_FP32_FIXUP)
     assert_parity(compare(fix, ref), label="fixup")
+
+
+@pytest.mark.parametrize("keys", [{"slow_shading": 1, "N": 20}, dict(SOFT, **FAST), {"iter_fog_enabled": 1}])
+@pytest.mark.parametrize("formula", [1, 10])
+def test_trig_de_and_ifs_hits_match_oracle(renderer, formula, keys):
+    """trig_DE and the kaleidoscopic IFS run kernels of their own in plain
+    scenes: the chained stencil (FP32 estimates, where the four-point one takes
+    FP64 ones), soft shadows with fast AO, and iteration fog (FP64 only)."""
+    from oracle import oracle
+    if formula == 1:
+        s = scene.mandelbulb_plain(31, 23)
+        s.power = 8.0
+    else:
+        s = scene.menger_view(31, 23, shaded=False)
+        s.ifs_scale, s.ifs_menger_sponge_mode = 3.0, 1
+        for i, d in enumerate([(1, -1, 0), (1, 0, -1), (0, 1, -1)]):
+            s.ifs_abs[i], s.ifs_offset[i], s.ifs_enabled[i] = 1, 1.0, 1
+            for c in range(3):
+                s.ifs_direction[i][c] = d[c]
+    s.formula = formula
+    a, b = scene.light_from_seed(5)
+    keys = dict(keys)
+    fog = keys.pop("iter_fog_enabled", 0)
+    scene.apply(s, dict(keys, main_light_alfa=a, main_light_beta=b))
+    s.iter_fog_enabled = fog
+    print(f"[hits] formula {formula} {keys} fog {fog}", flush=True)
+    ref, _ = oracle.render(s)
+    renderer.set_scene(s)
+    for prec in (_abi.PREC_FP64, _abi.PREC_FP32_FIXUP):
+        f, st = renderer.render(precision=prec)
+        m = compare(f, ref)
+        print(f"  {st.hits} hits {m}", flush=True)
+        assert st.hits > 0
+        assert_parity(m, label=f"precision {prec}")
