@@ -629,6 +629,17 @@ int band_cap(int precision, int ao_count) {
   return (int)std::min<size_t>((size_t)kBandRays, std::max<size_t>(4096, kAOBudget / per_ray));
 }
 
+// Values per hit that the fast AO keeps in the slot's AO buffer (its estimates;
+// none from quality 9 on, whose chains the kernel sums by itself: 80 values
+// per hit and more).
+int fast_ao_values(const DevScene &h) {
+  return h.ao && h.fast_ao && h.ao_quality >= 2 && h.ao_quality <= 8 ? h.ao_quality * h.ao_quality - 1 : 0;
+}
+int fast_ao_items(const Slot &sl, const DevScene &h) {
+  const int v = fast_ao_values(h);
+  return (size_t)sl.band.cap * (size_t)v * sl.band.rec_bytes <= sl.sh_ao_bytes ? v : 0;
+}
+
 int kernel_family(const mbr_scene &s) { return s.ifs_folding_mode ? kGenericFamily : s.formula; }
 
 // The precision a scene renders in.  The generic formulas run in FP64,
@@ -1217,6 +1228,7 @@ ShadeBufs frame_shade_bufs(Slot &sl, const DevScene &host, int formula, bool tri
   sbuf.slow_ao = host.ao && !host.fast_ao;
   sbuf.env = host.env_map;
   sbuf.fast_ao_on = host.ao && host.fast_ao;
+  sbuf.fast_items = fast_ao_items(sl, host);
   sbuf.shadow_fx = host.shadow && host.shadow_fx;
   sbuf.deep = host.deep;
   sbuf.slow_normals = host.slow_shading;
@@ -1331,6 +1343,7 @@ ShadeBufs shade_bufs(Slot &sl, const DevScene &host, int formula) {
   sbuf.slow_ao = host.ao && !host.fast_ao;
   sbuf.env = host.env_map;
   sbuf.fast_ao_on = host.ao && host.fast_ao;
+  sbuf.fast_items = fast_ao_items(sl, host);
   sbuf.shadow_fx = host.shadow && host.shadow_fx;
   sbuf.deep = 0;
   sbuf.slow_normals = host.slow_shading;
@@ -1491,8 +1504,9 @@ int mbr_render_device(mbr_ctx *c, const mbr_render_opts *opts, mbr_framebuffer *
   HIPCHECK(c, hipSetDevice(c->device));
   const bool slow_ao = c->host_sc.ao && !c->host_sc.fast_ao;
   const int ao_count = slow_ao ? c->host_sc.ao_count : 0;
+  const int ao_values = std::max(ao_count, fast_ao_values(c->host_sc));
   Slot &sl = c->slots[0];
-  rc = alloc_slot(c, sl, precision, band_cap(precision, ao_count), ao_count, c->host_sc.iter_fog != 0);
+  rc = alloc_slot(c, sl, precision, band_cap(precision, ao_count), ao_values, c->host_sc.iter_fog != 0);
   if (rc != MBR_OK) return rc;
   // reflection levels: a slot each after the first
   const int refl = c->host_sc.refl_max;
@@ -1504,7 +1518,7 @@ int mbr_render_device(mbr_ctx *c, const mbr_render_opts *opts, mbr_framebuffer *
     if (rc != MBR_OK) return rc;
     for (int k = 0; k < refl; k++) {
       Slot &lk = c->refl_slots[(size_t)k];
-      rc = alloc_slot(c, lk, precision, sl.band.cap, ao_count, c->host_sc.iter_fog != 0);
+      rc = alloc_slot(c, lk, precision, sl.band.cap, ao_values, c->host_sc.iter_fog != 0);
       if (rc == MBR_OK) rc = alloc_refl(c, lk, true);
       if (rc != MBR_OK) return rc;
       levels.push_back(&lk);
@@ -1519,7 +1533,7 @@ int mbr_render_device(mbr_ctx *c, const mbr_render_opts *opts, mbr_framebuffer *
   Slot *pair[2] = {&sl, &c->slots[1]};
   int n_bands = (int)((last - first + sl.band.cap - 1) / sl.band.cap);
   if (split) {
-    rc = alloc_slot(c, c->slots[1], precision, sl.band.cap, ao_count, c->host_sc.iter_fog != 0);
+    rc = alloc_slot(c, c->slots[1], precision, sl.band.cap, ao_values, c->host_sc.iter_fog != 0);
     if (rc != MBR_OK) return rc;
     if (!c->side[1]) HIPCHECK(c, hipStreamCreateWithFlags(&c->side[1], hipStreamNonBlocking));
     if (!c->split_fork) HIPCHECK(c, hipEventCreateWithFlags(&c->split_fork, hipEventDisableTiming));
@@ -2124,7 +2138,7 @@ int mbr_render_batch(mbr_ctx *c, const mbr_scene *scenes, int n, const mbr_textu
   // derive every scene on the host
   std::vector<BatchFrame> frames(n);
   long long ao_total = 0;
-  int max_ao = 0;
+  int max_ao = 0, max_fast = 0;
   for (int i = 0; i < n; i++) {
     rc = prepare_scene(c, &scenes[i], lightmap, frames[i].p);
     if (rc != MBR_OK) return c->fail(rc, "scene " + std::to_string(i) + ": " + c->err);
@@ -2141,6 +2155,7 @@ int mbr_render_batch(mbr_ctx *c, const mbr_scene *scenes, int n, const mbr_textu
     ao_total += frames[i].p.d.ao_count;
     const DevScene &d = frames[i].p.d;
     if (d.ao && !d.fast_ao) max_ao = std::max(max_ao, d.ao_count);
+    max_fast = std::max(max_fast, fast_ao_values(d));
   }
   // upload scene blocks and AO tables
   if (n > c->batch_sc_cap) {
@@ -2197,7 +2212,7 @@ int mbr_render_batch(mbr_ctx *c, const mbr_scene *scenes, int n, const mbr_textu
     return c->fail(MBR_ERR_INVALID_ARG, "slots must be 1..4 and blocks_per_cu 1..32");
   const int n_slots = cands.empty() ? slots : kMaxSlots;
   for (int k = 0; k < n_slots; k++) {
-    rc = alloc_slot(c, c->slots[k], precision, cap, max_ao);
+    rc = alloc_slot(c, c->slots[k], precision, cap, std::max(max_ao, max_fast));
     if (rc != MBR_OK) return rc;
   }
   mbr_batch_result res;

@@ -132,6 +132,7 @@ struct ShadeBufs {
   int lights;                   // 1: aux lights take part (k_aux runs after k_surface)
   int ip8;                      // 1: Mandelbulb of power 8 (kernels with the power fixed)
   int fast_ao_on;               // 1: FastAmbientOcclusion2 instead of the AmbientOcclusion rays
+  int fast_items;               // its estimates per hit when ao has room for them, else 0
   int env;                      // 1: environment mapping
   int shadow_fx;                // 1: shadow marches take their thresholds from the distance to the eye
 };

@@ -85,3 +85,25 @@ def test_trig_de_and_ifs_hits_match_oracle(renderer, formula, keys):
         print(f"  {st.hits} hits {m}", flush=True)
         assert st.hits > 0
         assert_parity(m, label=f"precision {prec}")
+
+
+@pytest.mark.parametrize("w,h", [(3, 2), (67, 41)])
+@pytest.mark.parametrize("quality", [1, 2, 8, 9])
+def test_fast_ao_items_match_oracle(renderer, quality, w, h):
+    """FastAmbientOcclusion2 without estimates (quality 1), as items (2 to 8) and
+    as chains (from 9 on), in frames of a few and of several waves' hits."""
+    from oracle import oracle
+    s = scene.menger_view(w, h, shaded=False)
+    a, b = scene.light_from_seed(5)
+    scene.apply(s, {"ambient_occlusion_enabled": 1, "fast_ambient_occlusion_mode": 1,
+                    "ambient_occlusion_quality": quality, "main_light_alfa": a, "main_light_beta": b})
+    print(f"[hits] fast AO quality {quality} {w}x{h}", flush=True)
+    ref, _ = oracle.render(s)
+    renderer.set_scene(s)
+    f64, st = renderer.render(precision=_abi.PREC_FP64)
+    m = compare(f64, ref)
+    print(f"  {st.hits} hits {m}", flush=True)
+    assert st.hits > 0 and m["flips"] == 0 and m["depth_rel_max"] <= 1e-12 and m["psnr_db"] >= 120, m
+    assert_planes_exact(m)
+    fix, _ = renderer.render(precision=_abi.PREC_FP32_FIXUP)
+    assert_parity(compare(fix, ref), label="fixup")
