@@ -320,6 +320,15 @@ __device__ __forceinline__ RecPlanes<RT> ray_records(const BandBufs &b, int r) {
   return rec;
 }
 
+// Whether a kernel of formula F keeps a copy of the scene's formula constants.
+// The plain variants read a few of them in every iteration, and the stores and
+// atomics of the loops keep the compiler from hoisting loads of the scene block:
+// a local copy keeps them in registers.  Not where the scene may rotate (the
+// Mandelbox's 13 matrices) or fold nine times (the kaleidoscopic IFS): their
+// copies are spilled and read back lane by lane, which cost 1.9 times the time
+// of the rotated Mandelbox's FP64 AO (480x320, 8.0 and 15.2 ms).
+constexpr bool local_scene(int F, int P) { return P && F != 10 && !(F == 8 && P == kPlain); }
+
 // Persistent march: one primary ray per lane, up to kMarchIters formula
 // iterations per pass, lane states and amortised bookkeeping as in k_ao.
 #ifndef MBR_MARCH_ITERS
@@ -337,8 +346,9 @@ __device__ __forceinline__ void march_body(const DevScene *__restrict__ scp, Ban
   // records are FP32; the FP64 mode keeps the trigonometric form
   constexpr bool kAlg = sizeof(RT) < 8 || IP != 0;
   const DevScene &sc = *scp;
-  const FractalK<T> f_local = Plain ? sc.frac<T>() : FractalK<T>{};
-  const FractalK<T> &f = Plain ? f_local : sc.frac<T>();  // see march64_body
+  constexpr bool kLocal = local_scene(F, Plain);
+  const FractalK<T> f_local = kLocal ? sc.frac<T>() : FractalK<T>{};
+  const FractalK<T> &f = kLocal ? f_local : sc.frac<T>();
   const int N = sc.N, minN = sc.minN;
   const int lane = __lane_id();
   const unsigned long long lt_mask = (lane == 0) ? 0ull : (~0ull >> (64 - lane));
@@ -497,11 +507,7 @@ __device__ __forceinline__ void march64_body(const DevScene *__restrict__ scp, B
   // records are FP32; the FP64 mode keeps the trigonometric form
   constexpr bool kAlg = sizeof(RT) < 8 || IP != 0;
   const DevScene &sc = *scp;
-  // the plain variants read a few formula constants in every iteration: a
-  // local copy keeps them in registers (the pass's stores and atomics keep
-  // the compiler from hoisting loads of the scene block out of the loop), but
-  // not the nine folds of the kaleidoscopic IFS (F = 10)
-  constexpr bool kLocal = Plain && F != 10;
+  constexpr bool kLocal = local_scene(F, Plain);
   const FractalK<double> f_local = kLocal ? sc.fd : FractalK<double>{};
   const FractalK<double> &f = kLocal ? f_local : sc.fd;
   const MarchK m = march_k(sc);
@@ -543,6 +549,12 @@ __device__ __forceinline__ void march64_body(const DevScene *__restrict__ scp, B
   auto begin_de = [&](double t) {
 #pragma clang fp contract(off)
     const V3<double> p = start + dir * t;
+    if constexpr (F == 0) {  // whole estimates: one call for all lanes, in the pass
+      call.p = p;
+      early = true;
+      state = MS_ITER;
+      return;
+    }
     DEInfo info;
     early = de_call_begin<double, F, Plain, kAlg, IP>(f, p, s.thr, N, minN, false, call, dist, info);
     state = early ? MS_DONE : MS_ITER;
@@ -647,7 +659,7 @@ __device__ __forceinline__ void march64_body(const DevScene *__restrict__ scp, B
     if (!(m_need | m_iter | m_done)) break;
     const int n_need = __popcll(m_need), n_iter = __popcll(m_iter), n_done = __popcll(m_done);
 
-    if (n_need && (4 * n_need >= n_need + n_iter + n_done || n_iter + n_done == 0)) {
+    if (n_need && (F == 0 || 4 * n_need >= n_need + n_iter + n_done || n_iter + n_done == 0)) {
       int stop = 0;
       const long long mine = q.take<Src == kRays>(b, __popcll(m_need & lt_mask), n_need, 12, stop);
       if (state == MS_NEED) {
@@ -701,9 +713,16 @@ __device__ __forceinline__ void march64_body(const DevScene *__restrict__ scp, B
     }
 
     if (state == MS_ITER) {
-      bool fin = false;
+      bool fin = F == 0;
+      if constexpr (F == 0) {
+        DEInfo info;
+        dist = calc_distance_generic<double, Plain>(f, call.p, s.thr, N, minN, false, info);
+        early_obj = info.object | (info.iters << 3);
+        cnt.iterations += (uint32_t)info.work;
+      } else {
 #pragma unroll
-      for (int it = 0; it < kMarchIters && !fin; it++) fin = de_call_step<double, F, Plain, kAlg, IP>(f, call, N);
+        for (int it = 0; it < kMarchIters && !fin; it++) fin = de_call_step<double, F, Plain, kAlg, IP>(f, call, N);
+      }
       if (fin) state = MS_DONE;
     }
 
@@ -1033,10 +1052,10 @@ template <class T, int F, bool Deep, int P, int IP>
 __global__ void __launch_bounds__(kBlock, (HitPolicy<T, F, Deep, P>::waves))
     k_hits(const DevScene *__restrict__ scp, BandBufs b, SurfBufs<T> sb, int kinds, unsigned long long *stats) {
   const DevScene &sc = *scp;
-  constexpr bool kLocal = P && F != 10;  // see march64_body
+  constexpr bool kLocal = local_scene(F, P);
   const FractalK<T> f_local = kLocal ? sc.frac<T>() : FractalK<T>{};
   const FractalK<T> &f = kLocal ? f_local : sc.frac<T>();
-  constexpr bool kLocal64 = P && (Deep || F == 1) && sizeof(T) < 8;
+  constexpr bool kLocal64 = kLocal && (Deep || F == 1) && sizeof(T) < 8;
   const FractalK<double> fd_local = kLocal64 ? sc.fd : FractalK<double>{};
   const FractalK<double> &fd = kLocal64 ? fd_local : sc.fd;
   const ShadeK<T> &k = sc.shade<T>();
@@ -1341,10 +1360,10 @@ template <class T, int F, bool Deep, int P, int IP>
 __global__ void __launch_bounds__(kBlock, (HitPolicy<T, F, Deep, P>::waves))
     k_fast_ao(const DevScene *__restrict__ scp, BandBufs b, SurfBufs<T> sb, unsigned long long *stats) {
   const DevScene &sc = *scp;
-  constexpr bool kLocal = P && F != 10;  // see march64_body
+  constexpr bool kLocal = local_scene(F, P);
   const FractalK<T> f_local = kLocal ? sc.frac<T>() : FractalK<T>{};
   const FractalK<T> &f = kLocal ? f_local : sc.frac<T>();
-  constexpr bool kLocal64 = P && (Deep || F == 1) && sizeof(T) < 8;
+  constexpr bool kLocal64 = kLocal && (Deep || F == 1) && sizeof(T) < 8;
   const FractalK<double> fd_local = kLocal64 ? sc.fd : FractalK<double>{};
   const FractalK<double> &fd = kLocal64 ? fd_local : sc.fd;
   const ShadeK<T> &k = sc.shade<T>();
@@ -1534,7 +1553,7 @@ __device__ __forceinline__ void ao_body(const DevScene *__restrict__ scp, BandBu
   // trig-free integer-power iteration in FP32, and in FP64 for the fixed power
   constexpr bool kAlg = sizeof(T) < 8 || IP != 0;
   const long long n_hits = (long long)b.counters[CNT_HITS];
-  constexpr bool kLocal = Plain && F != 10;  // see march64_body
+  constexpr bool kLocal = local_scene(F, Plain);
   const FractalK<T> f_local = kLocal ? sc.frac<T>() : FractalK<T>{};
   const FractalK<T> &f = kLocal ? f_local : sc.frac<T>();
   const ShadeK<T> &k = sc.shade<T>();
