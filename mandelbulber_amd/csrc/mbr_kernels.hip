@@ -1081,13 +1081,13 @@ __global__ void __launch_bounds__(kBlock, (HitPolicy<T, F, Deep, P>::waves))
     int guard = 0, early_it = 0;
     bool early = false;
     HitDE<T, F, Deep, P, IP> call;
-    auto finish = [&]() {
+    auto finish = [&]() __attribute__((always_inline)) {
       sb.spec[n + tid] = soft ? (T(1) - maxSoft) : shadowTemp;
       sb.fast_ao[tid] = thr;  // the detail size MainShadow leaves, for the AO
       state = MS_NEED;
     };
     // the estimate at distance i, or the ray's end
-    auto next = [&]() {
+    auto next = [&]() __attribute__((always_inline)) {
       if (!(i < factor && guard < kMaxShadeSteps)) {
         finish();
         return;
@@ -1174,12 +1174,12 @@ __global__ void __launch_bounds__(kBlock, (HitPolicy<T, F, Deep, P>::waves))
     T delta = 0, detail = 0, dist = 0;
     bool early = false;
     HitDE<T, F, Deep, P, IP> call;
-    auto begin = [&](V3<T> off) {
+    auto begin = [&](V3<T> off) __attribute__((always_inline)) {
       DEInfo info;
       early = call.begin(fd, f, point, point64, off, detail, N5, minN, true, dist, info);
       state = early ? MS_DONE : MS_ITER;
     };
-    auto stencil = [&]() {
+    auto stencil = [&]() __attribute__((always_inline)) {
       p2 = v3<T>((T)px, (T)py, (T)pz);
       begin(p2 * delta);
     };
@@ -1385,7 +1385,7 @@ __global__ void __launch_bounds__(kBlock, (HitPolicy<T, F, Deep, P>::waves))
   int i = 0;
   bool early = false;
   HitDE<T, F, Deep, P, IP> call;
-  auto next = [&]() {
+  auto next = [&]() __attribute__((always_inline)) {
     if (!split && i >= end) {
       T ao = T(1) - T(0.2) * aoTemp;
       if (ao < 0) ao = 0;
