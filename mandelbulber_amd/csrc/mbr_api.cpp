@@ -5,8 +5,8 @@
 // (src/interface.cpp:688-730, src/callbacks.cpp:1538-1555) into the device
 // scene block, after the parameter clamps of CheckPrameters
 // (src/interface.cpp:3587-3602).  mbr_render[_device] runs the frame as
-// bands of at most kBandRays rays: reset -> march -> FP64 continuation ->
-// shade over compacted hits -> finish, all enqueued on one stream with the
+// bands of at most kBandRays rays: reset -> march (FP32_MARCH: and its FP64
+// continuation) -> shade over compacted hits -> finish, all enqueued on one stream with the
 // work counts passed between launches in device memory; the host waits once
 // per frame.
 #include <hip/hip_runtime.h>
@@ -1240,7 +1240,7 @@ ShadeBufs frame_shade_bufs(Slot &sl, const DevScene &host, int formula, bool tri
 }
 
 // One band, rays [band_first, band_first + band_rays), through the buffers
-// of slot sl on stream st: reset -> march -> FP64 continuation -> shade ->
+// of slot sl on stream st: reset -> march (and its continuation) -> shade ->
 // finish.  With e (6 events) the launches are bracketed for timing.
 int enqueue_band(mbr_ctx *c, Slot &sl, const ShadeBufs &sbuf, int precision, const DevScene *d_sc,
                  const DevScene &host, int formula, AODev ao, long long band_first, int band_rays, const FrameOut &out,
@@ -1294,11 +1294,11 @@ int enqueue_frame(mbr_ctx *c, Slot &sl, int precision, const DevScene *d_sc, con
 // rays, or its continuation, surface and composition kernels leave the
 // vector units idle, the other band's kernels fill the CUs.  Each band's
 // results depend only on its own rays, so the frame equals the one-stream
-// frame bit for bit.  Measured on the 1080p power-8 bulb (MI355X): two
-// bands 13.5 ms against 14.4 ms on one stream; four or more bands, a
-// staggered start of the second stream and smaller march or AO grids were
-// all slower.  FP64 frames stay on one stream (two FP64 bands at once took
-// 133-143 ms against 127 ms).
+// frame bit for bit.  Measured on the 1080p power-8 bulb (MI355X) with the
+// kernels of that time: two bands 13.5 ms against 14.4 ms on one stream; four
+// or more bands, a staggered start of the second stream and smaller march or
+// AO grids were all slower.  FP64 frames stay on one stream (two FP64 bands at
+// once took 133-143 ms against 127 ms).
 constexpr long long kSplitRays = 1 << 18;
 constexpr int kSplitBands = 2;
 

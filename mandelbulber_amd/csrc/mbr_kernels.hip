@@ -1,16 +1,18 @@
 // mbr_kernels.hip — gfx950 kernels of the render core.
 //
-// One frame (or band of rows) runs as three launches:
-//   k_march   one lane per primary ray: DE-stepped march with step
-//             records, then the binary-search refinement in FP64
-//             (RayMarching, src/Render3D.cpp:79-199); hits are appended to a
-//             compacted hit list so shading runs on full waves of hits.
-//   k_shade   one lane per hit: normals, hard/soft shadow, specular, palette
-//             colour, ambient occlusion (ObjectShader, src/shaders.cpp:21).
-//   k_finish  one lane per ray: background for misses, VolumetricShader
-//             (glow, fog, volumetric fog) over the step record read back to
-//             front, and coalesced writes of the framebuffer planes
-//             (src/Render3D.cpp:530-589).
+// One frame (or band of rows) runs as these launches:
+//   k_march64   one lane per primary ray: DE-stepped march with step records,
+//               then the binary-search refinement, in FP64 (RayMarching,
+//               src/Render3D.cpp:79-199); hits are appended to a compacted hit
+//               list so shading runs on full waves of hits.  FP32_MARCH: k_march
+//               in FP32 first, then k_march64 over the rays it handed over.
+//   k_hits      shadow rays, normals and colours of the hits (ObjectShader,
+//               src/shaders.cpp:21); k_fast_ao or k_ao their ambient occlusion,
+//               k_compose the sums.
+//   k_finish    one lane per ray: background for misses, VolumetricShader
+//               (glow, fog, volumetric fog) over the step record read back to
+//               front, and coalesced writes of the framebuffer planes
+//               (src/Render3D.cpp:530-589).
 #include <type_traits>
 
 #include "mbr_kernels.hpp"
@@ -125,19 +127,14 @@ __device__ __forceinline__ void flush_stats(unsigned long long *stats, const uns
 }
 
 // ----------------------------------------------------------------- march
-// RayMarching (src/Render3D.cpp:79-199) is split around its distance
-// estimates.  march_before_de sets up step i (point, threshold);
+// The FP32 march (k_march) splits RayMarching (src/Render3D.cpp:79-199) around
+// its distance estimates.  march_before_de sets up step i (point, threshold);
 // march_after_de takes step i's distance and either continues, ends the ray
-// as a miss, or hands the ray over to the FP64 continuation.  The persistent
-// kernel k_march advances many rays this way, one formula iteration per
-// pass; the FP64 redo of k_march_fix runs the same functions sequentially,
-// so both produce identical records.
+// as a miss, or hands the ray over to the FP64 continuation (k_march64).
 //
-// Hand-over rule.  The FP64 path hands a ray over when step i is a hit; the
-// continuation repeats step i in FP64 and runs the binary search.  The FP32
-// path hands a ray over when step i's FP32 distance could be a hit once FP32
-// error is allowed for: below 1.001 x threshold, or within the drift margin
-// of it.
+// Hand-over rule.  A ray is handed over when step i's FP32 distance could be
+// a hit once FP32 error is allowed for: below 1.001 x threshold, or within the
+// drift margin of it.
 //
 // Drift model.  An FP32 distance differs from the FP64 distance at the same
 // point by about 1e-6 of the distance (rounding accumulated over the
@@ -1449,8 +1446,8 @@ __global__ void __launch_bounds__(kBlock, (HitPolicy<T, F, Deep, P>::waves))
   flush_stats(stats, v);
 }
 
-// AuxLightsShader (src/shaders.cpp:1051-1073) per hit, after k_surface: the
-// normal and detail size come from k_surface's entries in sb.aux, which are
+// AuxLightsShader (src/shaders.cpp:1051-1073) per hit, after k_hits_end: the
+// normal and detail size come from its entries in sb.aux, which are
 // replaced by the diffuse and specular sums.  A kernel of its own, so the
 // surface kernel of scenes without aux lights keeps its registers.
 template <class T, int F, bool Deep>
@@ -1654,7 +1651,7 @@ __device__ __forceinline__ void ao_body(const DevScene *__restrict__ scp, BandBu
             if constexpr (Deep) deep = (double)in.detail < 2.0 * kMixedSwitch * length(P64);
             start_dist = in.delta;
             end_dist = in.delta / k.resolution;
-            detail = sb.fast_ao[h];  // the detail size k_surface left (after MainShadow)
+            detail = sb.fast_ao[h];  // the detail size MainShadow left
             thr_f = (T)(float)in.dist_thresh;  // float dist_thresh (src/shaders.cpp:642)
           }
           item = (unsigned long long)h * count + d;

@@ -129,7 +129,7 @@ struct ShadeBufs {
   int slow_normals;             // the 11^3 normal stencil (slowShading)
   int plain;                    // 1: no primitives, limits, interior, iteration threshold, pre-folds, Julia
   int formula;
-  int lights;                   // 1: aux lights take part (k_aux runs after k_surface)
+  int lights;                   // 1: aux lights take part (k_aux runs after k_hits_end)
   int ip8;                      // 1: Mandelbulb of power 8 (kernels with the power fixed)
   int fast_ao_on;               // 1: FastAmbientOcclusion2 instead of the AmbientOcclusion rays
   int fast_items;               // its estimates per hit when ao has room for them, else 0
