@@ -1511,9 +1511,14 @@ __global__ void __launch_bounds__(kBlock) k_aux(const DevScene *__restrict__ scp
 // average).  The AO step logic of DONE lanes runs once 1/done_div of the
 // wave waits for it, the item hand-out of NEED lanes once 1/need_div does
 // (or nothing else can run), so their cost is shared by many lanes instead
-// of being paid on almost every pass.  FP32: 2 iterations, 1/3, 1/8; FP64
-// (twice the registers, 2 waves per SIMD): 1 iteration, 1/6, 1/8 (measured
-// best of the sweeps on MI355X).
+// of being paid on almost every pass.  FP32: 2 iterations, 1/3, 1/8 for the
+// Mandelbulb, whose iteration is the longest part of a pass, and 6 iterations
+// and 1/2 for the folding formulas, whose iterations are short and more per
+// estimate (1280x720 Mandelbox, AO quality 4, FP32_MARCH: AO of a band 7.47 ms
+// with 2, 6.92 with 4, 6.86 with 6, the frame 18.3 and 17.1 ms; 1001x563 Menger
+// 1.33, 1.25 and 1.22 ms, the frame 2.31 and 2.16).  FP64 (twice the registers,
+// 2 waves per SIMD): 1 iteration, 1/6, 1/8 (measured best of the sweeps on
+// MI355X).
 enum : int { AO_NEED = 0, AO_ITER = 1, AO_DONE = 2, AO_EXHAUSTED = 3 };
 // Per element type: formula iterations per pass, and the share of the wave
 // (1/div) that must wait in DONE or NEED before their block runs.
@@ -1535,11 +1540,12 @@ enum : int { AO_NEED = 0, AO_ITER = 1, AO_DONE = 2, AO_EXHAUSTED = 3 };
 #ifndef MBR_AO64_NEED_DIV
 #define MBR_AO64_NEED_DIV 8
 #endif
-template <class T>
+template <class T, int F>
 struct AOPolicy {
   static constexpr bool f64 = sizeof(T) == 8;
-  static constexpr int iters = f64 ? MBR_AO64_ITERS : MBR_AO_ITERS;
-  static constexpr int done_div = f64 ? MBR_AO64_DONE_DIV : MBR_AO_DONE_DIV;
+  static constexpr bool fold = F == 7 || F == 8;
+  static constexpr int iters = f64 ? MBR_AO64_ITERS : fold ? 6 : MBR_AO_ITERS;
+  static constexpr int done_div = f64 ? MBR_AO64_DONE_DIV : fold ? 2 : MBR_AO_DONE_DIV;
   static constexpr int need_div = f64 ? MBR_AO64_NEED_DIV : MBR_AO_NEED_DIV;
 };
 
@@ -1609,7 +1615,7 @@ __device__ __forceinline__ void ao_body(const DevScene *__restrict__ scp, BandBu
     if (!(m_need | m_iter | m_done)) break;
     const int n_need = __popcll(m_need), n_iter = __popcll(m_iter), n_done = __popcll(m_done);
 
-    if (n_need && (AOPolicy<T>::need_div * n_need >= n_need + n_iter + n_done || n_iter + n_done == 0)) {
+    if (n_need && (AOPolicy<T, F>::need_div * n_need >= n_need + n_iter + n_done || n_iter + n_done == 0)) {
       // hand out the next items to the lanes that need one, in lane order
       const unsigned n = (unsigned)n_need;
       const unsigned off = (unsigned)__popcll(m_need & lt_mask);
@@ -1667,7 +1673,7 @@ __device__ __forceinline__ void ao_body(const DevScene *__restrict__ scp, BandBu
     if (state == AO_ITER) {
       bool fin = false;
 #pragma unroll
-      for (int k = 0; k < AOPolicy<T>::iters && !fin; k++)
+      for (int k = 0; k < AOPolicy<T, F>::iters && !fin; k++)
         fin = de_call_step<T, F, Plain, kAlg, IP>(f, call, N);
       if (fin) state = AO_DONE;
     }
@@ -1675,7 +1681,7 @@ __device__ __forceinline__ void ao_body(const DevScene *__restrict__ scp, BandBu
     const unsigned long long m_done2 = __ballot(state == AO_DONE);
     const unsigned long long m_iter2 = __ballot(state == AO_ITER);
     const int n_done2 = __popcll(m_done2), n_iter2 = __popcll(m_iter2);
-    if (n_done2 && (AOPolicy<T>::done_div * n_done2 >= n_done2 + n_iter2 || n_iter2 == 0) && state == AO_DONE) {
+    if (n_done2 && (AOPolicy<T, F>::done_div * n_done2 >= n_done2 + n_iter2 || n_iter2 == 0) && state == AO_DONE) {
       cnt.de_calls += 1;
       if (!early) {
         DEInfo info;
