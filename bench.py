@@ -35,9 +35,9 @@ DIFF_KEYS = ("flip_frac", "hitmiss_px", "sheet_px", "depth_rel_max", "depth_rel_
 # HBM bytes per k_ao launch on this workload (FETCH_SIZE x 2 + WRITE_SIZE x 1,
 # the factors that make a 1 GiB device copy read 1 GiB and write 1 GiB),
 # from the rocprofv3 --pmc runs summarised in the file named here.
-AO_TRAFFIC_BYTES = 447.6e6
+AO_TRAFFIC_BYTES = 401.6e6
 AO_TRAFFIC_SOURCE = ("profiles/render_1080p_mandelbulb_pmc.txt (per launch, one of the frame's two bands: "
-                     "FETCH_SIZE 42.2 MiB x 2 + WRITE_SIZE 342.6 MiB)")
+                     "FETCH_SIZE 29.1 MiB x 2 + WRITE_SIZE 324.9 MiB)")
 
 
 def planes_on_gpu(torch, w, h):
@@ -391,7 +391,7 @@ def main():
     achieved_frame = ao_flops_frame / (ao_span * 1e-3) / 1e12
     roof = {"bound": "valu", "achieved": achieved, "peak": PEAK_TFLOPS["f32"], "unit": "TFLOP/s",
             "frac": achieved / PEAK_TFLOPS["f32"], "traffic": AO_TRAFFIC_BYTES if default_workload else None,
-            "traffic_source": AO_TRAFFIC_SOURCE if default_workload else None, "kernel": "k_ao_f32_plain<float, 2, 8>",
+            "traffic_source": AO_TRAFFIC_SOURCE if default_workload else None, "kernel": "k_ao_f32_plain<float, 2, 1, 8>",
             "flops_per_launch": ao_flops, "ms_per_launch": ao_ms,
             "launches_per_frame": launches / len(st32),
             "achieved_frame": achieved_frame, "frac_frame": achieved_frame / PEAK_TFLOPS["f32"],
