@@ -107,3 +107,20 @@ def test_fast_ao_items_match_oracle(renderer, quality, w, h):
     assert_planes_exact(m)
     fix, _ = renderer.render(precision=_abi.PREC_FP32_FIXUP)
     assert_parity(compare(fix, ref), label="fixup")
+
+
+@pytest.mark.parametrize("power", [2.0, 3.0, 7.0, 32.0, 7.5])
+def test_fp64_powers_match_oracle(renderer, power):
+    """The FP64 Mandelbulb forms r^(p - 1) by products for integer powers from
+    2 to 32 and by pow otherwise."""
+    from oracle import oracle
+    s = scene.mandelbulb_plain(41, 31)
+    s.power = power
+    print(f"[hits] power {power}", flush=True)
+    ref, _ = oracle.render(s)
+    renderer.set_scene(s)
+    f, st = renderer.render(precision=_abi.PREC_FP64)
+    m = compare(f, ref)
+    print(f"  {st.hits} hits {m}", flush=True)
+    assert st.hits > 0 and m["flips"] == 0
+    assert_parity(m, label=f"power {power}")
