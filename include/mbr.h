@@ -469,12 +469,14 @@ const char *mbr_last_error(const mbr_ctx *ctx);
 
 /* Stops the context's render in progress, from any thread: the reference
  * polls programClosed before every pixel (src/Render3D.cpp:369-378) and
- * returns.  Here the flag lives in pinned host memory that the march and AO
- * kernels read while handing out work, so a frame on the GPU stops within
- * a few hundred microseconds: rays not yet marched are left empty and AO
- * rays not yet started are skipped.  The render then returns
- * MBR_ERR_CANCELLED with an incomplete frame, and the flag is cleared.  A
- * cancel made while no render runs stops the next render at once. */
+ * returns.  Here the flag lives in pinned host memory that is read at the
+ * start of each band of rays, before its AO, and while the march and the AO
+ * rays are handed out (every 4096 rays, every 256 hits): rays not yet handed
+ * out are left empty and AO rays not yet handed out are skipped; those under
+ * way run to their end (up to 524288 rays are at once).  The
+ * render then returns MBR_ERR_CANCELLED with an incomplete frame, and the flag
+ * is cleared.  A cancel made while no render runs leaves the next render's
+ * frame empty. */
 int mbr_cancel(mbr_ctx *ctx);
 
 /* Replaces Params2Cl + CclSupport::SetParams (interface.cpp:3634,

@@ -196,7 +196,7 @@ __global__ void __launch_bounds__(kBlock, 2)
   const long long n_items = (long long)b.counters[CNT_HITS] * (Stencil ? 4 : 1);
   const int N = Stencil ? sc.N * 5 : sc.N, minN = Stencil ? 0 : sc.minN;
   const int lanes = item_lanes(n_items);
-  WaveQueue queue(&b.counters[Stencil ? CNT_NORMALQ : CNT_SHADOWQ], n_items, lanes);
+  WaveQueue<> queue(&b.counters[Stencil ? CNT_NORMALQ : CNT_SHADOWQ], n_items, lanes);
   const int lane = __lane_id();
   int state = lane < lanes ? MS_NEED : MS_EXHAUSTED;
   int r = 0, j = 0;
@@ -205,8 +205,7 @@ __global__ void __launch_bounds__(kBlock, 2)
   lane_loop<2>(
       state,
       [&](int rank, int n_need) {
-        int stop;
-        const long long mine = queue.take<false>(b, rank, n_need, 0, stop);
+        const long long mine = queue.take(b, rank, n_need);
         if (state != MS_NEED) return;
         if (mine < 0) {
           state = MS_EXHAUSTED;

@@ -332,6 +332,12 @@ constexpr bool local_scene(int F, int P) { return P && F != 10 && !(F == 8 && P 
 #define MBR_MARCH_ITERS 6
 #endif
 constexpr int kMarchIters = MBR_MARCH_ITERS;
+// hand-outs poll the cancel flag every 2^kPollRays rays of the march and every
+// 2^kPollHits hits of AO
+constexpr int kPollRays = 12, kPollHits = 8;
+// and a wave takes that many rays, or hits of that many AO directions, with one add
+constexpr int kRayRun = 128;
+constexpr unsigned kRunDirs = 2048;
 
 // IP: the integer power of the Mandelbulb when fixed at compile time (8).
 template <int F, int Plain, int IP>
@@ -355,7 +361,7 @@ __device__ __forceinline__ void march_body(const DevScene *__restrict__ scp, Ban
   __shared__ WaveListBuf hand_buf;
   WaveList hand(hand_buf);
   const int lanes = item_lanes(band_rays);
-  WaveQueue q(&b.counters[CNT_RAYQ], band_rays, lanes);
+  WaveQueue<true> q(&b.counters[CNT_RAYQ], band_rays, lanes, kRayRun, kPollRays);
   int state = lane < lanes ? MS_NEED : MS_EXHAUSTED;
   int r = 0;
   uint32_t ray_hash = 0;
@@ -385,8 +391,7 @@ __device__ __forceinline__ void march_body(const DevScene *__restrict__ scp, Ban
     const int n_need = __popcll(m_need), n_iter = __popcll(m_iter), n_done = __popcll(m_done);
 
     if (n_need && (4 * n_need >= n_need + n_iter + n_done || n_iter + n_done == 0)) {
-      int stop = 0;
-      const long long mine = q.take<true>(b, __popcll(m_need & lt_mask), n_need, 12, stop);
+      const long long mine = q.take(b, __popcll(m_need & lt_mask), n_need);
       if (state == MS_NEED) {
         if (mine < 0) {
           state = MS_EXHAUSTED;
@@ -397,7 +402,7 @@ __device__ __forceinline__ void march_body(const DevScene *__restrict__ scp, Ban
           const int x = p % sc.width, y = p / sc.width;
           // a cancelled band's remaining rays take the empty record of a
           // cut ray, so later kernels read defined (if meaningless) values
-          const bool cut = stop || view_vector(sc, x, y, dir);
+          const bool cut = q.stopped || view_vector(sc, x, y, dir);
           ray_hash = jitter_ray(sc.jitter_seed, sc.frame_no, sc.pixel_base + (uint32_t)p);
           s = ray_start_state(sc);
           if (cut) {
@@ -518,7 +523,8 @@ __device__ __forceinline__ void march64_body(const DevScene *__restrict__ scp, B
   WaveList redo_list(Src == kHand ? redo_buf : hit_buf);
   bool appended = false;
   const int lanes = item_lanes(n_items);
-  WaveQueue q(&b.counters[Src == kRays ? CNT_RAYQ : Src == kRedo ? CNT_REDOQ : CNT_HANDQ], n_items, lanes);
+  WaveQueue<Src == kRays> q(&b.counters[Src == kRays ? CNT_RAYQ : Src == kRedo ? CNT_REDOQ : CNT_HANDQ], n_items, lanes,
+                            kRayRun, kPollRays);
   const double search_limit = 1.0 - 0.01 * m.quality;
   const bool hit_refine = sc.hit_refine != 0;
   const double c0 = 1.0 - 0.005 * m.quality;
@@ -657,8 +663,7 @@ __device__ __forceinline__ void march64_body(const DevScene *__restrict__ scp, B
     const int n_need = __popcll(m_need), n_iter = __popcll(m_iter), n_done = __popcll(m_done);
 
     if (n_need && (F == 0 || 4 * n_need >= n_need + n_iter + n_done || n_iter + n_done == 0)) {
-      int stop = 0;
-      const long long mine = q.take<Src == kRays>(b, __popcll(m_need & lt_mask), n_need, 12, stop);
+      const long long mine = q.take(b, __popcll(m_need & lt_mask), n_need);
       if (state == MS_NEED) {
         if (mine < 0) {
           state = MS_EXHAUSTED;
@@ -679,7 +684,7 @@ __device__ __forceinline__ void march64_body(const DevScene *__restrict__ scp, B
             cut_ray = view_vector(sc, p % sc.width, p / sc.width, dir);
             if constexpr (Src == kRays) {
               b.ovf_off[r] = -1;
-              cut_ray = cut_ray || stop;
+              cut_ray = cut_ray || q.stopped;
             } else {
               cut_ray = false;  // the march handed it over
             }
@@ -934,6 +939,12 @@ __device__ __forceinline__ void put_lit(const DevScene &sc, const ShaderIn<T> &i
   }
 }
 
+// A cancel during the march or the surface shading stops AO before its first
+// hit (by one lane of the surface kernel, at the end of its items).
+__device__ __forceinline__ void poll_before_ao(const DevScene &sc, const BandBufs &b) {
+  if (sc.ao && !sc.fast_ao && blockIdx.x == 0 && threadIdx.x == 0) poll_cancel(b, &b.counters[CNT_AOQ]);
+}
+
 // The generic formulas' surface shading (of trig_DE and the kaleidoscopic IFS:
 // in scenes that are not plain), one lane per hit (their estimates
 // run whole, so there is nothing to interleave).
@@ -959,6 +970,7 @@ __global__ void __launch_bounds__(kBlock) k_surface_generic(const DevScene *__re
     if (sc.ao && sc.fast_ao) sb.fast_ao[tid] = fast_ao2<T, 0, false>(sc, in, cnt);
     else if (sc.ao) sb.fast_ao[tid] = in.detail;
   }
+  poll_before_ao(sc, b);
   unsigned long long v[ST_COUNT] = {0};
   v[ST_SHADE_DE] = cnt.de_calls;
   v[ST_SHADE_ITERS] = cnt.iterations;
@@ -1069,7 +1081,7 @@ __global__ void __launch_bounds__(kBlock, (HitPolicy<T, F, Deep, P>::waves))
     const int iter_fog = sc.iter_fog;
     const T soft_range = k.soft_range;
     const int lanes = item_lanes(n_hits);
-    WaveQueue queue(&b.counters[CNT_SHADOWQ], n_hits, lanes);
+    WaveQueue<> queue(&b.counters[CNT_SHADOWQ], n_hits, lanes);
     int state = lane < lanes ? MS_NEED : MS_EXHAUSTED;
     long long tid = 0;
     V3<T> point = v3<T>(0, 0, 0);
@@ -1099,8 +1111,7 @@ __global__ void __launch_bounds__(kBlock, (HitPolicy<T, F, Deep, P>::waves))
     lane_loop<kIters>(
         state,
         [&](int rank, int n_need) {
-          int stop;
-          const long long mine = queue.take<false>(b, rank, n_need, 0, stop);
+          const long long mine = queue.take(b, rank, n_need);
           if (state != MS_NEED) return;
           if (mine < 0) {
             state = MS_EXHAUSTED;
@@ -1162,7 +1173,7 @@ __global__ void __launch_bounds__(kBlock, (HitPolicy<T, F, Deep, P>::waves))
     const int N5 = sc.N * 5, slow = sc.slow_shading, minN = slow ? sc.minN : 0;
     const long long n_items = slow ? n_hits : 4 * n_hits;
     const int lanes = item_lanes(n_items);
-    WaveQueue queue(&b.counters[CNT_NORMALQ], n_items, lanes);
+    WaveQueue<> queue(&b.counters[CNT_NORMALQ], n_items, lanes);
     int state = lane < lanes ? MS_NEED : MS_EXHAUSTED;
     long long item = 0;
     V3<T> point = v3<T>(0, 0, 0), p2 = point, sum = point;
@@ -1183,8 +1194,7 @@ __global__ void __launch_bounds__(kBlock, (HitPolicy<T, F, Deep, P>::waves))
     lane_loop<kIters>(
         state,
         [&](int rank, int n_need) {
-          int stop;
-          const long long mine = queue.take<false>(b, rank, n_need, 0, stop);
+          const long long mine = queue.take(b, rank, n_need);
           if (state != MS_NEED) return;
           if (mine < 0) {
             state = MS_EXHAUSTED;
@@ -1257,10 +1267,9 @@ __global__ void __launch_bounds__(kBlock, (HitPolicy<T, F, Deep, P>::waves))
   if (kinds & HIT_COLOUR) {
     // whole orbits: their lengths differ little between neighbouring hits
     const int lanes = item_lanes(n_hits);
-    WaveQueue queue(&b.counters[CNT_COLOURQ], n_hits, lanes);
+    WaveQueue<> queue(&b.counters[CNT_COLOURQ], n_hits, lanes);
     for (;;) {
-      int stop;
-      const long long tid = queue.take<false>(b, lane < lanes ? lane : 64, lanes, 0, stop);
+      const long long tid = queue.take(b, lane < lanes ? lane : 64, lanes);
       if (!__ballot(tid >= 0)) break;
       if (tid < 0) continue;
       const int r = b.hit_list[tid];
@@ -1272,6 +1281,7 @@ __global__ void __launch_bounds__(kBlock, (HitPolicy<T, F, Deep, P>::waves))
       put_colour(b, sb, r, tid, surface_colour<T, Deep, formula_march64(F), F, P>(sc, in, cnt));
     }
   }
+  poll_before_ao(sc, b);
   unsigned long long v[ST_COUNT] = {0};
   v[ST_SHADE_DE] = cnt.de_calls;
   v[ST_SHADE_ITERS] = cnt.iterations;
@@ -1373,7 +1383,7 @@ __global__ void __launch_bounds__(kBlock, (HitPolicy<T, F, Deep, P>::waves))
   const int split = sb.fast_items;
   const long long n_items = split ? n_hits * split : n_hits;
   const int lanes = item_lanes(n_items);
-  WaveQueue queue(&b.counters[CNT_FASTQ], n_items, lanes);
+  WaveQueue<> queue(&b.counters[CNT_FASTQ], n_items, lanes);
   int state = lane < lanes ? MS_NEED : MS_EXHAUSTED;
   long long tid = 0;
   V3<T> point = v3<T>(0, 0, 0), normal = point;
@@ -1399,8 +1409,7 @@ __global__ void __launch_bounds__(kBlock, (HitPolicy<T, F, Deep, P>::waves))
   lane_loop<HitPolicy<T, F, Deep, P>::iters>(
       state,
       [&](int rank, int n_need) {
-        int stop;
-        const long long mine = queue.take<false>(b, rank, n_need, 0, stop);
+        const long long mine = queue.take(b, rank, n_need);
         if (state != MS_NEED) return;
         if (mine < 0) {
           state = MS_EXHAUSTED;
@@ -1574,7 +1583,8 @@ __device__ __forceinline__ void ao_body(const DevScene *__restrict__ scp, BandBu
   int part_bits = 0;
   while ((n_hits << (part_bits + 1)) <= waves && (count >> (part_bits + 1)) >= 16) part_bits++;
   const unsigned unit = (count + (1u << part_bits) - 1) >> part_bits;
-  WaveQueue queue(&b.counters[CNT_AOQ], n_hits << part_bits, 1);
+  WaveQueue<true> queue(&b.counters[CNT_AOQ], n_hits << part_bits, 1, unit < kRunDirs ? (int)(kRunDirs / unit) : 1,
+                        kPollHits + part_bits);
   long long wu = -1;
   unsigned wd = unit;
   int state = AO_NEED;
@@ -1629,11 +1639,10 @@ __device__ __forceinline__ void ao_body(const DevScene *__restrict__ scp, BandBu
         const bool beyond_unit = off >= avail;
         const unsigned j = beyond_unit ? off - avail : 0u;
         const unsigned q = unit >= 64 ? 0u : j / unit;  // several units only when they are small
-        int stop = 0;
-        const long long got = queue.take<true>(b, (int)q, (int)more, 8, stop);
+        const long long got = queue.take(b, (int)q, (int)more);
         if (beyond_unit) {
           // cancelled: no further hits (their AO intensities stay unwritten)
-          u = stop ? -1 : got;
+          u = queue.stopped ? -1 : got;
           d = j - q * unit;
         }
         // the last lane that takes one holds the last unit
@@ -2431,12 +2440,16 @@ hipError_t launch_march_fix(const DevScene *sc, const BandBufs &b, int band_firs
 #endif  // continuation
 
 #if MBR_UNIT(4)
-__global__ void k_band_reset(unsigned long long *counters) {
-  if (threadIdx.x < CNT_COUNT) counters[threadIdx.x] = 0;
+// Clears a band's counters; a render cancelled by now starts its band stopped.
+__global__ void k_band_reset(BandBufs b) {
+  const int i = (int)threadIdx.x;
+  if (i >= CNT_COUNT) return;
+  b.counters[i] = 0;
+  if (i == CNT_RAYQ || i == CNT_AOQ) poll_cancel(b, &b.counters[i]);
 }
 
 hipError_t launch_band_reset(const BandBufs &b, hipStream_t s) {
-  hipLaunchKernelGGL(k_band_reset, dim3(1), dim3(64), 0, s, b.counters);
+  hipLaunchKernelGGL(k_band_reset, dim3(1), dim3(64), 0, s, b);
   return hipGetLastError();
 }
 

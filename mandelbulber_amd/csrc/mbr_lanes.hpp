@@ -16,26 +16,35 @@ constexpr int kBlock = 256;
 enum : int { MS_NEED = 0, MS_ITER = 1, MS_DONE = 2, MS_EXHAUSTED = 3 };
 
 // Cancel polling (mbr_cancel, the reference's programClosed test per pixel,
-// src/Render3D.cpp:369-378).  take_work(queue, n) is the hand-out of a band
-// work queue (lane 0 only): it returns the first of n items and whether the
-// band was stopped.  A hand-out whose range crosses a multiple of
-// 2^poll_shift reads the host flag (a read over the bus, so not on every
-// hand-out); when set it adds kStopBit to the queue, so every later
-// hand-out sees the stop in the value its own atomic returns.
+// src/Render3D.cpp:369-378).  A band's work queue carries the stop in its
+// counter: kStopBit, set by whoever read the host flag (poll_cancel, a read
+// over the bus, so not for every hand-out) and found it set.
+//   k_band_reset  reads the flag before the march, the surface kernel before
+//                 AO: a wave that builds its queue sees a stop from before
+//                 its kernel, so also its fixed first items are dropped
+//   hand-outs     from the shared counter return the bit with their add; those
+//                 that cross a multiple of 2^poll_shift read the flag
+// (Hand-outs from a run taken before do not load the counter: with a load for
+// every hit a 1080p frame with AO took 13.0 ms instead of 9.3, loads and adds to
+// one address being served one after the other.  Polled queues take shorter
+// runs instead.)
 constexpr unsigned long long kStopBit = 1ull << 48;
 
-__device__ __forceinline__ unsigned long long take_work(const BandBufs &b, unsigned long long *queue,
-                                                        unsigned long long n, int poll_shift, int &stopped) {
-  unsigned long long v = atomicAdd(queue, n);
-  if (b.cancel && !(v & kStopBit)) {
-    const unsigned long long first = v & (kStopBit - 1);
-    if (((first + n) >> poll_shift) != (first >> poll_shift) && *b.cancel != 0) {
-      atomicAdd(queue, kStopBit);
-      v |= kStopBit;
-    }
-  }
-  stopped = (v & kStopBit) != 0;
-  return v & (kStopBit - 1);
+// By one lane: whether the flag is set; the queue then carries the stop.
+__device__ __forceinline__ bool poll_cancel(const BandBufs &b, unsigned long long *queue) {
+  if (!b.cancel || *b.cancel == 0) return false;
+  atomicOr(queue, kStopBit);
+  return true;
+}
+
+__device__ __forceinline__ bool crosses(long long first, long long n, int poll_shift) {
+  return ((first + n) >> poll_shift) != (first >> poll_shift);
+}
+
+// Lane 0's value, in scalar registers (what the queue keeps is the wave's).
+__device__ __forceinline__ unsigned long long first_lane(unsigned long long v) {
+  return (unsigned)__builtin_amdgcn_readfirstlane((int)v) |
+         (unsigned long long)(unsigned)__builtin_amdgcn_readfirstlane((int)(v >> 32)) << 32;
 }
 
 // Lanes of a wave that take items, for n items over the launch's waves: few
@@ -52,18 +61,26 @@ __device__ __forceinline__ int item_lanes(long long n) {
 // address pass at about 13 ns each on MI355X, whichever wave sends them: with
 // an add for every hand-out, 8192 waves spent 100 us just to find a small
 // frame's queue empty, so an item costs no add where there are lanes for all,
-// and a run grows with what is left (up to 4 waves' worth, and so that every
-// wave of the launch can still take 4 runs).
+// and a run grows with what is left (up to max_run, and so that every wave of
+// the launch can still take 4 runs).
+// Poll: hand-outs poll the cancel flag every 2^poll_shift items of the counter.
+template <bool Poll = false>
 struct WaveQueue {
   unsigned long long *queue;
   long long n, cur, end, shared;  // shared: first item handed out by the counter
-  int waves;
-  bool dry, stopped;
+  int waves, max_run, poll_shift;
+  bool dry, stopped;  // stopped (Poll): the band was
 
-  __device__ __forceinline__ WaveQueue(unsigned long long *queue_, long long n_, int lanes) {
+  __device__ __forceinline__ WaveQueue(unsigned long long *queue_, long long n_, int lanes, int max_run_ = 256,
+                                       int poll_shift_ = 0) {
     queue = queue_;
     n = n_;
-    stopped = false;
+    max_run = max_run_;
+    poll_shift = poll_shift_;
+    // what the kernels before left there, as a scalar load (first_lane keeps the
+    // compiler from a narrower vector load, which queues behind the adds of the
+    // waves that started first: 100 us of a 2.1 ms frame)
+    stopped = Poll && (first_lane(*queue) & kStopBit);
     waves = (int)gridDim.x * (kBlock / 64);
     // workgroups first, so that few items spread over the CUs
     const long long w = (long long)__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)) * gridDim.x + blockIdx.x;
@@ -74,25 +91,29 @@ struct WaveQueue {
     if (end > n) end = n;
     dry = shared >= n;
   }
-  // For the whole wave: lane `rank` of `need` lanes gets its item, or -1.
-  // Poll: the items are rays whose hand-out polls the cancel flag (take_work);
-  // stop is then set once the band was stopped.
-  template <bool Poll>
-  __device__ __forceinline__ long long take(const BandBufs &b, int rank, int need, int poll_shift, int &stop) {
+  // For the whole wave: lane `rank` of `need` lanes gets its item, or -1.  Items
+  // are also handed out once `stopped` is set: what a cancelled band leaves of
+  // them is the caller's.
+  __device__ __forceinline__ long long take(const BandBufs &b, int rank, int need) {
     const int have = (int)(end - cur < need ? end - cur : need);
     long long mine = rank < have ? cur + rank : -1;
     cur += have;
     if (have < need && !dry) {
       const long long left = n - end;
       const long long fair = left / (4ll * waves);
-      const long long run = fair < need - have ? need - have : fair > 256 ? 256 : fair;
+      const long long run = fair < need - have ? need - have : fair > max_run ? max_run : fair;
       unsigned long long base = 0;
       if (__lane_id() == 0) {
-        if constexpr (Poll) base = take_work(b, queue, (unsigned long long)run, poll_shift, stop);
-        else base = atomicAdd(queue, (unsigned long long)run);
+        base = atomicAdd(queue, (unsigned long long)run);
+        if constexpr (Poll) {
+          if (!(base & kStopBit) && crosses((long long)base, run, poll_shift) && poll_cancel(b, queue)) base |= kStopBit;
+        }
       }
-      base = __shfl(base, 0);
-      if constexpr (Poll) stop = __shfl(stop, 0);
+      base = first_lane(base);
+      if constexpr (Poll) {
+        stopped = (base & kStopBit) != 0;
+        base &= kStopBit - 1;
+      }
       const long long first = shared + (long long)base;
       cur = first + (need - have);
       end = first + run;
@@ -102,9 +123,7 @@ struct WaveQueue {
       }
       if (cur > end) cur = end;
       if (rank >= have && rank < need && first + (rank - have) < n) mine = first + (rank - have);
-      if constexpr (Poll) stopped = stop != 0;
     }
-    if constexpr (Poll) stop = stopped;
     return mine;
   }
 };
