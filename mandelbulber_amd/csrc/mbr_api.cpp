@@ -631,13 +631,32 @@ int band_cap(int precision, int ao_count) {
 
 // Values per hit that the fast AO keeps in the slot's AO buffer (its estimates;
 // none from quality 9 on, whose chains the kernel sums by itself: 80 values
-// per hit and more).
+// per hit and more; none where the generic surface kernel sums them).
 int fast_ao_values(const DevScene &h) {
-  return h.ao && h.fast_ao && h.ao_quality >= 2 && h.ao_quality <= 8 ? h.ao_quality * h.ao_quality - 1 : 0;
+  if (!h.ao || !h.fast_ao || h.ao_quality < 2 || h.ao_quality > 8) return 0;
+  if (h.fd.ifs_fold || (formula_generic(h.fd.formula) && !(h.plain && formula_march64(h.fd.formula)))) return 0;
+  return h.ao_quality * h.ao_quality - 1;
+}
+// Bytes of them for a band of the frame.
+size_t fast_ao_bytes(const DevScene &h, int cap, int rec_bytes) {
+  const long long hits = std::min<long long>(cap, (long long)h.width * h.height);
+  return (size_t)hits * (size_t)fast_ao_values(h) * (size_t)rec_bytes;
+}
+// Room for `need` bytes of them in the slot's AO buffer.  Without it (no memory
+// left) the kernel sums a hit's estimates one after the other.
+void want_fast_ao(Slot &sl, size_t need) {
+  if (need <= sl.sh_ao_bytes) return;
+  void *buf = nullptr;
+  if (hipMalloc(&buf, need) != hipSuccess) {
+    (void)hipGetLastError();
+    return;
+  }
+  if (sl.sh_ao) (void)hipFree(sl.sh_ao);
+  sl.sh_ao = buf;
+  sl.sh_ao_bytes = need;
 }
 int fast_ao_items(const Slot &sl, const DevScene &h) {
-  const int v = fast_ao_values(h);
-  return (size_t)sl.band.cap * (size_t)v * sl.band.rec_bytes <= sl.sh_ao_bytes ? v : 0;
+  return fast_ao_bytes(h, sl.band.cap, sl.band.rec_bytes) <= sl.sh_ao_bytes ? fast_ao_values(h) : 0;
 }
 
 int kernel_family(const mbr_scene &s) { return s.ifs_folding_mode ? kGenericFamily : s.formula; }
@@ -1504,10 +1523,11 @@ int mbr_render_device(mbr_ctx *c, const mbr_render_opts *opts, mbr_framebuffer *
   HIPCHECK(c, hipSetDevice(c->device));
   const bool slow_ao = c->host_sc.ao && !c->host_sc.fast_ao;
   const int ao_count = slow_ao ? c->host_sc.ao_count : 0;
-  const int ao_values = std::max(ao_count, fast_ao_values(c->host_sc));
   Slot &sl = c->slots[0];
-  rc = alloc_slot(c, sl, precision, band_cap(precision, ao_count), ao_values, c->host_sc.iter_fog != 0);
+  rc = alloc_slot(c, sl, precision, band_cap(precision, ao_count), ao_count, c->host_sc.iter_fog != 0);
   if (rc != MBR_OK) return rc;
+  const size_t fast_ao = fast_ao_bytes(c->host_sc, sl.band.cap, sl.band.rec_bytes);
+  want_fast_ao(sl, fast_ao);
   // reflection levels: a slot each after the first
   const int refl = c->host_sc.refl_max;
   std::vector<Slot *> levels;
@@ -1518,9 +1538,10 @@ int mbr_render_device(mbr_ctx *c, const mbr_render_opts *opts, mbr_framebuffer *
     if (rc != MBR_OK) return rc;
     for (int k = 0; k < refl; k++) {
       Slot &lk = c->refl_slots[(size_t)k];
-      rc = alloc_slot(c, lk, precision, sl.band.cap, ao_values, c->host_sc.iter_fog != 0);
+      rc = alloc_slot(c, lk, precision, sl.band.cap, ao_count, c->host_sc.iter_fog != 0);
       if (rc == MBR_OK) rc = alloc_refl(c, lk, true);
       if (rc != MBR_OK) return rc;
+      want_fast_ao(lk, fast_ao);
       levels.push_back(&lk);
     }
   }
@@ -1533,8 +1554,9 @@ int mbr_render_device(mbr_ctx *c, const mbr_render_opts *opts, mbr_framebuffer *
   Slot *pair[2] = {&sl, &c->slots[1]};
   int n_bands = (int)((last - first + sl.band.cap - 1) / sl.band.cap);
   if (split) {
-    rc = alloc_slot(c, c->slots[1], precision, sl.band.cap, ao_values, c->host_sc.iter_fog != 0);
+    rc = alloc_slot(c, c->slots[1], precision, sl.band.cap, ao_count, c->host_sc.iter_fog != 0);
     if (rc != MBR_OK) return rc;
+    want_fast_ao(c->slots[1], fast_ao);
     if (!c->side[1]) HIPCHECK(c, hipStreamCreateWithFlags(&c->side[1], hipStreamNonBlocking));
     if (!c->split_fork) HIPCHECK(c, hipEventCreateWithFlags(&c->split_fork, hipEventDisableTiming));
     if (!c->split_join) HIPCHECK(c, hipEventCreateWithFlags(&c->split_join, hipEventDisableTiming));
@@ -2138,7 +2160,7 @@ int mbr_render_batch(mbr_ctx *c, const mbr_scene *scenes, int n, const mbr_textu
   // derive every scene on the host
   std::vector<BatchFrame> frames(n);
   long long ao_total = 0;
-  int max_ao = 0, max_fast = 0;
+  int max_ao = 0;
   for (int i = 0; i < n; i++) {
     rc = prepare_scene(c, &scenes[i], lightmap, frames[i].p);
     if (rc != MBR_OK) return c->fail(rc, "scene " + std::to_string(i) + ": " + c->err);
@@ -2155,7 +2177,6 @@ int mbr_render_batch(mbr_ctx *c, const mbr_scene *scenes, int n, const mbr_textu
     ao_total += frames[i].p.d.ao_count;
     const DevScene &d = frames[i].p.d;
     if (d.ao && !d.fast_ao) max_ao = std::max(max_ao, d.ao_count);
-    max_fast = std::max(max_fast, fast_ao_values(d));
   }
   // upload scene blocks and AO tables
   if (n > c->batch_sc_cap) {
@@ -2212,8 +2233,12 @@ int mbr_render_batch(mbr_ctx *c, const mbr_scene *scenes, int n, const mbr_textu
     return c->fail(MBR_ERR_INVALID_ARG, "slots must be 1..4 and blocks_per_cu 1..32");
   const int n_slots = cands.empty() ? slots : kMaxSlots;
   for (int k = 0; k < n_slots; k++) {
-    rc = alloc_slot(c, c->slots[k], precision, cap, std::max(max_ao, max_fast));
+    rc = alloc_slot(c, c->slots[k], precision, cap, max_ao);
     if (rc != MBR_OK) return rc;
+    size_t fast_ao = 0;
+    for (const BatchFrame &f : frames)
+      fast_ao = std::max(fast_ao, fast_ao_bytes(f.p.d, cap, c->slots[k].band.rec_bytes));
+    want_fast_ao(c->slots[k], fast_ao);
   }
   mbr_batch_result res;
   std::memset(&res, 0, sizeof res);
