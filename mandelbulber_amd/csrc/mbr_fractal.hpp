@@ -844,6 +844,11 @@ MBR_HD void de_begin(const FractalK<T> &f, V3<T> p, DEIter<T> &s) {
       s.r = r2 * s.inv_r;
     }
   }
+  if constexpr (F == 7 && sizeof(T) == 8) {
+    // the sort's maxima drop a NaN among three coordinates, but not all three
+    const bool nan = __builtin_isunordered(p.x, p.y) || __builtin_isunordered(p.z, p.z);
+    if (nan) s.z = V3<T>{T(__builtin_nan("")), T(__builtin_nan("")), T(__builtin_nan(""))};
+  }
 }
 
 // !(|z| <= R) of the folding formulas' escape test from q = |z|^2, for R =
@@ -862,11 +867,13 @@ MBR_HD bool beyond(float q) {
   return !(q <= (R == 1000 ? 0x1.e84802p+19f : 0x1.000002p+20f));
 }
 
-// The larger and the smaller of two values, and z limited to [-lim, lim].
+// The larger and the smaller of two values, and z limited to [-lim, lim].  A NaN
+// stays in FP32 (v_maximum3_f32, which also needs no canonical operands); in
+// FP64, whose v_max_f64 gives the other operand, de_begin sees to it.
 MBR_HD double larger(double a, double b) { return __builtin_fmax(a, b); }
 MBR_HD double smaller(double a, double b) { return __builtin_fmin(a, b); }
-MBR_HD float larger(float a, float b) { return __builtin_fmaxf(a, b); }
-MBR_HD float smaller(float a, float b) { return __builtin_fminf(a, b); }
+MBR_HD float larger(float a, float b) { return __builtin_elementwise_maximum(a, b); }
+MBR_HD float smaller(float a, float b) { return __builtin_elementwise_minimum(a, b); }
 MBR_HD double limited(double z, double lim) { return smaller(larger(z, -lim), lim); }
 MBR_HD float limited(float z, float lim) {
 #if defined(__HIP_DEVICE_COMPILE__)
@@ -1077,7 +1084,8 @@ MBR_HD bool de_iter(const FractalK<T> &f, DEIter<T> &s, int N) {
     esc = !(r <= f.bailout);
   } else if constexpr (F == 7) {  // menger_sponge
     // |x|, |y|, |z| in descending order: the reference's three conditional
-    // swaps, as maxima and minima (2 instructions each for 4 in FP32, 6 in FP64)
+    // swaps, as maxima and minima (2 instructions each for 4 in FP32, 6 in
+    // FP64); with a NaN among them all three are, and the orbit has escaped
     const T ax = M::fabs(z.x), ay = M::fabs(z.y), az = M::fabs(z.z);
     const T hi = larger(ax, ay), lo = smaller(ax, ay);
     const T mid = smaller(hi, az);
