@@ -419,9 +419,11 @@ typedef struct mbr_stats {
                                             rays run two bands at a time, so these may
                                             add up to more than ms_total */
   uint64_t rays, hits;
-  uint64_t march_de_calls;         /* DE calls of primary march + bisection */
+  uint64_t march_de_calls;         /* DE calls of primary march + bisection; in the
+                                      FP64 march modes a hit's last march step counts
+                                      for both (it runs once) */
   uint64_t shade_de_calls;         /* DE calls of normals, shadow, AO, colour */
-  uint64_t iterations;             /* formula iterations over all DE calls */
+  uint64_t iterations;             /* formula iterations run, over all DE calls */
   uint64_t march_iterations;       /* ... of which in the march kernel */
   uint64_t shade_iterations;       /* ... of which in the shade kernel */
   uint64_t march_launches, shade_launches, finish_launches;

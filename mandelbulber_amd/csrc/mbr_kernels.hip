@@ -750,10 +750,9 @@ __device__ __forceinline__ void march64_body(const DevScene *__restrict__ scp, B
         }
         if (dist < s.thr) {
           if constexpr (Src == kRays) {
-            // the call counters count this estimate for the march and for the
-            // search that starts from it
+            // mbr_stats.march_de_calls counts it for the march and for the search
+            // that starts from it; it runs once, and its iterations count once
             cnt.de_calls += 1;
-            if (!early) cnt.iterations += (uint32_t)(call.it.L < N ? call.it.L + 1 : N);
           }
           below = dist < 0.1 * s.thr;
           step = s.step * 0.5;
