@@ -10,7 +10,7 @@
 #include <algorithm>
 #include <cmath>
 #include <cstdint>
-#include <system_error>
+#include <exception>
 #include <thread>
 #include <utility>
 #include <vector>
@@ -48,9 +48,11 @@ inline void zpartition(ZEntry *d, int l, int p, int &i_out, int &j_out) {
 }
 
 // The two sides of a partition are independent ranges, so the order in which
-// they are sorted does not change the result: up to kForks large ones go to
-// threads of their own, the larger side of the others to a stack (at most
-// log2 n of them).
+// they are sorted does not change the result: the smaller sides of a range's
+// first kForks partitions, where large, go to threads of their own (which fork
+// again, each with the forks its parent has left: at most 2^kForks - 1 = 15
+// threads in all), the larger side of the others to a stack (at most log2 n of
+// them).  Without a thread to be had the range is sorted here.
 constexpr int kForks = 4;
 void zsort(ZEntry *d, int lo, int hi, int forks) {
   std::pair<int, int> stack[32];
@@ -70,7 +72,7 @@ void zsort(ZEntry *d, int lo, int hi, int forks) {
         lo = large.first;
         hi = large.second;
         continue;
-      } catch (const std::system_error &) {  // no thread to be had
+      } catch (const std::exception &) {  // no thread, or no memory for its state
         forks = forked;
       }
     }
