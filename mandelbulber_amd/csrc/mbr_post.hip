@@ -7,8 +7,9 @@
 // keeps the steepest horizon -dz/dr per direction and adds colour x AO x
 // intensity x (1 - opacity) to its own compiled 16-bit value.  No pixel
 // reads another pixel's output, so one lane per pixel needs no ordering.
-// The arithmetic is the reference's FP64 in the reference's order with
-// contraction off; the direction table comes from the host's libm.
+// The arithmetic is the reference's FP64 with contraction off (samples compare
+// by cross products instead of quotients); the direction table comes from the
+// host's libm.
 // Workgroups cover 16x16 pixel tiles so the near samples of a tile share
 // cache lines; the far samples (up to width/2 away) come from L2.
 #include <hipcub/hipcub.hpp>
@@ -112,12 +113,14 @@ __global__ void __launch_bounds__(kTile *kTile)
         const double xx = x + rr * ca, yy = y + rr * sa;
         if ((int)xx == x && (int)yy == y) continue;
         if (xx < 0 || xx > p.width - 1 || yy < 0 || yy > p.height - 1) continue;
-        const double z2 = zb[(size_t)(int)yy * p.width + (int)xx];
+        const float zf = zb[(size_t)(int)yy * p.width + (int)xx];
+        const double z2 = zf;
         double xx2, yy2;
         ssao_sample(p, xx, yy, z2, xx2, yy2);
         const double dx = xx2 - x2, dy = yy2 - y2, dz = z2 - z;
         const double d = dx * dx + dy * dy;
-        if (-dz * fabs(dz) * best_d > best_n * fabs(best_n) * d) {
+        // (a depth of -inf has no slope, but its products compare as the steepest)
+        if (-dz * fabs(dz) * best_d > best_n * fabs(best_n) * d && zf > -__builtin_inff()) {
           best_n = -dz;
           best_d = d;
         }
