@@ -4,6 +4,7 @@
 #pragma once
 
 #include <algorithm>
+#include <atomic>
 
 #include "mbr_kernels.hpp"
 
@@ -158,20 +159,31 @@ __device__ __forceinline__ void lane_loop(int &state, Fetch fetch, Step step, Do
   }
 }
 
+// Workgroups of a kernel that fit the current device at once; `known` holds them
+// per device (0: not asked yet), since devices may differ in their CUs.
+constexpr int kKnownDevices = 32;
+inline int resident_blocks(const void *kernel, std::atomic<int> (&known)[kKnownDevices]) {
+  int dev = 0, per_cu = 0, cus = 0;
+  if (hipGetDevice(&dev) != hipSuccess) return 1 << 20;
+  const bool keep = dev >= 0 && dev < kKnownDevices;
+  int n = keep ? known[dev].load(std::memory_order_relaxed) : 0;
+  if (n > 0) return n;
+  if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kernel, kBlock, 0) != hipSuccess ||
+      hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || per_cu * cus <= 0)
+    return 1 << 20;
+  n = per_cu * cus;
+  if (keep) known[dev].store(n, std::memory_order_relaxed);
+  return n;
+}
 
 // Launch of a persistent kernel: at most the workgroups that fit the chip at
 // once (and `blocks`, the caller's share), so that no wave starts on its first
-// items only after the others ran out.
+// items only after the others ran out.  (Where another stream's kernels hold
+// the chip some still do.)
 template <auto Kernel, class... A>
 static void launch_resident(int blocks, hipStream_t s, A... args) {
-  static const int resident = [] {
-    int per_cu = 0, dev = 0, cus = 0;
-    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, Kernel, kBlock, 0) != hipSuccess ||
-        hipGetDevice(&dev) != hipSuccess ||
-        hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || per_cu * cus <= 0)
-      return 1 << 20;
-    return per_cu * cus;
-  }();
+  static std::atomic<int> known[kKnownDevices];
+  const int resident = resident_blocks((const void *)Kernel, known);
   hipLaunchKernelGGL(Kernel, dim3((unsigned)std::max(1, std::min(blocks, resident))), dim3(kBlock), 0, s, args...);
 }
 
