@@ -1037,15 +1037,24 @@ struct HitDE {
   }
 };
 
+// The step of the normal's stencil.
+template <class T>
+__device__ __forceinline__ T stencil_size(const DevScene &sc, const ShaderIn<T> &in) {
+  const ShadeK<T> &k = sc.shade<T>();
+  if (sc.interior) return in.dist_thresh * k.quality * T(0.2) * k.smoothness;
+  return in.delta * k.smoothness;
+}
+
 // Surface shading of the hits (ObjectShader's estimates) as three kinds of
 // items that depend on the hit's march alone and run side by side: the shadow
 // ray (MainShadow, chained estimates), the normal's four estimates (one item
-// each; slowShading's 11^3 chained as one) and the colouring orbit.  A wave
+// each; slowShading's stencil has a kernel of its own) and the colouring orbit.  A wave
 // works through the shadow rays, then the normals, then the colours; waves
 // whose lanes still follow long rays leave the rest of the queues to others.
 // One lane per hit instead ran them one after the other at 20-27% active
 // lanes and 11-13% VALU busy, and the deep-zoom variant at one wave per SIMD
-// (256 + 107 registers).  hit_lit forms the shade from the results: estimates in sb.base and sb.spec[0], the shadow factor in sb.spec[1], the detail size
+// (256 + 107 registers).  hit_lit forms the shade from the results: estimates
+// in sb.base and sb.spec[0], the shadow factor in sb.spec[1], the detail size
 // MainShadow leaves in sb.fast_ao.
 enum : int { HIT_SHADOW = 1, HIT_NORMAL = 2, HIT_COLOUR = 4 };
 template <class T, int F, bool Deep, int P>
@@ -1169,27 +1178,15 @@ __global__ void __launch_bounds__(kBlock, (HitPolicy<T, F, Deep, P>::waves))
   if (kinds & HIT_NORMAL) {
     // differences of FP32 estimates a stencil step apart keep few digits
     constexpr bool kEst64 = formula_march64(F) && sizeof(T) < 8;
-    const int N5 = sc.N * 5, slow = sc.slow_shading, minN = slow ? sc.minN : 0;
-    const long long n_items = slow ? n_hits : 4 * n_hits;
+    const int N5 = sc.N * 5;
+    const long long n_items = 4 * n_hits;
     const int lanes = item_lanes(n_items);
     WaveQueue<> queue(&b.counters[CNT_NORMALQ], n_items, lanes);
     int state = lane < lanes ? MS_NEED : MS_EXHAUSTED;
     long long item = 0;
-    V3<T> point = v3<T>(0, 0, 0), p2 = point, sum = point;
-    V3<double> point64 = v3<double>(0, 0, 0);
-    double px = 0, py = 0, pz = 0;
-    T delta = 0, detail = 0, dist = 0;
+    T detail = 0, dist = 0;
     bool early = false;
     HitDE<T, F, Deep, P, IP> call;
-    auto begin = [&](V3<T> off) __attribute__((always_inline)) {
-      DEInfo info;
-      early = call.begin(fd, f, point, point64, off, detail, N5, minN, true, dist, info);
-      state = early ? MS_DONE : MS_ITER;
-    };
-    auto stencil = [&]() __attribute__((always_inline)) {
-      p2 = v3<T>((T)px, (T)py, (T)pz);
-      begin(p2 * delta);
-    };
     lane_loop<kIters>(
         state,
         [&](int rank, int n_need) {
@@ -1201,65 +1198,39 @@ __global__ void __launch_bounds__(kBlock, (HitPolicy<T, F, Deep, P>::waves))
           }
           item = mine;
           ShaderIn<T> in;
-          load_hit(sc, b, b.hit_list[slow ? item : item >> 2], in);
-          point = in.point;
-          point64 = in.point64;
+          load_hit(sc, b, b.hit_list[item >> 2], in);
           detail = in.detail;
-          delta = in.delta * k.smoothness;
-          if (sc.interior) delta = in.dist_thresh * k.quality * T(0.2) * k.smoothness;
-          if (slow) {
-            sum = v3<T>(0, 0, 0);
-            px = py = pz = -1.0;
-            stencil();
+          const T delta = stencil_size<T>(sc, in);
+          const int j = (int)(item & 3);
+          DEInfo info;
+          if constexpr (kEst64) {
+            const double d = (double)delta;
+            call.begin64(fd, in.point64 + v3<double>(j == 1 ? d : 0.0, j == 2 ? d : 0.0, j == 3 ? d : 0.0),
+                         (double)detail, N5, 0, true, info);
+            state = MS_ITER;
           } else {
-            const int j = (int)(item & 3);
-            if constexpr (kEst64) {
-              DEInfo info;
-              const double d = (double)delta;
-              call.begin64(fd, point64 + v3<double>(j == 1 ? d : 0.0, j == 2 ? d : 0.0, j == 3 ? d : 0.0),
-                           (double)detail, N5, minN, true, info);
-              state = MS_ITER;
-              return;
-            }
-            begin(v3<T>(j == 1 ? delta : T(0), j == 2 ? delta : T(0), j == 3 ? delta : T(0)));
+            const V3<T> off = v3<T>(j == 1 ? delta : T(0), j == 2 ? delta : T(0), j == 3 ? delta : T(0));
+            early = call.begin(fd, f, in.point, in.point64, off, detail, N5, 0, true, dist, info);
+            state = early ? MS_DONE : MS_ITER;
           }
         },
         [&]() { return call.step(fd, f, N5); },
         [&]() {
           cnt.de_calls += 1;
-          if constexpr (kEst64) {
-            if (!slow) {
-              DEInfo info;
-              sb.est[item & 3][item >> 2] = call.end64(fd, (double)detail, N5, minN, true, info);
-              cnt.iterations += (uint32_t)info.work;
-              state = MS_NEED;
-              return;
-            }
-          }
-          if (!early) {
-            DEInfo info;
-            dist = call.end(fd, f, detail, N5, minN, true, info);
-            cnt.iterations += (uint32_t)info.work;
-          }
           state = MS_NEED;
-          if (!slow) {
-            const long long j = item & 3, tid = item >> 2;
+          const long long j = item & 3, tid = item >> 2;
+          DEInfo info;
+          if constexpr (kEst64) {
+            sb.est[j][tid] = call.end64(fd, (double)detail, N5, 0, true, info);
+            cnt.iterations += (uint32_t)info.work;
+          } else {
+            if (!early) {
+              dist = call.end(fd, f, detail, N5, 0, true, info);
+              cnt.iterations += (uint32_t)info.work;
+            }
             if (j < 3) sb.base[j * n + tid] = dist;
             else sb.spec[tid] = dist;
-            return;
           }
-          // the 11^3 stencil with the reference's accumulated loop variables
-          sum = sum + p2 * dist;
-          pz += 0.2;
-          if (!(pz <= 1.0)) { pz = -1.0; py += 0.2; }
-          if (!(py <= 1.0)) { py = -1.0; px += 0.2; }
-          if (px <= 1.0) {
-            stencil();
-            return;
-          }
-          sb.base[item] = sum.x;
-          sb.base[n + item] = sum.y;
-          sb.base[2 * n + item] = sum.z;
         });
   }
 
@@ -1281,6 +1252,69 @@ __global__ void __launch_bounds__(kBlock, (HitPolicy<T, F, Deep, P>::waves))
     }
   }
   poll_before_ao(sc, b);
+  unsigned long long v[ST_COUNT] = {0};
+  v[ST_SHADE_DE] = cnt.de_calls;
+  v[ST_SHADE_ITERS] = cnt.iterations;
+  flush_stats(stats, v);
+}
+
+// CalculateNormals with slowShading (src/shaders.cpp:720-757): the estimates of
+// an 11^3 stencil about the hit, each weighting its offset, summed in the
+// reference's order; the sum in sb.base.  A wave per hit and a lane per
+// estimate, added up lane by lane.  As a chain of estimates on one lane of
+// k_hits a 120x90 FP64 bulb's frame took 14.4 ms, with this 1.4.
+template <class T, int F, bool Deep, int P, int IP>
+__global__ void __launch_bounds__(kBlock, (HitPolicy<T, F, Deep, P>::waves))
+    k_slow_normals(const DevScene *__restrict__ scp, BandBufs b, SurfBufs<T> sb, unsigned long long *stats) {
+  const DevScene &sc = *scp;
+  constexpr bool kLocal = local_scene(F, P);
+  const FractalK<T> f_local = kLocal ? sc.frac<T>() : FractalK<T>{};
+  const FractalK<T> &f = kLocal ? f_local : sc.frac<T>();
+  const FractalK<double> &fd = sc.fd;
+  const int N5 = sc.N * 5, minN = sc.minN;
+  const long long n_hits = (long long)b.counters[CNT_HITS];
+  const long long n = sb.n;
+  const int lane = __lane_id();
+  // the stencil's coordinates: the reference's loop variable adds 0.2 up to 1
+  int side = 0;
+  for (double v = -1.0; v <= 1.0; v += 0.2) side++;
+  auto coord = [](int k) {
+    double v = -1.0;
+    for (int i = 0; i < k; i++) v += 0.2;
+    return v;
+  };
+  const int points = side * side * side;
+  LaneCount cnt = {0, 0};
+  const long long waves = (long long)gridDim.x * (kBlock / 64);
+  for (long long tid = (long long)blockIdx.x * (kBlock / 64) + (threadIdx.x >> 6); tid < n_hits; tid += waves) {
+    ShaderIn<T> in;
+    load_hit(sc, b, b.hit_list[tid], in);
+    const T delta = stencil_size<T>(sc, in);
+    V3<T> sum = v3<T>(0, 0, 0);
+    for (int first = 0; first < points; first += 64) {
+      const int q = first + lane;
+      const V3<T> p2 = v3<T>((T)coord(q / (side * side)), (T)coord(q / side % side), (T)coord(q % side));
+      T dist = 0;
+      if (q < points) {
+        HitDE<T, F, Deep, P, IP> call;
+        DEInfo info;
+        cnt.de_calls += 1;
+        if (!call.begin(fd, f, in.point, in.point64, p2 * delta, in.detail, N5, minN, true, dist, info)) {
+          while (!call.step(fd, f, N5)) {
+          }
+          dist = call.end(fd, f, in.detail, N5, minN, true, info);
+          cnt.iterations += (uint32_t)info.work;
+        }
+      }
+      for (int l = 0; l < 64 && first + l < points; l++)
+        sum = sum + v3<T>(__shfl(p2.x, l), __shfl(p2.y, l), __shfl(p2.z, l)) * __shfl(dist, l);
+    }
+    if (lane == 0) {
+      sb.base[tid] = sum.x;
+      sb.base[n + tid] = sum.y;
+      sb.base[2 * n + tid] = sum.z;
+    }
+  }
   unsigned long long v[ST_COUNT] = {0};
   v[ST_SHADE_DE] = cnt.de_calls;
   v[ST_SHADE_ITERS] = cnt.iterations;
@@ -2512,7 +2546,16 @@ hipError_t shade_run(const DevScene *sc, const BandBufs &b, int band_first, AODe
   auto hits = [&](int kinds) {
     variants([&](auto d, auto f, auto pl, auto ip) {
       constexpr int F = decltype(f)::value, Pl = decltype(pl)::value, IP = decltype(ip)::value;
-      launch_resident<k_hits<T, F, decltype(d)::value, Pl, IP>>(persist_blocks, s, sc, b, sb, kinds, stats);
+      if ((kinds & HIT_NORMAL) && sbuf.slow_normals) {
+        launch_resident<k_slow_normals<T, F, decltype(d)::value, Pl, IP>>(persist_blocks, s, sc, b, sb, stats);
+        kinds &= ~HIT_NORMAL;
+      }
+      // deep zooms: a quarter of the workgroups (2 per CU), which keep the FP64
+      // units busy and leave room for the other stream's march (4K Mandelbox
+      // 78.4 ms with as many as fit, 76.4 with 4 per CU, 75.6 with 2; 1280x720
+      // 14.1, 13.5 with 3 and 13.0 with 2; 640x360 on one stream 6.2 and 6.0)
+      const int blocks = decltype(d)::value ? persist_blocks / 4 : persist_blocks;
+      launch_resident<k_hits<T, F, decltype(d)::value, Pl, IP>>(blocks, s, sc, b, sb, kinds, stats);
     });
   };
   // plain scenes take a variant without the optional terms' branches (and the
