@@ -1475,7 +1475,7 @@ void fill_stats(mbr_stats *stats, const unsigned long long *v, long long rays, i
   stats->fp64_redo_rays = v[ST_REDO];
   stats->ao_de_calls = v[ST_AO_DE];
   stats->ao_iterations = v[ST_AO_ITERS];
-  stats->ao_steps = v[ST_AO_STEPS];
+  stats->ao_steps = v[ST_AO_DE];  // an estimate each
 }
 
 // After a render has finished on the device: MBR_ERR_CANCELLED when

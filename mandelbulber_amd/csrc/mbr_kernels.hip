@@ -161,7 +161,7 @@ struct MarchOut {
   V3<double> point;
   double scan, distThresh, dist;
   int buffCount, object;
-  bool found, missed;
+  bool found;
 };
 
 struct RayState {
@@ -409,7 +409,7 @@ __device__ __forceinline__ void march_body(const DevScene *__restrict__ scp, Ban
             MarchOut o;
             o.point = v3<double>(0, 0, 0);
             o.scan = 0; o.distThresh = 0; o.dist = 0; o.buffCount = 0; o.object = OBJ_FRACTAL;
-            o.found = false; o.missed = false;
+            o.found = false;
             write_ray(b, r, o);
           } else {
             begin_de();
@@ -449,7 +449,6 @@ __device__ __forceinline__ void march_body(const DevScene *__restrict__ scp, Ban
         o.buffCount = s.i;
         o.object = s.object;
         o.found = false;
-        o.missed = false;
         write_ray(b, r, o);
         state = MS_NEED;
       } else {
@@ -594,7 +593,6 @@ __device__ __forceinline__ void march64_body(const DevScene *__restrict__ scp, B
     o.buffCount = s.i;
     o.object = s.object;
     o.found = found;
-    o.missed = false;
     write_ray(b, r, o);
     if (found) hit_list.append(r);
     appended |= found;
@@ -705,7 +703,7 @@ __device__ __forceinline__ void march64_body(const DevScene *__restrict__ scp, B
             MarchOut o;
             o.point = v3<double>(0, 0, 0);
             o.scan = 0; o.distThresh = 0; o.dist = 0; o.buffCount = 0; o.object = OBJ_FRACTAL;
-            o.found = false; o.missed = false;
+            o.found = false;
             write_ray(b, r, o);
           } else {
             begin_march();
@@ -960,13 +958,13 @@ __global__ void __launch_bounds__(kBlock) k_surface_generic(const DevScene *__re
     ShaderIn<T> in;
     load_hit(sc, b, r, in);
     in.view = cvt<T>(ray_dir(sc, b, band_first, r));
-    in.normal = normals<T, 0, false>(sc, in, cnt);
+    in.normal = normals<T, 0>(sc, in, cnt);
     T shadow = 1;
-    if (sc.shadow) shadow = main_shadow<T, 0, false>(sc, in, cnt);
+    if (sc.shadow) shadow = main_shadow<T, 0>(sc, in, cnt);
     const RGBT<T> colour = surface_colour<T, false, true>(sc, in, cnt);
     put_lit<T>(sc, in, light_hit<T>(sc, in, shadow), tid, sb);
     put_colour(b, sb, r, tid, colour);
-    if (sc.ao && sc.fast_ao) sb.fast_ao[tid] = fast_ao2<T, 0, false>(sc, in, cnt);
+    if (sc.ao && sc.fast_ao) sb.fast_ao[tid] = fast_ao2<T, 0>(sc, in, cnt);
     else if (sc.ao) sb.fast_ao[tid] = in.detail;
   }
   poll_before_ao(sc, b);
@@ -1632,7 +1630,6 @@ __device__ __forceinline__ void ao_body(const DevScene *__restrict__ scp, BandBu
   bool early = false;  // the estimate ended in begin_de, without iterating
   DECall<T> call;
   LaneCount cnt = {0, 0};
-  unsigned long long ao_steps = 0;
 
   // start the distance estimate at P + dir * r; DONE when no iteration runs
   auto begin_de = [&]() {
@@ -1732,7 +1729,6 @@ __device__ __forceinline__ void ao_body(const DevScene *__restrict__ scp, BandBu
         cnt.iterations += (uint32_t)info.work;
       }
       // one step of the AO ray (src/shaders.cpp:625-662)
-      ao_steps++;
       if (dist < thr_f || mi) {
         T shadowTemp = T(1) - (end_dist - r) / end_dist;
         if (shadowTemp < T(0)) shadowTemp = 0;
@@ -1755,7 +1751,6 @@ __device__ __forceinline__ void ao_body(const DevScene *__restrict__ scp, BandBu
   v[ST_SHADE_ITERS] = cnt.iterations;
   v[ST_AO_DE] = cnt.de_calls;
   v[ST_AO_ITERS] = cnt.iterations;
-  v[ST_AO_STEPS] = ao_steps;
   flush_stats(stats, v);
 }
 
@@ -1936,7 +1931,7 @@ struct FxStages {
     RGBT<T> nc = {0, 0, 0};
     const T mi = (T)sc.main_light_intensity, dl = k.direct_light;
     if (mi * dl > T(0)) {
-      const T sh = main_shadow<T, F, false>(sc, pin, cnt);
+      const T sh = main_shadow<T, F>(sc, pin, cnt);
       nc.R += sh * T(sc.main_light_colour[0]) / T(65536) * mi * dl;
       nc.G += sh * T(sc.main_light_colour[1]) / T(65536) * mi * dl;
       nc.B += sh * T(sc.main_light_colour[2]) / T(65536) * mi * dl;
@@ -1959,7 +1954,7 @@ struct FxStages {
       if constexpr (sizeof(T) == 8) tab.dir = ao.dir_d; else tab.dir = ao.dir_f;
       tab.rgb = ao.rgb;
       tab.count = ao.count;
-      const RGBT<T> a = ambient_occlusion<T, F, false>(sc, pin, tab, cnt);
+      const RGBT<T> a = ambient_occlusion<T, F>(sc, pin, tab, cnt);
       nc.R += a.R * k.global_ilum;
       nc.G += a.G * k.global_ilum;
       nc.B += a.B * k.global_ilum;
@@ -2000,7 +1995,7 @@ struct FxStages {
       }
     }
     if (sc.vol_main) {
-      const T sh = main_shadow<T, F, false>(sc, pin, cnt);
+      const T sh = main_shadow<T, F>(sc, pin, cnt);
       const T I0 = (T)sc.vol_intensity[0];
       o.rgb.R += sh * step * I0 * T(sc.main_light_colour[0]) / T(65536);
       o.rgb.G += sh * step * I0 * T(sc.main_light_colour[1]) / T(65536);
@@ -2179,7 +2174,7 @@ __global__ void __launch_bounds__(kBlock) k_refl_setup(const DevScene *__restric
     ShaderIn<double> in;
     load_hit(sc, prev, r, in);
     in.view = dir;
-    const V3<double> n = normals<double, F, false>(sc, in, cnt);
+    const V3<double> n = normals<double, F>(sc, in, cnt);
     const V3<double> d2 = dir - (n * dot(dir, n)) * 2.0;
     const double thr = prev.thr[r];
     const V3<double> o = in.point64 + d2 * thr;
@@ -2384,7 +2379,6 @@ hipError_t launch_refl_setup(const DevScene *sc, const BandBufs &prev, const Ban
 
 hipError_t launch_refl_march(const DevScene *sc, const BandBufs &next, int band_first, int formula, int blocks,
                              unsigned long long *stats, hipStream_t s) {
-  const dim3 grid((unsigned)std::max(1, blocks));
   if (formula_generic(formula))
     launch_resident<k_march64<double, 0, 0, 0, kRefl>>(blocks, s, sc, next, band_first, 0, stats);
   else if (formula == 7)
@@ -2429,7 +2423,6 @@ hipError_t launch_march(int precision, const DevScene *sc, const BandBufs &b, in
   if (band_rays <= 0) return hipSuccess;
   // generic formulas: FP64, or the FP64 march of FP32_FIXUP (FP32 records)
   if (formula_generic(formula) && precision > 1) return hipErrorInvalidValue;
-  const dim3 grid((unsigned)std::max(1, persist_blocks));
   if (precision == 2) {
     auto go = [&](auto f_tag, auto plain_tag, auto ip_tag) {
       constexpr int F = decltype(f_tag)::value;
@@ -2458,7 +2451,6 @@ hipError_t launch_march(int precision, const DevScene *sc, const BandBufs &b, in
 hipError_t launch_march_fix(const DevScene *sc, const BandBufs &b, int band_first, int formula, int plain,
                             int persist_blocks, unsigned long long *stats, hipStream_t s, bool ip8) {
   if (formula_generic(formula)) return hipErrorInvalidValue;
-  const dim3 grid((unsigned)std::max(1, persist_blocks));
   auto hand = [&](auto f_tag, auto plain_tag, auto ip_tag) {
     constexpr int F = decltype(f_tag)::value, IP = decltype(ip_tag)::value;
     constexpr int Pl = decltype(plain_tag)::value;

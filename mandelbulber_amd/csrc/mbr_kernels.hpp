@@ -14,7 +14,7 @@ enum StatIdx {
   ST_OVF_RAYS,   // rays whose step record outgrew the slab
   ST_POOL_MISS,  // records dropped because the overflow pool was full
   ST_OVF_CHUNKS, // overflow chunks taken
-  ST_AO_DE, ST_AO_ITERS, ST_AO_STEPS,
+  ST_AO_DE, ST_AO_ITERS,
   ST_COUNT = 14
 };
 

@@ -6,7 +6,6 @@
 //   ambient_occlusion<T>  AmbientOcclusion       src/shaders.cpp:607-673
 //   surface_colour<T>     SurfaceColour          src/shaders.cpp:813-926
 //   index_to_colour       IndexToColour          src/shaders.cpp:1273-1305
-//   object_shader<T>      ObjectShader           src/shaders.cpp:21-112
 //   background<T>         BackgroundShader       src/shaders.cpp:114-183
 //   volumetric<T>         VolumetricShader       src/shaders.cpp:185-478
 //   aux_shadow<T>         AuxShadow              src/shaders.cpp:1075-1132
@@ -68,7 +67,7 @@ MBR_HD T de(const DevScene &sc, V3<T> p, T detail, int N, int minN, bool normalM
 // of deep-zoom scenes): the point is formed in FP64 and the estimate starts
 // in FP64 (calc_distance_p64); otherwise the point and the estimate are in
 // the caller's precision.
-template <class T, int F, bool Deep>
+template <class T, int F, bool Deep = false>
 MBR_HD T de_at(const DevScene &sc, const ShaderIn<T> &in, V3<T> off, T detail, int N, int minN, bool normalMode,
                DEInfo &info, LaneCount &cnt) {
   if constexpr (Deep && sizeof(T) < 8 && F != 0) {
@@ -81,7 +80,7 @@ MBR_HD T de_at(const DevScene &sc, const ShaderIn<T> &in, V3<T> off, T detail, i
   }
 }
 
-template <class T, int F = 0, bool Deep = false>
+template <class T, int F = 0>
 MBR_HD V3<T> normals(const DevScene &sc, ShaderIn<T> &in, LaneCount &cnt) {
   const ShadeK<T> &k = sc.shade<T>();
   V3<T> n = v3<T>(0, 0, 0);
@@ -111,10 +110,10 @@ MBR_HD V3<T> normals(const DevScene &sc, ShaderIn<T> &in, LaneCount &cnt) {
   if (!sc.slow_shading) {
     T delta = in.delta * k.smoothness;
     if (sc.interior) delta = in.dist_thresh * k.quality * T(0.2) * k.smoothness;
-    T s1 = de_at<T, F, Deep>(sc, in, v3<T>(0, 0, 0), in.detail, N5, 0, true, info, cnt);
-    T s2 = de_at<T, F, Deep>(sc, in, v3<T>(delta, 0, 0), in.detail, N5, 0, true, info, cnt);
-    T s3 = de_at<T, F, Deep>(sc, in, v3<T>(0, delta, 0), in.detail, N5, 0, true, info, cnt);
-    T s4 = de_at<T, F, Deep>(sc, in, v3<T>(0, 0, delta), in.detail, N5, 0, true, info, cnt);
+    T s1 = de_at<T, F>(sc, in, v3<T>(0, 0, 0), in.detail, N5, 0, true, info, cnt);
+    T s2 = de_at<T, F>(sc, in, v3<T>(delta, 0, 0), in.detail, N5, 0, true, info, cnt);
+    T s3 = de_at<T, F>(sc, in, v3<T>(0, delta, 0), in.detail, N5, 0, true, info, cnt);
+    T s4 = de_at<T, F>(sc, in, v3<T>(0, 0, delta), in.detail, N5, 0, true, info, cnt);
     n = v3<T>(s2 - s1, s3 - s1, s4 - s1);
   } else {
     T delta = in.delta * k.smoothness;
@@ -124,7 +123,7 @@ MBR_HD V3<T> normals(const DevScene &sc, ShaderIn<T> &in, LaneCount &cnt) {
       for (double py = -1.0; py <= 1.0; py += 0.2)
         for (double pz = -1.0; pz <= 1.0; pz += 0.2) {
           V3<T> p2 = v3<T>((T)px, (T)py, (T)pz);
-          T d = de_at<T, F, Deep>(sc, in, p2 * delta, in.detail, N5, sc.minN, true, info, cnt);
+          T d = de_at<T, F>(sc, in, p2 * delta, in.detail, N5, sc.minN, true, info, cnt);
           n = n + p2 * d;
         }
   }
@@ -164,7 +163,7 @@ MBR_HD T fog_opacity(const DevScene &sc, T dist_step, int iters) {
   return iter_opacity<T>(dist_step, T(iters), T(sc.N), (T)sc.iter_fog_trim, (T)sc.iter_fog_opacity);
 }
 
-template <class T, int F = 0, bool Deep = false>
+template <class T, int F = 0>
 MBR_HD T main_shadow(const DevScene &sc, ShaderIn<T> &in, LaneCount &cnt) {
   const ShadeK<T> &k = sc.shade<T>();
   T factor = in.delta / k.resolution;
@@ -182,7 +181,7 @@ MBR_HD T main_shadow(const DevScene &sc, ShaderIn<T> &in, LaneCount &cnt) {
 
     const float dist_thresh = sc.shadow_fx ? fx_thresh<T>(sc, in.point + in.light * i) : (float)in.dist_thresh;
     in.detail = (T)dist_thresh;
-    dist = de_at<T, F, Deep>(sc, in, in.light * i, in.detail, sc.N, sc.minN, false, info, cnt);
+    dist = de_at<T, F>(sc, in, in.light * i, in.detail, sc.N, sc.minN, false, info, cnt);
     if (sc.bsoft) {
       T angle = (dist - (T)dist_thresh) / i;
       if (angle < 0) angle = 0;
@@ -203,7 +202,7 @@ MBR_HD T main_shadow(const DevScene &sc, ShaderIn<T> &in, LaneCount &cnt) {
   return sc.bsoft ? (T(1) - maxSoft) : shadowTemp;
 }
 
-template <class T, int F = 0, bool Deep = false>
+template <class T, int F = 0>
 MBR_HD T fast_ao2(const DevScene &sc, ShaderIn<T> &in, LaneCount &cnt) {
   const ShadeK<T> &k = sc.shade<T>();
   T delta = in.dist_thresh;
@@ -214,7 +213,7 @@ MBR_HD T fast_ao2(const DevScene &sc, ShaderIn<T> &in, LaneCount &cnt) {
   for (int i = 1; i < q * q; i++) {
     inv2i *= T(0.5);  // 1/pow(2,i), exact
     T scan = T(i * i) * delta;
-    T dist = de_at<T, F, Deep>(sc, in, in.normal * scan, in.detail, sc.N, sc.minN, false, info, cnt);
+    T dist = de_at<T, F>(sc, in, in.normal * scan, in.detail, sc.N, sc.minN, false, info, cnt);
     aoTemp += inv2i * (scan - k.fast_ao_tune * dist) / in.dist_thresh;
   }
   T ao = T(1) - T(0.2) * aoTemp;
@@ -229,7 +228,7 @@ struct AOTable {
   int count;
 };
 
-template <class T, int F = 0, bool Deep = false>
+template <class T, int F = 0>
 MBR_HD RGBT<T> ambient_occlusion(const DevScene &sc, ShaderIn<T> &in, const AOTable<T> &tab, LaneCount &cnt) {
   const ShadeK<T> &k = sc.shade<T>();
   RGBT<T> ao = {0, 0, 0};
@@ -243,7 +242,7 @@ MBR_HD RGBT<T> ambient_occlusion(const DevScene &sc, ShaderIn<T> &in, const AOTa
     T shadowTemp = 1;
     int guard = 0;
     for (T r = start_dist; r < end_dist && guard < kMaxShadeSteps; r += dist * T(2), guard++) {
-      dist = de_at<T, F, Deep>(sc, in, dir * r, in.detail, sc.N, sc.minN, false, info, cnt);
+      dist = de_at<T, F>(sc, in, dir * r, in.detail, sc.N, sc.minN, false, info, cnt);
       if (dist < (T)dist_thresh || info.max_iter || shadowTemp < T(0)) {
         shadowTemp -= (end_dist - r) / end_dist;
         if (shadowTemp < T(0)) shadowTemp = 0;
@@ -417,42 +416,6 @@ MBR_HD RGBT<T> surface_colour(const DevScene &sc, const ShaderIn<T> &in, LaneCou
     default: pc = sc.plane_col; break;
   }
   out.R = T(pc[0]) / T(65536); out.G = T(pc[1]) / T(65536); out.B = T(pc[2]) / T(65536);
-  return out;
-}
-
-// ObjectShader: returns object + specular terms; *colour_out is the surface
-// colour (colourBuffer source).
-template <class T, int F = 0, bool Deep = false>
-MBR_HD RGBT<T> object_shader(const DevScene &sc, ShaderIn<T> &in, const AOTable<T> &tab, RGBT<T> &colour_out,
-                             LaneCount &cnt) {
-  const ShadeK<T> &k = sc.shade<T>();
-  in.normal = normals<T, F, Deep>(sc, in, cnt);
-  T sh = dot(in.normal, in.light);
-  if (sh < 0) sh = 0;
-  const T shade = k.direct_light * ((T(1) - k.shading) + k.shading * sh);
-  T shadow = 1;
-  if (sc.shadow) shadow = main_shadow<T, F, Deep>(sc, in, cnt);
-  V3<T> half = normalize(in.light - in.view);
-  T shade2 = dot(in.normal, half);
-  if (shade2 < T(0)) shade2 = 0;
-  shade2 = Math<T>::pow(shade2, T(30));
-  if (shade2 > T(15)) shade2 = 15;
-  const T specular = shade2 * k.specular;
-  RGBT<T> colour = surface_colour<T, Deep, sizeof(T) == 8 || F == 0>(sc, in, cnt);
-  colour_out = colour;
-  RGBT<T> ambient = {0, 0, 0};
-  if (sc.ao) {
-    if (sc.fast_ao) {
-      T a = fast_ao2<T, F, Deep>(sc, in, cnt);
-      ambient = RGBT<T>{a, a, a};
-    } else {
-      ambient = ambient_occlusion<T, F, Deep>(sc, in, tab, cnt);
-    }
-  }
-  RGBT<T> out;
-  out.R = (ambient.R * k.global_ilum + k.main_light[0] * shade * shadow) * colour.R + k.main_light[0] * specular * shadow;
-  out.G = (ambient.G * k.global_ilum + k.main_light[1] * shade * shadow) * colour.G + k.main_light[1] * specular * shadow;
-  out.B = (ambient.B * k.global_ilum + k.main_light[2] * shade * shadow) * colour.B + k.main_light[2] * specular * shadow;
   return out;
 }
 
