@@ -35,9 +35,9 @@ DIFF_KEYS = ("flip_frac", "hitmiss_px", "sheet_px", "depth_rel_max", "depth_rel_
 # HBM bytes per k_ao launch on this workload (FETCH_SIZE x 2 + WRITE_SIZE x 1,
 # the factors that make a 1 GiB device copy read 1 GiB and write 1 GiB),
 # from the rocprofv3 --pmc runs summarised in the file named here.
-AO_TRAFFIC_BYTES = 401.6e6
+AO_TRAFFIC_BYTES = 408.2e6
 AO_TRAFFIC_SOURCE = ("profiles/render_1080p_mandelbulb_pmc.txt (per launch, one of the frame's two bands: "
-                     "FETCH_SIZE 29.1 MiB x 2 + WRITE_SIZE 324.9 MiB)")
+                     "FETCH_SIZE 31.5 MiB x 2 + WRITE_SIZE 326.3 MiB)")
 
 
 def planes_on_gpu(torch, w, h):

@@ -570,7 +570,8 @@ typedef struct mbr_batch_opts {
   int precision;                   /* enum mbr_precision */
   void *stream;                    /* hipStream_t the graph is launched on; NULL = the context's */
   int slots;                       /* concurrent frame chains 1..4; 0 = tuned or 2 */
-  int blocks_per_cu;               /* workgroups per CU of the persistent kernels; 0 = tuned or 8 */
+  int blocks_per_cu;               /* workgroups per CU of the persistent kernels, as far as
+                                      they fit (2 to 8 by kernel); 0 = tuned or 8 */
   int autotune;                    /* 1: time every (slots, blocks_per_cu) candidate on this batch,
                                       keep the fastest in the context for later batches */
   int replays;                     /* graph launches (>= 1); the last one's frames are returned */

@@ -1313,11 +1313,12 @@ int enqueue_frame(mbr_ctx *c, Slot &sl, int precision, const DevScene *d_sc, con
 // rays, or its continuation, surface and composition kernels leave the
 // vector units idle, the other band's kernels fill the CUs.  Each band's
 // results depend only on its own rays, so the frame equals the one-stream
-// frame bit for bit.  Measured on the 1080p power-8 bulb (MI355X) with the
-// kernels of that time: two bands 13.5 ms against 14.4 ms on one stream; four
-// or more bands, a staggered start of the second stream and smaller march or
-// AO grids were all slower.  FP64 frames stay on one stream (two FP64 bands at
-// once took 133-143 ms against 127 ms).
+// frame bit for bit.  Measured (MI355X, ms, one stream / two bands / four bands):
+// 1080p power-8 bulb with AO quality 8 9.5 / 9.3 / 10.0, without shading 2.6 /
+// 2.5 / 2.9, 1280x720 Mandelbox FP32_MARCH 18.0 / 17.2 / 20.1, its 4K deep zoom
+// 109 / 75 / 76, 1280x720 13.7 / 13.1 / 19.5; against it 1001x563 Menger 2.01 /
+// 2.09 / 2.8.  FP64 frames stay on one stream: two bands at once gain 1 to 2%
+// (1080p bulb 63.6 and 62.3 ms, 1280x720 Mandelbox 42.2 and 42.0).
 constexpr long long kSplitRays = 1 << 18;
 constexpr int kSplitBands = 2;
 

@@ -6,9 +6,9 @@
 //               src/Render3D.cpp:79-199); hits are appended to a compacted hit
 //               list so shading runs on full waves of hits.  FP32_MARCH: k_march
 //               in FP32 first, then k_march64 over the rays it handed over.
-//   k_hits      shadow rays, normals and colours of the hits (ObjectShader,
-//               src/shaders.cpp:21); k_fast_ao or k_ao their ambient occlusion,
-//               k_compose the sums.
+//   k_hits      shadow rays, normals (slowShading's: k_slow_normals) and colours
+//               of the hits (ObjectShader, src/shaders.cpp:21); k_fast_ao or
+//               k_ao their ambient occlusion, k_compose the sums.
 //   k_finish    one lane per ray: background for misses, VolumetricShader
 //               (glow, fog, volumetric fog) over the step record read back to
 //               front, and coalesced writes of the framebuffer planes
@@ -1556,9 +1556,9 @@ __global__ void __launch_bounds__(kBlock) k_aux(const DevScene *__restrict__ scp
 // and 1/2 for the folding formulas, whose iterations are short and more per
 // estimate (1280x720 Mandelbox, AO quality 4, FP32_MARCH: AO of a band 7.47 ms
 // with 2, 6.92 with 4, 6.86 with 6, the frame 18.3 and 17.1 ms; 1001x563 Menger
-// 1.33, 1.25 and 1.22 ms, the frame 2.31 and 2.16).  FP64 (twice the registers,
-// 2 waves per SIMD): 1 iteration, 1/6, 1/8 (measured best of the sweeps on
-// MI355X).
+// 1.33, 1.25 and 1.22 ms, the frame 2.31 and 2.16).  FP64: 1 iteration, 1/6, 1/8
+// (best of the sweeps of the trigonometric Mandelbulb, with 2 waves per SIMD;
+// the folding formulas take the same, not swept apart).
 enum : int { AO_NEED = 0, AO_ITER = 1, AO_DONE = 2, AO_EXHAUSTED = 3 };
 // Per element type: formula iterations per pass, and the share of the wave
 // (1/div) that must wait in DONE or NEED before their block runs.
@@ -2333,9 +2333,10 @@ static inline void march_variant(int formula, int plain, bool ip8, Go go) {
   std::integral_constant<int, kPlain> yes;
   std::integral_constant<int, kOptions> no;
   std::integral_constant<int, kStandardBox> box;
-  // trig_DE and the kaleidoscopic IFS: compiled by themselves their kernels take
-  // 228 and 124 registers and no scratch memory, the generic ones (30 formulas,
-  // finite differences, whole estimates) 512 and 1.7 KB.  400x300 trig_DE with
+  // trig_DE and the kaleidoscopic IFS: compiled by themselves their march takes
+  // 226 and 122 registers and no scratch memory (trig_DE's FP32 AO spills 10 of
+  // its 80), the generic ones (30 formulas, finite differences, whole estimates)
+  // 512 and 1.8 KB.  400x300 trig_DE with
   // soft shadows and fast AO, FP32_FIXUP: 15.6 -> 10.4 ms (march 5.5 -> 1.4).
   // The optional terms stay with the generic kernels.
   if (formula_march64(formula) && plain) {
