@@ -25,10 +25,12 @@ def renderer():
 def _planes(w, h):
     import torch
     d = torch.device("cuda:0")
-    return {"rgb": torch.zeros((3, h, w), device=d), "z": torch.zeros((h, w), device=d),
-            "colour": torch.full((3, h, w), 7, dtype=torch.uint8, device=d),
-            "alpha": torch.zeros((h, w), dtype=torch.int16, device=d),
-            "opacity": torch.zeros((h, w), dtype=torch.int16, device=d)}
+    planes = {"rgb": torch.zeros((3, h, w), device=d), "z": torch.zeros((h, w), device=d),
+              "colour": torch.full((3, h, w), 7, dtype=torch.uint8, device=d),
+              "alpha": torch.zeros((h, w), dtype=torch.int16, device=d),
+              "opacity": torch.zeros((h, w), dtype=torch.int16, device=d)}
+    torch.cuda.synchronize()  # the context renders on a stream of its own
+    return planes
 
 
 @pytest.mark.parametrize("call", ["render_device", "render_device_noalloc"])
