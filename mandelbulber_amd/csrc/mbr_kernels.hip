@@ -2470,8 +2470,8 @@ hipError_t launch_march_fix(const DevScene *sc, const BandBufs &b, int band_firs
 __global__ void k_band_reset(BandBufs b) {
   const int i = (int)threadIdx.x;
   if (i >= CNT_COUNT) return;
-  b.counters[i] = 0;
-  if (i == CNT_RAYQ || i == CNT_AOQ) poll_cancel(b, &b.counters[i]);
+  const bool stop = (i == CNT_RAYQ || i == CNT_AOQ) && b.cancel && *b.cancel != 0;
+  b.counters[i] = stop ? kStopBit : 0;
 }
 
 hipError_t launch_band_reset(const BandBufs &b, hipStream_t s) {
